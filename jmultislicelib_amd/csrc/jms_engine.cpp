@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 #include <algorithm>
 #include <cmath>
+#include <cstdint>
 #include <cstdio>
 #include <cstring>
 #include <array>
@@ -47,6 +48,41 @@ struct DevBuf {
   T* as() const { return (T*)p; }
 };
 
+// the zero gap of a Fourier-space array: columns [x0, x1) around nx/2 that
+// are zero in every row, rows [y0, y1) around ny/2 zero in every column
+struct Gap {
+  int x0 = 0, x1 = 0, y0 = 0, y1 = 0;
+};
+// values [i0, i1) of a complex row all zero (either sign): the bits ORed,
+// which the compiler vectorises
+bool zeros(const float* row, int i0, int i1) {
+  uint32_t any = 0;
+  for (int k = 2 * i0; k < 2 * i1; ++k) {
+    uint32_t u;
+    std::memcpy(&u, row + k, 4);
+    any |= u;
+  }
+  return (any & 0x7fffffffu) == 0;
+}
+Gap zero_gap(const float* a, int nx, int ny, bool rows) {
+  Gap g{0, nx, 0, 0};
+  auto row = [&](int y) { return a + 2 * (size_t)y * nx; };
+  const int cx = nx / 2, cy = ny / 2;
+  for (int y = 0; y < ny && g.x0 < g.x1; ++y) {
+    if (zeros(row(y), g.x0, g.x1)) continue;
+    int l = cx, r = cx;
+    while (l > g.x0 && zeros(row(y), l - 1, l)) --l;
+    while (r < g.x1 && zeros(row(y), r, r + 1)) ++r;
+    g.x0 = l;
+    g.x1 = r;
+  }
+  if (!rows) return g;
+  g.y0 = g.y1 = cy;
+  while (g.y0 > 0 && zeros(row(g.y0 - 1), 0, nx)) --g.y0;
+  while (g.y1 < ny && zeros(row(g.y1), 0, nx)) ++g.y1;
+  return g;
+}
+
 struct Timer {
   double ms = 0.0;
   long long count = 0;
@@ -76,6 +112,7 @@ struct jms_hip_engine {
   int npro = 0;
   std::vector<int> proidx;
   DevBuf pro, pro_t;  // row-major and column-major ([x][y]) copies
+  std::vector<Gap> pro_gap;  // zero gap of each propagator
   // object slices
   int nobjslc = 0;
   std::vector<int> objslc;
@@ -83,8 +120,10 @@ struct jms_hip_engine {
   int ndetslc = 0, ndet = 0, detflags = 0;
   std::vector<int> det_objslc;
   DevBuf detw, detw_t;
+  std::vector<char> det_inf;  // detectors with weights that are not finite
   // incident wave
   DevBuf wav0, cppl, cppl_t;
+  Gap wav0_gap, wav_gap;  // zero gap (columns) of the probe and of the single-wave path's wave
   bool have_cppl = false;
   // staged scan
   int s_npos = 0, s_npass = 0;
@@ -107,6 +146,7 @@ struct jms_hip_engine {
   bool use_graph = false;
   std::map<std::array<int, 4>, hipGraphExec_t> graphs;
   std::array<const void*, 16> graph_bufs{};
+  std::array<int, 4> graph_band{};  // and to the band the launches were made for
   // this device's scratch of the allocation-free batch entry (resolved at create)
   float* scratch = nullptr;
   // staged batches keep their waves in 16-column panels (set with the grid)
@@ -140,6 +180,26 @@ struct jms_hip_engine {
             pro.p, pro_t.p, detw.p, detw_t.p, twx.p, twy.p, cppl.p, cppl_t.p};
   }
   int ntiles_col() const { return jms::col_tiles(ny, nx); }
+  // The columns and rows that the waves leave out: where the propagators of
+  // all object slices vanish.  A detector weight that is not finite makes
+  // 0 * weight count, so those keep every column.
+  jms::BandHost band() const {
+    Gap g{0, nx, 0, ny};
+    if (nobjslc < 1) return jms::BandHost();
+    for (char c : det_inf)
+      if (c) return jms::BandHost();
+    for (int o : objslc) {
+      const Gap& p = pro_gap[proidx[o % nscslc]];
+      g.x0 = std::max(g.x0, p.x0);
+      g.x1 = std::min(g.x1, p.x1);
+      g.y0 = std::max(g.y0, p.y0);
+      g.y1 = std::min(g.y1, p.y1);
+    }
+    return jms::band_of(nx, ny, g.x0, g.x1, g.y0, g.y1);
+  }
+  // the probe is zero there too, so the first passes leave the columns out as well
+  static bool holds(const Gap& g, const jms::BandHost& b) { return g.x0 <= b.x0 && g.x1 >= b.x1; }
+  bool probe_in(const jms::BandHost& b) const { return holds(wav0_gap, b); }
 };
 
 namespace {
@@ -227,11 +287,14 @@ struct BatchChans {
 // (stride n); `ppar` (float4 per wave) and `var` (nobjslc ints per wave)
 // describe them; src/src_stride the INIT source.  Readout partial sums go to
 // `partial` ([wave][plane][detector][column tile]), combined into `res`
-// (npos results) when npass > 0; `ch` are the single-wave channels.
+// (npos results) when npass > 0; `ch` are the single-wave channels.  `bd`:
+// the columns left out from the first slice on, and with `src_in` (the source
+// is zero there) in the passes before it; `keep`: leave psi(k) of the exit
+// plane in the waves (batches only read the sums).
 int enqueue_batch(jms_hip_engine* e, void* waves, float* partial, int nwave, int islc0, const void* src,
                   long long src_stride, const void* ppar, const int* var, int npos, int npass,
                   const float* weights, float* res, int accumulate, const BatchChans& ch, bool timed,
-                  bool panel = false) {
+                  const jms::BandHost& bd, bool src_in, bool keep, bool panel = false) {
   // panel waves (staged batches): integrated readouts only, the waves are internal
   if (panel && (ch.real_space() || ch.dif || ch.wff || ch.dif_avg || ch.wff_avg))
     return e->fail(135, "panel waves carry no readout channels");
@@ -269,6 +332,7 @@ int enqueue_batch(jms_hip_engine* e, void* waves, float* partial, int nwave, int
   rc.chan_wstride = ca.chan_wstride;
   ca.twy = e->twy.p;
   ca.panel = panel;
+  ca.keep = keep;
   hipError_t err;
   auto plane_setup = [&](int plane) {
     const int id = (plane >= 0 && plane <= S) ? e->det_objslc[plane] : -1;
@@ -283,12 +347,14 @@ int enqueue_batch(jms_hip_engine* e, void* waves, float* partial, int nwave, int
     ca.ppar = ppar;
     ca.pro = nullptr;
     plane_setup(islc0);
+    if (src_in && islc0 < S) ca.band = bd;
     TimedLaunch tl(e, 1, timed);
     err = jms::launch_col_pass(e->ny, nwave, true, islc0 >= S, ca, e->st);
     if (err != hipSuccess) return e->fail(130, "column pass (init)", err);
   }
   ca.src = nullptr;
   ca.ppar = nullptr;
+  ca.band = bd;
   for (int j = islc0; j < S; ++j) {
     const int js = e->objslc[j] % e->nscslc;
     {
@@ -299,7 +365,8 @@ int enqueue_batch(jms_hip_engine* e, void* waves, float* partial, int nwave, int
       TimedLaunch tl(e, 0, timed);
       err = jms::launch_row_pass(e->nx, e->ny, nwave, (float2*)waves, e->n,
                                  e->pgr.as<float2>(), e->slcoffset[js], (long long)e->npgx * e->npgy,
-                                 var, S, j, e->twx.as<float2>(), rc, mode, panel, e->st);
+                                 var, S, j, e->twx.as<float2>(), rc, mode, panel,
+                                 j > islc0 || src_in ? bd : jms::BandHost(), e->st);
       if (err != hipSuccess) return e->fail(131, "row pass", err);
     }
     ca.pro = e->pro.as<float2>() + (long long)e->proidx[js] * e->n;
@@ -348,7 +415,7 @@ int enqueue_exit_real_readout(jms_hip_engine* e, int nwave, const BatchChans& ch
   hipError_t err = jms::launch_col_fft(e->nx, e->ny, nwave, e->waves.as<float2>(), +1, e->twy.as<float2>(), e->st);
   if (err == hipSuccess)
     err = jms::launch_row_pass(e->nx, e->ny, nwave, e->waves.as<float2>(), e->n, e->pgr.as<float2>(), 0, 0,
-                               nullptr, 0, 0, e->twx.as<float2>(), rc, 2, false, e->st);
+                               nullptr, 0, 0, e->twx.as<float2>(), rc, 2, false, jms::BandHost(), e->st);
   if (err != hipSuccess) return e->fail(134, "exit-plane real-space readout", err);
   return 0;
 }
@@ -440,6 +507,8 @@ int jms_hip_set_grid(jms_hip_engine* e, int nx, int ny, float a0x, float a0y, fl
   e->nx = nx; e->ny = ny; e->n = (long long)nx * ny;
   e->a0x = a0x; e->a0y = a0y; e->wl = wl;
   e->panel = jms::panel_ok(nx, ny);
+  e->pro_gap.assign(e->pro_gap.size(), Gap());
+  e->wav0_gap = e->wav_gap = Gap();
   std::vector<float> tw;
   make_twiddles(nx, tw);
   hipError_t err = e->twx.ensure(tw.size() * sizeof(float));
@@ -641,6 +710,7 @@ int jms_hip_setup_propagators(jms_hip_engine* e, int npro, int nslc, const int* 
   e->drop_graphs();
   e->npro = npro;
   e->proidx.assign(proidx, proidx + nslc);
+  e->pro_gap.assign(npro, Gap());
   hipError_t err = e->pro.ensure(sizeof(float) * 2 * (size_t)npro * e->n);
   if (err == hipSuccess) err = e->pro_t.ensure(sizeof(float) * 2 * (size_t)npro * e->n);
   if (err != hipSuccess) return e->fail(102, "allocate propagators", err);
@@ -652,6 +722,7 @@ int jms_hip_upload_propagator(jms_hip_engine* e, int ipro, const float* pro) {
   if (ipro < 0 || ipro >= e->npro || !pro) return e->fail(2, "invalid propagator upload");
   (void)hipSetDevice(e->device);
   (void)hipStreamSynchronize(e->st);  // launches already enqueued may still read what this replaces
+  e->pro_gap[ipro] = zero_gap(pro, e->nx, e->ny, true);
   hipError_t err = hipMemcpy(e->pro.as<float2>() + (long long)ipro * e->n, pro,
                              sizeof(float) * 2 * (size_t)e->n, hipMemcpyHostToDevice);
   if (err == hipSuccess) {
@@ -694,6 +765,7 @@ int jms_hip_setup_detection(jms_hip_engine* e, int ndetslc, const int* det_objsl
   e->ndet = ndet;
   e->detflags = flags;
   e->det_objslc.assign(det_objslc, det_objslc + e->nobjslc + 1);
+  e->det_inf.assign(ndet, 0);
   // averaging channels start empty (DetectorSetup, JMultiSlice.cpp:784-800)
   {
     const size_t nchan = (size_t)ndetslc * e->n;
@@ -737,6 +809,13 @@ int jms_hip_upload_detector(jms_hip_engine* e, int idet, const float* det, int m
   } else {
     std::memcpy(wgt.data(), det, sizeof(float) * (size_t)e->n);
   }
+  uint32_t inf = 0;  // some weight not finite
+  for (float x : wgt) {
+    uint32_t u;
+    std::memcpy(&u, &x, 4);
+    inf |= ((u & 0x7f800000u) == 0x7f800000u);
+  }
+  e->det_inf[idet] = inf != 0;
   std::vector<float> wt = to_colmajor(wgt.data(), e->nx, e->ny);
   const size_t nb = sizeof(float) * (size_t)e->n;
   hipError_t err = hipMemcpy(e->detw.as<float>() + (long long)idet * e->n, wgt.data(), nb, hipMemcpyHostToDevice);
@@ -752,6 +831,7 @@ int jms_hip_set_probe(jms_hip_engine* e, const float* wav0) {
   (void)hipSetDevice(e->device);
   (void)hipStreamSynchronize(e->st);  // launches already enqueued may still read what this replaces
   const size_t nb = sizeof(float) * 2 * (size_t)e->n;
+  e->wav0_gap = zero_gap(wav0, e->nx, e->ny, false);
   hipError_t err = e->wav0.ensure(nb);
   if (err == hipSuccess) err = hipMemcpy(e->wav0.p, wav0, nb, hipMemcpyHostToDevice);
   if (err != hipSuccess) return e->fail(102, "upload probe", err);
@@ -794,11 +874,13 @@ int jms_hip_probe(jms_hip_engine* e, const float* prm, int nabrr, const float* a
   (void)hipStreamSynchronize(e->st);  // launches already enqueued may still read what this replaces
   const size_t nb = sizeof(float) * 2 * (size_t)e->n;
   DevBuf partial;
+  e->wav0_gap = Gap();
   hipError_t err = e->wav0.ensure(nb);
   if (err == hipSuccess) err = partial.ensure(sizeof(double) * (size_t)((e->n + 255) / 256));
   if (err == hipSuccess) err = jms::launch_probe(e->wav0.as<float2>(), partial.as<double>(), a, e->st);
   if (err == hipSuccess) err = hipStreamSynchronize(e->st);
   if (err == hipSuccess && out) err = hipMemcpy(out, e->wav0.p, nb, hipMemcpyDeviceToHost);
+  if (err == hipSuccess && out) e->wav0_gap = zero_gap(out, e->nx, e->ny, false);
   partial.release();
   if (err != hipSuccess) return e->fail(102, "probe on the device", err);
   return 0;
@@ -910,6 +992,8 @@ int jms_hip_run_staged(jms_hip_engine* e, int pos0, int npos, int islc0) {
   if (rc) return rc;
   const int S = e->nobjslc;
   const int per = e->ndetslc * std::max(1, e->ndet);
+  const jms::BandHost bd = e->band();
+  const bool src_in = e->probe_in(bd);
   for (int p = pos0; p < pos0 + npos; p += bpos) {
     const int np = std::min(bpos, pos0 + npos - p);
     const int nw = np * npass;
@@ -926,9 +1010,11 @@ int jms_hip_run_staged(jms_hip_engine* e, int pos0, int npos, int islc0) {
         err = hipMemcpyAsync(e->cur_var.p, var, sizeof(int) * (size_t)nw * S, hipMemcpyDeviceToDevice, e->st);
       if (err != hipSuccess) return e->fail(120, "stage batch", err);
       const auto bufs = e->batch_buffers();
-      if (bufs != e->graph_bufs) {
+      const std::array<int, 4> gband{bd.x0, bd.x1, bd.rows, src_in};
+      if (bufs != e->graph_bufs || gband != e->graph_band) {
         e->drop_graphs();
         e->graph_bufs = bufs;
+        e->graph_band = gband;
       }
       const std::array<int, 4> key{nw, islc0, np, npass};
       auto it = e->graphs.find(key);
@@ -939,7 +1025,7 @@ int jms_hip_run_staged(jms_hip_engine* e, int pos0, int npos, int islc0) {
         rc = enqueue_batch(e, e->waves.p, e->partial.as<float>(), nw, islc0, e->wav0.p, 0, e->cur_ppar.p,
                            e->cur_var.as<int>(), np,
                            npass, e->s_weights.as<float>(), e->cur_res.as<float>(), 0, BatchChans(), false,
-                           e->panel);
+                           bd, src_in, false, e->panel);
         hipError_t err2 = hipStreamEndCapture(e->st, &g);
         if (rc) { if (g) (void)hipGraphDestroy(g); return rc; }
         if (err2 != hipSuccess) return e->fail(122, "end capture", err2);
@@ -959,7 +1045,7 @@ int jms_hip_run_staged(jms_hip_engine* e, int pos0, int npos, int islc0) {
     } else {
       rc = enqueue_batch(e, e->waves.p, e->partial.as<float>(), nw, islc0, e->wav0.p, 0, ppar, var, np, npass,
                          e->s_weights.as<float>(), res,
-                         0, BatchChans(), e->timing, e->panel);
+                         0, BatchChans(), e->timing, bd, src_in, false, e->panel);
       if (rc) return rc;
     }
   }
@@ -987,8 +1073,9 @@ int jms_hip_run_batch_noalloc(jms_hip_engine* e, int islc0, int nwave, void* wav
   if (!e->scratch) return e->fail(7, "no scratch address");
   islc0 = std::max(0, std::min(islc0, e->nobjslc));
   (void)hipSetDevice(e->device);
+  const jms::BandHost bd = e->band();
   return enqueue_batch(e, waves, e->scratch, nwave, islc0, e->wav0.p, 0, ppar, var, npos, npass, weights, res, 0,
-                       BatchChans(), false, e->panel);
+                       BatchChans(), false, bd, e->probe_in(bd), false, e->panel);
 }
 
 // ---------------------------------------------------------------------------
@@ -1237,6 +1324,16 @@ int jms_hip_group_run(jms_hip_group* g) {
     if (err != hipSuccess) return g->fail(103, "upload group tables", err);
     g->host.swap(host);
   }
+  // one band for all members: the columns and rows that every member leaves out
+  jms::BandHost bd = lead->band();
+  for (auto* e : g->eng) {
+    if (e->nobjslc < 1) continue;  // only its INIT pass, which covers its own columns
+    const jms::BandHost b = e->band();
+    bd.x0 = std::max(bd.x0, b.x0);
+    bd.x1 = std::min(bd.x1, b.x1);
+    bd.rows = bd.rows && b.rows;
+    if (!bd.on() || !b.on() || !e->probe_in(b)) bd.x0 = bd.x1 = 0;
+  }
   const char* base = (const char*)g->tab.p;
   const long long n = (long long)g->nx * g->ny;
   const int ld = g->smax + 1;
@@ -1256,7 +1353,8 @@ int jms_hip_group_run(jms_hip_group* g) {
       ga.step = plane;
       TimedLaunch tl(lead, 1, lead->timing);
       return jms::launch_col_pass_grp(g->nx, g->ny, w1 - w0, init, exit_, group_detects(g, rd, plane, w0, w1), ntc,
-                                      lead->twy.as<float2>(), ga, lead->panel, st);
+                                      lead->twy.as<float2>(), ga, lead->panel,
+                                      init && exit_ ? jms::BandHost() : bd, st);
     };
     err = col(0, true, 0, rd.active[0], false);
     if (err == hipSuccess) err = col(0, true, rd.active[0], rd.nwave, true);
@@ -1265,7 +1363,8 @@ int jms_hip_group_run(jms_hip_group* g) {
       ga.step = s;
       {
         TimedLaunch tl(lead, 0, lead->timing);
-        err = jms::launch_row_pass_grp(g->nx, g->ny, rd.active[s], n, n, lead->twx.as<float2>(), ga, lead->panel, st);
+        err = jms::launch_row_pass_grp(g->nx, g->ny, rd.active[s], n, n, lead->twx.as<float2>(), ga, lead->panel, bd,
+                                       st);
       }
       if (err == hipSuccess) err = col(s + 1, false, 0, rd.active[s + 1], false);
       if (err == hipSuccess) err = col(s + 1, false, rd.active[s + 1], rd.active[s], true);
@@ -1320,6 +1419,7 @@ int jms_hip_wave_offset(jms_hip_engine* e, float dx, float dy, float dz, int ibt
   if (err != hipSuccess) return e->fail(103, "allocate wave", err);
   int ish0 = ibtx % e->nx; if (ish0 < 0) ish0 += e->nx;  // JMultiSlice.cpp:1990-1991
   int ish1 = ibty % e->ny; if (ish1 < 0) ish1 += e->ny;
+  e->wav_gap = ish0 == 0 ? e->wav0_gap : Gap();
   err = jms::launch_offset_wave(e->wav.as<float2>(), e->wav0.as<float2>(), e->nx, e->ny, 1.f / e->a0x,
                                 1.f / e->a0y, dx, dy, dz * e->wl * 0.5f,
                                 (use_cppl && e->have_cppl) ? e->cppl.as<float>() : nullptr, ish0, ish1, e->st);
@@ -1333,6 +1433,7 @@ int jms_hip_wave_set(jms_hip_engine* e, const float* wav) {
   (void)hipSetDevice(e->device);
   (void)hipStreamSynchronize(e->st);  // launches already enqueued may still read what this replaces
   hipError_t err = e->wav.ensure(sizeof(float) * 2 * (size_t)e->n);
+  e->wav_gap = zero_gap(wav, e->nx, e->ny, false);
   if (err == hipSuccess) err = hipMemcpy(e->wav.p, wav, sizeof(float) * 2 * (size_t)e->n, hipMemcpyHostToDevice);
   if (err != hipSuccess) return e->fail(102, "set wave", err);
   return 0;
@@ -1396,10 +1497,14 @@ int jms_hip_multislice(jms_hip_engine* e, int islc0, const int* var, float weigh
   if (fl & JMS_HIP_DETECT_IMAGE_AVG) ch.img_avg = e->img_avg.as<float>();
   if (fl & JMS_HIP_DETECT_WAVEF_AVG) ch.wff_avg = e->wff_avg.p;
   if (fl & JMS_HIP_DETECT_WAVER_AVG) ch.wfr_avg = e->wfr_avg.p;
+  const jms::BandHost bd = e->band();
+  const bool src_in = e->holds(e->wav_gap, bd);
+  if (islc0 < S) e->wav_gap = Gap();  // until the run is enqueued
   rc = enqueue_batch(e, e->waves.p, e->partial.as<float>(), 1, islc0, e->wav.p, e->n, nullptr,
                      e->var1.as<int>(), 1, 1, e->w1.as<float>(),
-                     e->res1.as<float>(), 1, ch, e->timing);
+                     e->res1.as<float>(), 1, ch, e->timing, bd, src_in, true);
   if (rc) return rc;
+  if (islc0 < S) e->wav_gap = Gap{bd.x0, bd.x1, 0, 0};
   // the run leaves psi(k) of the exit plane in the batch slot; keep it as the wave
   err = hipMemcpyAsync(e->wav.p, e->waves.p, sizeof(float) * 2 * (size_t)e->n, hipMemcpyDeviceToDevice, e->st);
   if (err != hipSuccess) return e->fail(113, "multislice run", err);

@@ -561,4 +561,21 @@ struct IOMap {
   static constexpr bool FULL = (NB * T == NBF);
 };
 
+// Slots of a first-stage butterfly of radix R0 on a band-limited line: slot q
+// covers elements [q N/R0, (q+1) N/R0).  The propagators vanish beyond two
+// thirds of the Nyquist frequency, so the elements around N/2 that a
+// band-limited line neither stores nor needs (the gap) reach from about N/3
+// to 2 N/3: slots strictly inside are always dead (zero on input, unused on
+// output, so the butterfly is pruned at compile time), the two that hold the
+// gap's ends are tested per element, the others are always live.
+template <int N, int R0>
+struct BandSlots {
+  static constexpr int LO = R0 / 3, HI = R0 - 1 - LO;  // the slots of the gap's ends
+  static constexpr bool part(int q) { return q == LO || q == HI; }
+  static constexpr bool dead(int q) { return q > LO && q < HI; }
+  // a gap [g0, g1) these classes hold for
+  static constexpr int G0_MIN = LO * (N / R0), G0_MAX = (LO + 1) * (N / R0);
+  static constexpr int G1_MIN = HI * (N / R0), G1_MAX = (HI + 1) * (N / R0);
+};
+
 }  // namespace jms

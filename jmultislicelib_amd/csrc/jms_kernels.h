@@ -4,7 +4,22 @@
 
 namespace jms {
 
-// Arguments of one column pass (see k_col_pass in jms_kernels.hip).
+// Band-limited waves.  The propagators vanish beyond two thirds of the Nyquist
+// frequency (CalculatePropagator, JMultiSlice.cpp:1015-1040), so after a
+// column pass the wave is zero on the columns around nx/2.  Columns [x0, x1)
+// (whole column tiles) are then neither stored between the passes nor
+// transformed; rows: the column transforms leave out the rows around ny/2
+// where the propagators vanish too.
+struct BandHost {
+  int x0 = 0, x1 = 0;
+  bool rows = false;
+  bool on() const { return x1 > x0; }
+};
+// the band the passes of an nx x ny grid use, given columns [gx0, gx1) and
+// rows [gy0, gy1) where every propagator of the run vanishes
+BandHost band_of(int nx, int ny, int gx0, int gx1, int gy0, int gy1);
+
+// Arguments of one column pass (see ColArgs in jms_kernels_impl.hpp).
 struct ColArgsHost {
   void* wave = nullptr;          // batch of waves (float2), wave_stride items apart
   int nx = 0;
@@ -36,6 +51,8 @@ struct ColArgsHost {
   const float* detw_t = nullptr; // [ndet][nx][ny] detector weights
   const float* cppl_t = nullptr; // constant phase plate or nullptr
   bool panel = false;            // the waves are in 16-column panels (panel_ok)
+  BandHost band;                 // columns and rows left out
+  bool keep = false;             // EXIT: store psi(k), the columns left out cleared
 };
 
 // real-space readout channels of one detection plane for the row pass
@@ -126,13 +143,14 @@ struct GrpArgs {
 bool grp_supported(int nx, int ny);
 // row pass of step ga.step over nwave waves of the map (from ga.w0)
 hipError_t launch_row_pass_grp(int nx, int ny, int nwave, long long wave_stride, long long npg,
-                               const float2* twx, const GrpArgs& ga, bool panel, hipStream_t st);
+                               const float2* twx, const GrpArgs& ga, bool panel, const BandHost& bd,
+                               hipStream_t st);
 // column pass producing plane ga.step (propagator of step ga.step - 1 unless
 // init) over nwave waves of the map; detect: some job of the launch reads
 // plane ga.step out (each wave checks its own job's plane table)
 hipError_t launch_col_pass_grp(int nx, int ny, int nwave, bool init, bool exit_, bool detect,
                                long long part_dstride, const float2* twy, const GrpArgs& ga,
-                               bool panel, hipStream_t st);
+                               bool panel, const BandHost& bd, hipStream_t st);
 
 constexpr int kMaxDetPerSweep = 8;
 
@@ -143,10 +161,11 @@ int col_tiles(int ny, int nx);
 // mode 0: slice; 1: slice with the real-space readout of `rc` first;
 // 2: inverse x-transform and readout only (exit plane, after a column IFFT).
 // panel: the waves are in 16-column panels (mode 0 only; see panel_ok)
+// bd: columns that are neither read nor written (not in mode 2)
 hipError_t launch_row_pass(int nx, int ny, int nwave, float2* wave, long long wave_stride,
                            const float2* pgr, long long slc_off, long long npg, const int* var_tab,
                            int var_ld, int jslc, const float2* twx, const RowChanHost& rc, int mode,
-                           bool panel, hipStream_t st);
+                           bool panel, const BandHost& bd, hipStream_t st);
 // whether the staged batches of an nx x ny grid keep their waves in panels of
 // 16 columns: element (y, x) at (x / 16) * 16 ny + 16 y + x % 16 (column
 // tiles contiguous); chosen per line length where the passes run faster so

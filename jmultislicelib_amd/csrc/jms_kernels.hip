@@ -16,7 +16,7 @@ template <int N>
 hipError_t launch_row_pass_n(int ny, int nwave, float2* wave, long long wave_stride,
                              const float2* pgr, long long slc_off, long long npg,
                              const int* var_tab, int var_ld, int jslc, const float2* twx,
-                             const RowChanHost& rc, int mode, bool panel, hipStream_t st);
+                             const RowChanHost& rc, int mode, bool panel, const BandHost& bd, hipStream_t st);
 template <int N>
 hipError_t launch_col_pass_n(int nwave, bool init, bool exit_, const ColArgsHost& h,
                              hipStream_t st);
@@ -28,10 +28,15 @@ hipError_t launch_col_fft_n(int nx, int nbatch, float2* data, long long stride, 
                             const float2* twy, hipStream_t st);
 template <int N>
 hipError_t launch_row_pass_grp_n(int ny, int nwave, long long wave_stride, long long npg, const float2* twx,
-                                 const GrpArgs& ga, bool panel, hipStream_t st);
+                                 const GrpArgs& ga, bool panel, const BandHost& bd, hipStream_t st);
 template <int N>
 hipError_t launch_col_pass_grp_n(int nx, int nwave, bool init, bool exit_, bool detect, long long part_dstride,
-                                 const float2* twy, const GrpArgs& ga, bool panel, hipStream_t st);
+                                 const float2* twy, const GrpArgs& ga, bool panel, const BandHost& bd,
+                                 hipStream_t st);
+template <int NX>
+void band_row_n(int x0, int x1, int tile, BandHost& b);
+template <int NY>
+bool band_col_n(int y0, int y1);
 
 // frequency index of position i on an n-point grid in FFT order
 // (JMultiSlice.cpp:1699-1712)
@@ -362,15 +367,32 @@ int col_tiles(int ny, int nx) {
   }
 }
 
+BandHost band_of(int nx, int ny, int gx0, int gx1, int gy0, int gy1) {
+  BandHost b;
+  int tile = 0;
+  switch (ny) {
+#define JMS_CASE(N) case N: tile = Cfg<N>::CC; b.rows = band_col_n<N>(gy0, gy1); break;
+    JMS_SIZES(JMS_CASE)
+#undef JMS_CASE
+    default: return b;
+  }
+  switch (nx) {
+#define JMS_CASE(N) case N: band_row_n<N>(gx0, gx1, tile, b); break;
+    JMS_SIZES(JMS_CASE)
+#undef JMS_CASE
+  }
+  return b;
+}
+
 hipError_t launch_row_pass(int nx, int ny, int nwave, float2* wave, long long wave_stride,
                            const float2* pgr, long long slc_off, long long npg, const int* var_tab,
                            int var_ld, int jslc, const float2* twx, const RowChanHost& rc, int mode,
-                           bool panel, hipStream_t st) {
+                           bool panel, const BandHost& bd, hipStream_t st) {
   switch (nx) {
 #define JMS_CASE(N)                                                                         \
   case N:                                                                                   \
     return launch_row_pass_n<N>(ny, nwave, wave, wave_stride, pgr, slc_off, npg, var_tab, \
-                                var_ld, jslc, twx, rc, mode, panel, st);
+                                var_ld, jslc, twx, rc, mode, panel, bd, st);
     JMS_SIZES(JMS_CASE)
 #undef JMS_CASE
     default: return hipErrorInvalidValue;
@@ -415,9 +437,10 @@ bool grp_supported(int nx, int ny) {
 }
 
 hipError_t launch_row_pass_grp(int nx, int ny, int nwave, long long wave_stride, long long npg,
-                               const float2* twx, const GrpArgs& ga, bool panel, hipStream_t st) {
+                               const float2* twx, const GrpArgs& ga, bool panel, const BandHost& bd,
+                               hipStream_t st) {
   switch (nx) {
-#define JMS_CASE(N) case N: return launch_row_pass_grp_n<N>(ny, nwave, wave_stride, npg, twx, ga, panel, st);
+#define JMS_CASE(N) case N: return launch_row_pass_grp_n<N>(ny, nwave, wave_stride, npg, twx, ga, panel, bd, st);
     JMS_SIZES(JMS_CASE)
 #undef JMS_CASE
     default: return hipErrorInvalidValue;
@@ -426,10 +449,10 @@ hipError_t launch_row_pass_grp(int nx, int ny, int nwave, long long wave_stride,
 
 hipError_t launch_col_pass_grp(int nx, int ny, int nwave, bool init, bool exit_, bool detect,
                                long long part_dstride, const float2* twy, const GrpArgs& ga,
-                               bool panel, hipStream_t st) {
+                               bool panel, const BandHost& bd, hipStream_t st) {
   switch (ny) {
 #define JMS_CASE(N) \
-  case N: return launch_col_pass_grp_n<N>(nx, nwave, init, exit_, detect, part_dstride, twy, ga, panel, st);
+  case N: return launch_col_pass_grp_n<N>(nx, nwave, init, exit_, detect, part_dstride, twy, ga, panel, bd, st);
     JMS_SIZES(JMS_CASE)
 #undef JMS_CASE
     default: return hipErrorInvalidValue;

@@ -21,6 +21,7 @@
 // instantiates them once per supported length (one translation unit each).
 #pragma once
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <cstdint>
 #include "jms_fft_device.hpp"
 #include "jms_kernels.h"
@@ -117,6 +118,25 @@ __device__ __forceinline__ int panel_off(int x) {
   return (x & ~(kPanel - 1)) * NY + (x & (kPanel - 1));
 }
 
+// the value of x, hidden from the optimiser: table reads indexed with it are
+// repeated where they are needed instead of being kept live in registers
+// from an earlier identical read
+__device__ __forceinline__ int opaque(int x) {
+  __asm__ volatile("" : "+v"(x));
+  return x;
+}
+
+// base[idx] addressed by a 32-bit byte offset (idx * sizeof(T) < 2^32), so
+// that a wavefront-uniform base stays in scalar registers
+template <class T>
+__device__ __forceinline__ T* at32(T* base, int idx) {
+  return reinterpret_cast<T*>(reinterpret_cast<char*>(base) + (unsigned)(idx * (int)sizeof(T)));
+}
+template <class T>
+__device__ __forceinline__ const T* at32(const T* base, int idx) {
+  return reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + (unsigned)(idx * (int)sizeof(T)));
+}
+
 // real-space readout channels of one detection plane (per wave: weight
 // cwgt[w], channel stride chan_wstride items, plane offset chan_off items)
 struct RowChan {
@@ -141,15 +161,19 @@ struct RowChan {
 //   GRP:    grouped launch (MODE 0): block row y is wave ga.w0 + y of the
 //           wave map; wave buffer, variant table, gratings and the slice of
 //           step jslc come from its job's tables.
+//   BAND:   columns [gx0, gx1) are zero in the propagators on both sides of
+//           the slice (BandSlots): they are neither read nor written.  The
+//           pass is bound by its wave traffic, so that third of it is time.
 // grid: (ceil(ny/LPB), nwave); block: T*LPB
 // ---------------------------------------------------------------------------
-template <int N, int MODE = 0, class C_ = Cfg<N>, bool GRP = false, bool PANEL = false>
+template <int N, int MODE = 0, class C_ = Cfg<N>, bool GRP = false, bool PANEL = false, bool BAND = false>
 __global__ __launch_bounds__(C_::T * C_::LPB) __attribute__((amdgpu_waves_per_eu(C_::WPE_ROW))) void k_row_pass(
     float2* __restrict__ wave, int ny, long long wave_stride, const float2* __restrict__ pgr,
     long long slc_off, long long npg, const int* __restrict__ var_tab, int var_ld, int jslc,
-    const float2* __restrict__ twg, RowChan rc, GrpArgs ga) {
+    const float2* __restrict__ twg, RowChan rc, GrpArgs ga, int gx0, int gx1) {
   static_assert(!GRP || MODE == 0, "grouped row passes carry no real-space readout");
   static_assert(!PANEL || (MODE == 0 && N % kPanel == 0), "panel waves: whole panels, staged batches only");
+  static_assert(!BAND || MODE != 2, "the exit-plane readout reads whole rows");
   using P = typename C_::P;
   constexpr int T = C_::T, LPB = C_::LPB;
   using L = LineLayout<N, C_::PADSH_ROW, C_::SW>;
@@ -178,13 +202,26 @@ __global__ __launch_bounds__(C_::T * C_::LPB) __attribute__((amdgpu_waves_per_eu
   }
   const int row = bx * LPB + line;
   const bool valid = row < ny;
-  // PANEL: element x of the row at (x / 16) * 16 ny + x % 16 from the row start
-  float2* wrow = wave + w * wave_stride + (long long)row * (PANEL ? kPanel : N);
+  // Addresses are a block-uniform base (scalar registers) plus a 32-bit
+  // offset per thread.  PANEL: element x of the row at (x / 16) * 16 ny +
+  // x % 16 from the row start.
+  float2* wblk = wave + w * wave_stride + (long long)bx * LPB * (PANEL ? kPanel : N);
+  const int wline = line * (PANEL ? kPanel : N);
   auto wx = [&](int x) { return PANEL ? (x & ~(kPanel - 1)) * ny + (x & (kPanel - 1)) : x; };
   const int var = MODE == 2 ? 0 : var_tab[w * var_ld + jslc];
-  const float2* grow = pgr + slc_off + (long long)var * npg + (long long)row * N;
+  const float2* gblk = pgr + slc_off + (long long)var * npg + (long long)bx * LPB * N;
   using M0 = IOMap<N, T, P, false>;
   using M1 = IOMap<N, T, P, true>;
+  using BS = BandSlots<N, radix_at<P, false>(0)>;
+  // the wave element of slot q, butterfly b: where q whole slots are a
+  // uniform distance apart, only the first slot's offset is per thread
+  auto wptr = [&](int b, auto Q) {
+    constexpr int q = decltype(Q)::value;
+    if constexpr (!PANEL) return at32(wblk + q * M0::NBF, wline + b);
+    else if constexpr (M0::NBF % kPanel == 0) return at32(wblk + (long long)q * M0::NBF * ny, wline + wx(b));
+    else return at32(wblk, wline + wx(b + q * M0::NBF));
+  };
+  auto stored = [&](int x) { return x < gx0 || x >= gx1; };
   float2 v[NREG];
   if (valid) {
     static_for<0, M0::NB>([&](auto I) {
@@ -193,7 +230,15 @@ __global__ __launch_bounds__(C_::T * C_::LPB) __attribute__((amdgpu_waves_per_eu
       if (M0::FULL || b < M0::NBF) {
         static_for<0, M0::R0>([&](auto Q) {
           constexpr int q = decltype(Q)::value;
-          v[i * M0::R0 + q] = ldg<C_::NT_ROW>(wrow + wx(b + q * M0::NBF));
+          float2& z = v[i * M0::R0 + q];
+          if constexpr (BAND && BS::dead(q)) {
+            z = make_float2(0.f, 0.f);
+          } else if constexpr (BAND && BS::part(q)) {
+            z = make_float2(0.f, 0.f);
+            if (stored(b + q * M0::NBF)) z = ldg<C_::NT_ROW>(wptr(b, Q));
+          } else {
+            z = ldg<C_::NT_ROW>(wptr(b, Q));
+          }
         });
       }
     });
@@ -232,7 +277,7 @@ __global__ __launch_bounds__(C_::T * C_::LPB) __attribute__((amdgpu_waves_per_eu
       if (M1::FULL || b < M1::NBF) {
         static_for<0, M1::R0>([&](auto Q) {
           constexpr int q = decltype(Q)::value;
-          v[i * M1::R0 + q] = cmul(v[i * M1::R0 + q], grow[b + q * M1::NBF]);
+          v[i * M1::R0 + q] = cmul(v[i * M1::R0 + q], *at32(gblk + q * M1::NBF, line * N + b));
         });
       }
     });
@@ -245,7 +290,13 @@ __global__ __launch_bounds__(C_::T * C_::LPB) __attribute__((amdgpu_waves_per_eu
       if (M0::FULL || b < M0::NBF) {
         static_for<0, M0::R0>([&](auto Q) {
           constexpr int q = decltype(Q)::value;
-          stg<C_::NT_ROW>(wrow + wx(b + q * M0::NBF), v[i * M0::R0 + q]);
+          const float2 z = v[i * M0::R0 + q];
+          if constexpr (BAND && BS::dead(q)) {
+          } else if constexpr (BAND && BS::part(q)) {
+            if (stored(b + q * M0::NBF)) stg<C_::NT_ROW>(wptr(b, Q), z);
+          } else {
+            stg<C_::NT_ROW>(wptr(b, Q), z);
+          }
         });
       }
     });
@@ -289,7 +340,7 @@ __device__ __forceinline__ void block_reduce_det(float (&acc)[kMaxDet], int ndet
 //   else : psi <- P * FFT_y(wave)
 //   detect: partial[(w, idet, d, tile)] = sum_{column tile} |psi|^2 * detw[d]
 //   EXIT : store psi(k); else store IFFT_y(psi)
-// grid: (ceil(nx/C), nwave); block: TC*C
+// Two kernels: k_col_pass_w (N <= 768) and k_col_pass_x (1024, 2048).
 // ---------------------------------------------------------------------------
 struct ColArgs {
   int dsx, dsy;             // diffraction de-scan [pixel]: readouts see psi(i + d)
@@ -322,181 +373,23 @@ struct ColArgs {
   const float* detw_t;      // [ndet][nx][ny] detector weights
   const float* cppl_t;      // constant phase plate
   GrpArgs grp;              // grouped launch: wave map and job / plane tables
+  // band-limited waves: tiles [tg0, tg0 + tgn) hold only columns where every
+  // propagator is zero.  They are left out of the launch (block bx >= tg0
+  // takes tile bx + tgn), or, with tclr (EXIT, the wave is kept), cleared.
+  int tg0, tgn, tclr;
+  int keep;                 // EXIT: store psi(k)
 };
 
-template <int N, bool INIT, bool EXIT, class C_ = Cfg<N>>
-__global__ __launch_bounds__(C_::TC * C_::C) void k_col_pass(ColArgs a) {
-  using P = typename C_::PC;
-  constexpr int T = C_::TC, C = C_::C;
-  using L = TileLayout<N, C, C_::PADSH>;
-  constexpr int NREG = regs_needed<N, T, P>();
-  __shared__ float2 s_tw[N];
-  __shared__ float2 s_buf[L::words(1)];
-  const int tid = threadIdx.x;
-  const int c = tid % C, t = tid / C;
-  for (int e = tid; e < N; e += T * C) s_tw[e] = a.twg[e];
-  const long long w = blockIdx.y;
-  const int nx = a.nx;
-  const int x = blockIdx.x * C + c;
-  const bool valid = x < nx;
-  float2* wcol = a.wave + w * a.wave_stride + x;
-  using M0 = IOMap<N, T, P, false>;
-  using M1 = IOMap<N, T, P, true>;
-  float2 v[NREG];
-  if constexpr (INIT) {
-    if (valid) {
-      const float2* s = a.src + w * a.src_stride + x;
-      float dx = 0.f, dy = 0.f, fz = 0.f;
-      const bool pp = a.ppar != nullptr;
-      if (pp) {
-        const float4 q4 = a.ppar[w];
-        dx = q4.x; dy = q4.y; fz = q4.z;
-      }
-      const float kx = (float)fidx(x, nx) * a.kscx;
-      static_for<0, M1::NB>([&](auto I) {
-        constexpr int i = decltype(I)::value;
-        const int b = t + i * T;
-        if (M1::FULL || b < M1::NBF) {
-          static_for<0, M1::R0>([&](auto Q) {
-            constexpr int q = decltype(Q)::value;
-            const int e = b + q * M1::NBF;
-            float2 val = s[(long long)e * nx];
-            if (pp) {
-              const float ky = (float)fidx(e, N) * a.kscy;
-              const float ksqr = kx * kx + ky * ky;
-              float chi = -6.28318531f * (dx * kx + dy * ky + fz * ksqr);
-              if (a.cppl) chi -= a.cppl[(long long)e * nx + x];
-              float sn, cs;
-              sincosf(chi, &sn, &cs);
-              val = cmul(val, make_float2(cs, sn));
-            }
-            v[i * M1::R0 + q] = val;
-          });
-        }
-      });
-    }
-    __syncthreads();
-  } else {
-    if (valid) {
-      static_for<0, M0::NB>([&](auto I) {
-        constexpr int i = decltype(I)::value;
-        const int b = t + i * T;
-        if (M0::FULL || b < M0::NBF) {
-          static_for<0, M0::R0>([&](auto Q) {
-            constexpr int q = decltype(Q)::value;
-            v[i * M0::R0 + q] = wcol[(long long)(b + q * M0::NBF) * nx];
-          });
-        }
-      });
-    }
-    __syncthreads();
-    LineFFT<N, T, -1, P, false, L, NREG, C_::TWR>::run(v, s_buf, c, s_tw, t, SyncBlock{});
-    if (valid) {
-      const float2* pcol = a.pro + x;
-      static_for<0, M1::NB>([&](auto I) {
-        constexpr int i = decltype(I)::value;
-        const int b = t + i * T;
-        if (M1::FULL || b < M1::NBF) {
-          static_for<0, M1::R0>([&](auto Q) {
-            constexpr int q = decltype(Q)::value;
-            v[i * M1::R0 + q] = cmul(v[i * M1::R0 + q], pcol[(long long)(b + q * M1::NBF) * nx]);
-          });
-        }
-      });
-    }
-  }
-  if (a.detect) {
-    float acc[kMaxDet];
-#pragma unroll
-    for (int d = 0; d < kMaxDet; ++d) acc[d] = 0.f;
-    if (valid) {
-      const long long n = (long long)N * nx;
-      // de-scan (DescanDifN, JMultiSlice.cpp:2184-2275): the detectors integrate
-      // psi(i + d), i.e. pixel i is weighted with det(i - d)
-      const int xs = wrap_sub(x, a.dsx, nx);
-      for (int d = 0; d < a.ndet && d < kMaxDet; ++d) {  // uniform loop over detectors
-        const float* dw = a.detw + d * n + xs;
-        float wt[NREG];
-        static_for<0, M1::NB>([&](auto I) {  // all weight loads of this detector first
-          constexpr int i = decltype(I)::value;
-          const int b = t + i * T;
-          static_for<0, M1::R0>([&](auto Q) {
-            constexpr int q = decltype(Q)::value;
-            wt[i * M1::R0 + q] = (M1::FULL || b < M1::NBF)
-                                     ? dw[(long long)wrap_sub(b + q * M1::NBF, a.dsy, N) * nx] : 0.f;
-          });
-        });
-        float sacc = 0.f;
-        static_for<0, M1::NB>([&](auto I) {
-          constexpr int i = decltype(I)::value;
-          const int b = t + i * T;
-          if (M1::FULL || b < M1::NBF) {
-            static_for<0, M1::R0>([&](auto Q) {
-              constexpr int q = decltype(Q)::value;
-              const float2 z = v[i * M1::R0 + q];
-              sacc += (z.x * z.x + z.y * z.y) * wt[i * M1::R0 + q];
-            });
-          }
-        });
-#pragma unroll
-        for (int dd = 0; dd < kMaxDet; ++dd)
-          if (dd == d) acc[dd] += sacc;
-      }
-    }
-    block_reduce_det(acc, a.ndet, (float*)s_buf,
-                     a.partial + w * a.part_wstride + a.part_off + blockIdx.x, a.part_dstride);
-    __syncthreads();
-    if (valid && (a.dif || a.wff || a.dif_avg || a.wff_avg)) {  // ReadoutDifDet_d channels (JMultiSlice.cpp:4310-4356)
-      const float wg = a.cwgt[w];
-      const long long cb = w * a.chan_wstride + a.chan_off;
-      static_for<0, M1::NB>([&](auto I) {
-        constexpr int i = decltype(I)::value;
-        const int b = t + i * T;
-        if (M1::FULL || b < M1::NBF) {
-          static_for<0, M1::R0>([&](auto Q) {
-            constexpr int q = decltype(Q)::value;
-            const long long idx = cb + (long long)wrap_sub(b + q * M1::NBF, a.dsy, N) * nx + wrap_sub(x, a.dsx, nx);
-            const float2 z = v[i * M1::R0 + q];
-            const float pz = z.x * z.x + z.y * z.y;
-            if (a.dif) a.dif[idx] += wg * pz;
-            if (a.dif_avg) a.dif_avg[idx] += wg * pz;
-            if (a.wff) { float2 o = a.wff[idx]; o.x += z.x * wg; o.y += z.y * wg; a.wff[idx] = o; }
-            if (a.wff_avg) { float2 o = a.wff_avg[idx]; o.x += z.x * wg; o.y += z.y * wg; a.wff_avg[idx] = o; }
-          });
-        }
-      });
-    }
-  }
-  if constexpr (EXIT) {
-    if (valid) {
-      static_for<0, M1::NB>([&](auto I) {
-        constexpr int i = decltype(I)::value;
-        const int b = t + i * T;
-        if (M1::FULL || b < M1::NBF) {
-          static_for<0, M1::R0>([&](auto Q) {
-            constexpr int q = decltype(Q)::value;
-            wcol[(long long)(b + q * M1::NBF) * nx] = v[i * M1::R0 + q];
-          });
-        }
-      });
-    }
-  } else {
-    LineFFT<N, T, +1, P, true, L, NREG, C_::TWR>::run(v, s_buf, c, s_tw, t, SyncBlock{});
-    if (valid) {
-      static_for<0, M0::NB>([&](auto I) {
-        constexpr int i = decltype(I)::value;
-        const int b = t + i * T;
-        if (M0::FULL || b < M0::NBF) {
-          static_for<0, M0::R0>([&](auto Q) {
-            constexpr int q = decltype(Q)::value;
-            wcol[(long long)(b + q * M0::NBF) * nx] = v[i * M0::R0 + q];
-          });
-        }
-      });
-    }
-  }
+// the tile of block bx (see ColArgs)
+__device__ __forceinline__ int tile_of(const ColArgs& a, int bx) {
+  return (!a.tclr && bx >= a.tg0) ? bx + a.tgn : bx;
 }
-
+// the readout sums of the tiles left out of a band-limited launch are zero:
+// written by one block of each wave
+__device__ __forceinline__ void clear_gap_partials(const ColArgs& a, long long w, int nthreads) {
+  float* p = a.partial + w * a.part_wstride + a.part_off + a.tg0;
+  for (int i = threadIdx.x; i < a.ndet * a.tgn; i += nthreads) p[(i / a.tgn) * a.part_dstride + i % a.tgn] = 0.f;
+}
 
 // Tile of C adjacent columns x N rows staged through LDS (column c at
 // L::idx(c, e)); thread tid moves elements i = tid + k*BS, i.e. row i / C,
@@ -553,9 +446,13 @@ struct ColTile {
 // output is in LDS), so the body resumes at stage 1.  FOUT: the inverse
 // transform stops after writing its second-to-last stage to LDS; the caller
 // does the last stage.
-template <int N, bool INIT, bool EXIT, bool DET, class C_, bool FIN = false, bool FOUT = false>
+// BAND: the propagators vanish on the rows of the dead slots (BandSlots of
+// the transform's last radix): psi is zero there without the product, and the
+// butterflies on both sides of it are pruned.
+template <int N, bool INIT, bool EXIT, bool DET, class C_, bool FIN = false, bool FOUT = false, bool BAND = false>
 __device__ __forceinline__ void col_body(const ColArgs& a, long long w, float2* s_buf, const float2* s_tw,
-                                         float* s_red, int c, int t, int x, bool valid) {
+                                         float* s_red, int c, int t, int x, int tile, bool valid) {
+  static_assert(!INIT || !BAND, "the incident wave has no propagator");
   using P = typename C_::PC;
   constexpr int T = C_::TW;
   using L = ColLayout<N, C_::PADSH_COL, C_::SW>;
@@ -565,6 +462,8 @@ __device__ __forceinline__ void col_body(const ColArgs& a, long long w, float2* 
   // a column inside one wavefront needs wave barriers only; a column over
   // several wavefronts (T = 128) synchronises the block
   using CS = std::conditional_t<(T <= 64), SyncWave, SyncBlock>;
+  using BSL = BandSlots<N, radix_at<P, true>(0)>;
+  constexpr auto dead = [](int q) { return BAND && BSL::dead(q); };
   const int nx = a.nx;
   const long long n = (long long)N * nx;
   const long long colb = (long long)(valid ? x : x - c) * N;  // column-major offset
@@ -624,7 +523,8 @@ __device__ __forceinline__ void col_body(const ColArgs& a, long long w, float2* 
       if (M1::FULL || b < M1::NBF) {
         static_for<0, M1::R0>([&](auto Q) {
           constexpr int q = decltype(Q)::value;
-          v[i * M1::R0 + q] = cmul(v[i * M1::R0 + q], pcol[b + q * M1::NBF]);
+          if constexpr (dead(q)) v[i * M1::R0 + q] = make_float2(0.f, 0.f);
+          else v[i * M1::R0 + q] = cmul(v[i * M1::R0 + q], pcol[b + q * M1::NBF]);
         });
       }
     });
@@ -656,7 +556,8 @@ __device__ __forceinline__ void col_body(const ColArgs& a, long long w, float2* 
           const int b = t + i * T;
           static_for<0, M1::R0>([&](auto Q) {
             constexpr int q = decltype(Q)::value;
-            wt[i * M1::R0 + q] = (M1::FULL || b < M1::NBF) ? dw[wrap_sub(b + q * M1::NBF, a.dsy, N)] : 0.f;
+            if constexpr (!dead(q))
+              wt[i * M1::R0 + q] = (M1::FULL || b < M1::NBF) ? dw[wrap_sub(b + q * M1::NBF, a.dsy, N)] : 0.f;
           });
         });
         float sacc = 0.f;
@@ -666,7 +567,7 @@ __device__ __forceinline__ void col_body(const ColArgs& a, long long w, float2* 
           if (M1::FULL || b < M1::NBF) {
             static_for<0, M1::R0>([&](auto Q) {
               constexpr int q = decltype(Q)::value;
-              sacc += pw[i * M1::R0 + q] * wt[i * M1::R0 + q];
+              if constexpr (!dead(q)) sacc += pw[i * M1::R0 + q] * wt[i * M1::R0 + q];
             });
           }
         });
@@ -675,8 +576,7 @@ __device__ __forceinline__ void col_body(const ColArgs& a, long long w, float2* 
           if (dd == d) acc[dd] += sacc;
       }
     }
-    block_reduce_det(acc, a.ndet, s_red, a.partial + w * a.part_wstride + a.part_off + blockIdx.x,
-                     a.part_dstride);
+    block_reduce_det(acc, a.ndet, s_red, a.partial + w * a.part_wstride + a.part_off + tile, a.part_dstride);
     if (valid && (a.dif || a.wff || a.dif_avg || a.wff_avg)) {  // ReadoutDifDet_d channels (JMultiSlice.cpp:4310-4356)
       const float wg = a.cwgt[w];
       const long long cb = w * a.chan_wstride + a.chan_off;
@@ -686,6 +586,7 @@ __device__ __forceinline__ void col_body(const ColArgs& a, long long w, float2* 
         if (M1::FULL || b < M1::NBF) {
           static_for<0, M1::R0>([&](auto Q) {
             constexpr int q = decltype(Q)::value;
+            if constexpr (dead(q)) return;
             const long long idx = cb + (long long)wrap_sub(b + q * M1::NBF, a.dsy, N) * nx + wrap_sub(x, a.dsx, nx);
             const float2 z = v[i * M1::R0 + q];
             const float pz = z.x * z.x + z.y * z.y;
@@ -739,7 +640,8 @@ __device__ __forceinline__ void col_body(const ColArgs& a, long long w, float2* 
 // cppl_t) so that the lanes of a column access them contiguously.
 // grid: (ceil(nx/CW), nwave); block: TW*CW
 // ---------------------------------------------------------------------------
-template <int N, bool INIT, bool EXIT, bool DET, class C_ = Cfg<N>, bool GRP = false, bool PANEL = false>
+template <int N, bool INIT, bool EXIT, bool DET, class C_ = Cfg<N>, bool GRP = false, bool PANEL = false,
+          bool BAND = false>
 __global__ __launch_bounds__(C_::TW * C_::CW) __attribute__((amdgpu_waves_per_eu(C_::WPE_COL))) void k_col_pass_w(
     ColArgs a0) {
   constexpr int T = C_::TW, C = C_::CW, BS = T * C;
@@ -781,8 +683,10 @@ __global__ __launch_bounds__(C_::TW * C_::CW) __attribute__((amdgpu_waves_per_eu
     if constexpr (!INIT) a.pro_t = (const float2*)pl[a0.grp.step - 1].pro_t;
   }
   const int nx = a.nx;
-  const int x0 = blockIdx.x * C;
+  const int tile = tile_of(a, blockIdx.x);
+  const int x0 = tile * C;
   const int ncol = (nx - x0 < C) ? (nx - x0) : C;
+  if (DET && a.detect && blockIdx.x == 0) clear_gap_partials(a, w, BS);
   // PANEL: the waves are stored in panels of 16 columns (element (y, x) at
   // (x / 16) * 16 N + 16 y + x % 16), so the rows of a tile are contiguous
   static_assert(!PANEL || C <= kPanel, "a panel holds whole tiles");
@@ -800,6 +704,14 @@ __global__ __launch_bounds__(C_::TW * C_::CW) __attribute__((amdgpu_waves_per_eu
   constexpr bool FIO = C_::FIO && P::S >= 2 && N / radix_at<P, false>(0) == T && TL::KST == NREG;
   constexpr bool FIN = FIO && !INIT, FOUT = FIO && !EXIT;
   const int cs = tid % C, bs = tid / C;  // sweep mapping: column, first-stage butterfly
+  if constexpr (EXIT) {
+    if (a.tclr && tile >= a.tg0 && tile < a.tg0 + a.tgn) {  // uniform over the block
+      float2 st[TL::KST];
+      static_for<0, TL::KST>([&](auto K) { st[decltype(K)::value] = make_float2(0.f, 0.f); });
+      TL::store(st, wv_base, wrs, ncol, tid);
+      return;
+    }
+  }
   {
     float2 st[TL::KST];
     TL::load(st, INIT ? (a.src + w * a.src_stride + x0) : wv_base, INIT ? nx : wrs, ncol, tid);
@@ -811,7 +723,10 @@ __global__ __launch_bounds__(C_::TW * C_::CW) __attribute__((amdgpu_waves_per_eu
     }
   }
   __syncthreads();
-  col_body<N, INIT, EXIT, DET, C_, FIN, FOUT>(a, w, s_buf, s_tw, s_red, c, t, x0 + c, c < ncol);
+  col_body<N, INIT, EXIT, DET, C_, FIN, FOUT, BAND && !INIT>(a, w, s_buf, s_tw, s_red, c, t, x0 + c, tile, c < ncol);
+  if constexpr (EXIT) {
+    if (!a.keep) return;
+  }
   __syncthreads();
   {
     float2 st[TL::KST];
@@ -852,25 +767,6 @@ __global__ __launch_bounds__(C_::TW * C_::CW) __attribute__((amdgpu_waves_per_eu
 // map, whose job and plane tables supply the buffers and tables.
 // grid: (ceil(nx/CT), nwave); block: 64*CT
 // ---------------------------------------------------------------------------
-// the value of x, hidden from the optimiser: table reads indexed with it are
-// repeated where they are needed instead of being kept live in registers
-// from an earlier identical read
-__device__ __forceinline__ int opaque(int x) {
-  __asm__ volatile("" : "+v"(x));
-  return x;
-}
-
-// base[idx] addressed by a 32-bit byte offset (idx * sizeof(T) < 2^32), so
-// that a wavefront-uniform base stays in scalar registers
-template <class T>
-__device__ __forceinline__ T* at32(T* base, int idx) {
-  return reinterpret_cast<T*>(reinterpret_cast<char*>(base) + (unsigned)(idx * (int)sizeof(T)));
-}
-template <class T>
-__device__ __forceinline__ const T* at32(const T* base, int idx) {
-  return reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + (unsigned)(idx * (int)sizeof(T)));
-}
-
 // v[k] *= W_N^(DIR * n1 * k), k = 1..M-1, N = 64*M, from two exact table
 // reads per factor: W^(n1*(8a + b)) = W^(8a*n1) * W^(b*n1) (n1*k < N); tw
 // holds the first half of the table, W^(e + N/2) = -W^e
@@ -947,8 +843,10 @@ __global__ __launch_bounds__(64 * C_::XCT) __attribute__((amdgpu_waves_per_eu(4)
     if constexpr (!INIT) a.pro = (const float2*)pl[a0.grp.step - 1].pro;
   }
   const int nx = a.nx;
-  const int x0 = bx * CT;
+  const int tile = tile_of(a, bx);
+  const int x0 = tile * CT;
   const int ncol = (nx - x0 < CT) ? (nx - x0) : CT;
+  if (DET && a.detect && bx == 0) clear_gap_partials(a, w, NT);
   // PANEL: the tile lies in one panel (element (y, x) at p N + 16 y + x - p,
   // p = x0 rounded down to a multiple of 16)
   static_assert(!PANEL || kPanel % CT == 0, "a tile lies in one panel");
@@ -986,6 +884,13 @@ __global__ __launch_bounds__(64 * C_::XCT) __attribute__((amdgpu_waves_per_eu(4)
   const long long rstep = (long long)M * nx;  // elements from slot c to c + 1
   // A layout: row n1 + 64*n2 = (uniform row 64*n2) + per-thread offset
   const long long astep = 64LL * wrs;
+  if constexpr (EXIT) {
+    if (a.tclr && tile >= a.tg0 && tile < a.tg0 + a.tgn) {  // uniform over the block
+      if (ca < ncol)
+        for (int n2 = 0; n2 < M; ++n2) *at32(wbase + n2 * astep, n1 * wrs + ca) = make_float2(0.f, 0.f);
+      return;
+    }
+  }
   float2 v[M];  // A: v[n2] (rows n1 + 64*n2); B: v[16r + c]
   if constexpr (!INIT) {
     static_for<0, M>([&](auto I) {
@@ -1095,7 +1000,7 @@ __global__ __launch_bounds__(64 * C_::XCT) __attribute__((amdgpu_waves_per_eu(4)
       }
     }
     if constexpr (EXIT) {
-      if (validb) {
+      if (validb && a.keep) {
         float2* wv0 = PANEL ? wbase + 16 * r * kPanel : a.wave + w * a.wave_stride + 16 * r * nx;
         const long long rs_w = PANEL ? (long long)M * kPanel : rstep;
         const int ob_w = PANEL ? kyb * kPanel + cb : ob;
@@ -1108,7 +1013,7 @@ __global__ __launch_bounds__(64 * C_::XCT) __attribute__((amdgpu_waves_per_eu(4)
   });
   if constexpr (DET) {
     if (a.detect)  // uniform over the block (one wave)
-      block_reduce_det(acc, a.ndet, s_red, a.partial + w * a.part_wstride + a.part_off + bx, a.part_dstride);
+      block_reduce_det(acc, a.ndet, s_red, a.partial + w * a.part_wstride + a.part_off + tile, a.part_dstride);
   }
   if constexpr (!EXIT) {
     static_for<0, R>([&](auto RR) {
@@ -1249,59 +1154,69 @@ template <int N>
 hipError_t launch_row_pass_n(int ny, int nwave, float2* wave, long long wave_stride,
                              const float2* pgr, long long slc_off, long long npg,
                              const int* var_tab, int var_ld, int jslc, const float2* twx,
-                             const RowChanHost& h, int mode, bool panel, hipStream_t st) {
+                             const RowChanHost& h, int mode, bool panel, const BandHost& bd, hipStream_t st) {
   dim3 g((ny + Cfg<N>::LPB - 1) / Cfg<N>::LPB, nwave), b(Cfg<N>::T * Cfg<N>::LPB);
   RowChan rc;
   rc.img = h.img; rc.img_avg = h.img_avg;
   rc.wfr = (float2*)h.wfr; rc.wfr_avg = (float2*)h.wfr_avg;
   rc.cwgt = h.cwgt; rc.chan_wstride = h.chan_wstride; rc.chan_off = h.chan_off;
   if (panel && (mode != 0 || !Cfg<N>::PANEL)) return hipErrorInvalidValue;
-  if (mode == 1)
-    hipLaunchKernelGGL((k_row_pass<N, 1>), g, b, 0, st, wave, ny, wave_stride, pgr, slc_off, npg,
-                       var_tab, var_ld, jslc, twx, rc, GrpArgs{});
-  else if (mode == 2)
-    hipLaunchKernelGGL((k_row_pass<N, 2>), g, b, 0, st, wave, ny, wave_stride, pgr, slc_off, npg,
-                       var_tab, var_ld, jslc, twx, rc, GrpArgs{});
-  else if (!panel)
-    hipLaunchKernelGGL((k_row_pass<N, 0>), g, b, 0, st, wave, ny, wave_stride, pgr, slc_off, npg,
-                       var_tab, var_ld, jslc, twx, rc, GrpArgs{});
-  else if constexpr (Cfg<N>::PANEL)
-    hipLaunchKernelGGL((k_row_pass<N, 0, Cfg<N>, false, true>), g, b, 0, st, wave, ny, wave_stride, pgr, slc_off,
-                       npg, var_tab, var_ld, jslc, twx, rc, GrpArgs{});
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, g, b, 0, st, wave, ny, wave_stride, pgr, slc_off, npg, var_tab, var_ld, jslc, twx, rc,
+                       GrpArgs{}, bd.x0, bd.x1);
+  };
+  using CF = Cfg<N>;
+  const bool band = bd.on();
+  if (mode == 2) go(k_row_pass<N, 2>);
+  else if (mode == 1 && band) go(k_row_pass<N, 1, CF, false, false, true>);
+  else if (mode == 1) go(k_row_pass<N, 1>);
+  else if (!panel && band) go(k_row_pass<N, 0, CF, false, false, true>);
+  else if (!panel) go(k_row_pass<N, 0>);
+  else if constexpr (CF::PANEL) {
+    if (band) go(k_row_pass<N, 0, CF, false, true, true>);
+    else go(k_row_pass<N, 0, CF, false, true>);
+  }
   return hipGetLastError();
 }
 
 // grouped row pass (waves of several jobs, one slice step)
 template <int N>
 hipError_t launch_row_pass_grp_n(int ny, int nwave, long long wave_stride, long long npg, const float2* twx,
-                                 const GrpArgs& ga, bool panel, hipStream_t st) {
-  dim3 g((ny + Cfg<N>::LPB - 1) / Cfg<N>::LPB, nwave), b(Cfg<N>::T * Cfg<N>::LPB);
-  if (panel && !Cfg<N>::PANEL) return hipErrorInvalidValue;
-  if (!panel)
-    hipLaunchKernelGGL((k_row_pass<N, 0, Cfg<N>, true>), g, b, 0, st, nullptr, ny, wave_stride, nullptr, 0LL, npg,
-                       nullptr, 0, ga.step, twx, RowChan{}, ga);
-  else if constexpr (Cfg<N>::PANEL)
-    hipLaunchKernelGGL((k_row_pass<N, 0, Cfg<N>, true, true>), g, b, 0, st, nullptr, ny, wave_stride, nullptr, 0LL,
-                       npg, nullptr, 0, ga.step, twx, RowChan{}, ga);
+                                 const GrpArgs& ga, bool panel, const BandHost& bd, hipStream_t st) {
+  using CF = Cfg<N>;
+  dim3 g((ny + CF::LPB - 1) / CF::LPB, nwave), b(CF::T * CF::LPB);
+  if (panel && !CF::PANEL) return hipErrorInvalidValue;
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, g, b, 0, st, nullptr, ny, wave_stride, nullptr, 0LL, npg, nullptr, 0, ga.step, twx,
+                       RowChan{}, ga, bd.x0, bd.x1);
+  };
+  const bool band = bd.on();
+  if (!panel && band) go(k_row_pass<N, 0, CF, true, false, true>);
+  else if (!panel) go(k_row_pass<N, 0, CF, true>);
+  else if constexpr (CF::PANEL) {
+    if (band) go(k_row_pass<N, 0, CF, true, true, true>);
+    else go(k_row_pass<N, 0, CF, true, true>);
+  }
   return hipGetLastError();
 }
 
 // the column kernels' instantiations by pass kind (INIT, EXIT, readout)
 template <int N, class CF, bool GRP, bool PANEL>
-void launch_col_w(dim3 g, dim3 b, bool init, bool exit_, bool detect, const ColArgs& a, hipStream_t st) {
+void launch_col_w(dim3 g, dim3 b, bool init, bool exit_, bool detect, bool band, const ColArgs& a, hipStream_t st) {
   // detection planes get their own instantiation: the readout's registers
   // would otherwise halve the occupancy of every other slice
-  if (detect) {
-    if (init && exit_) hipLaunchKernelGGL((k_col_pass_w<N, true, true, true, CF, GRP, PANEL>), g, b, 0, st, a);
-    else if (init) hipLaunchKernelGGL((k_col_pass_w<N, true, false, true, CF, GRP, PANEL>), g, b, 0, st, a);
-    else if (exit_) hipLaunchKernelGGL((k_col_pass_w<N, false, true, true, CF, GRP, PANEL>), g, b, 0, st, a);
-    else hipLaunchKernelGGL((k_col_pass_w<N, false, false, true, CF, GRP, PANEL>), g, b, 0, st, a);
-  } else {
-    if (init && exit_) hipLaunchKernelGGL((k_col_pass_w<N, true, true, false, CF, GRP, PANEL>), g, b, 0, st, a);
-    else if (init) hipLaunchKernelGGL((k_col_pass_w<N, true, false, false, CF, GRP, PANEL>), g, b, 0, st, a);
-    else if (exit_) hipLaunchKernelGGL((k_col_pass_w<N, false, true, false, CF, GRP, PANEL>), g, b, 0, st, a);
-    else hipLaunchKernelGGL((k_col_pass_w<N, false, false, false, CF, GRP, PANEL>), g, b, 0, st, a);
-  }
+  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, g, b, 0, st, a); };
+  auto pick = [&](auto D) {
+    constexpr bool DET = decltype(D)::value;
+    if (init && exit_) go(k_col_pass_w<N, true, true, DET, CF, GRP, PANEL>);
+    else if (init) go(k_col_pass_w<N, true, false, DET, CF, GRP, PANEL>);
+    else if (exit_ && band) go(k_col_pass_w<N, false, true, DET, CF, GRP, PANEL, true>);
+    else if (exit_) go(k_col_pass_w<N, false, true, DET, CF, GRP, PANEL>);
+    else if (band) go(k_col_pass_w<N, false, false, DET, CF, GRP, PANEL, true>);
+    else go(k_col_pass_w<N, false, false, DET, CF, GRP, PANEL>);
+  };
+  if (detect) pick(std::true_type{});
+  else pick(std::false_type{});
 }
 template <int N, class CF, bool PANEL, bool GRP = false>
 void launch_col_x(dim3 g, dim3 b, bool init, bool exit_, bool detect, const ColArgs& a, hipStream_t st) {
@@ -1336,22 +1251,22 @@ hipError_t launch_col_pass_n(int nwave, bool init, bool exit_, const ColArgsHost
   a.detw_t = h.detw_t;
   a.cppl_t = h.cppl_t;
   using CF = Cfg<N>;
+  static_assert(CF::XL || CF::WL, "every line length has a column kernel");
   if (h.panel && !CF::PANEL) return hipErrorInvalidValue;
+  const int tiles = (h.nx + CF::CC - 1) / CF::CC;
+  a.tg0 = h.band.x0 / CF::CC;
+  a.tgn = h.band.on() ? (h.band.x1 - h.band.x0) / CF::CC : 0;
+  a.keep = h.keep;
+  a.tclr = exit_ && h.keep;
+  dim3 g(a.tclr ? tiles : tiles - a.tgn, nwave);
   if constexpr (CF::XL) {
-    dim3 g((h.nx + CF::XCT - 1) / CF::XCT, nwave), b(64 * CF::XCT);
+    dim3 b(64 * CF::XCT);
     if (!h.panel) launch_col_x<N, CF, false>(g, b, init, exit_, h.detect, a, st);
     else if constexpr (CF::PANEL) launch_col_x<N, CF, true>(g, b, init, exit_, h.detect, a, st);
-  } else if constexpr (CF::WL) {
-    dim3 g((h.nx + CF::CW - 1) / CF::CW, nwave), b(CF::TW * CF::CW);
-    if (!h.panel) launch_col_w<N, CF, false, false>(g, b, init, exit_, h.detect, a, st);
-    else if constexpr (CF::PANEL) launch_col_w<N, CF, false, true>(g, b, init, exit_, h.detect, a, st);
   } else {
-    if (h.panel) return hipErrorInvalidValue;
-    dim3 g((h.nx + CF::C - 1) / CF::C, nwave), b(CF::TC * CF::C);
-    if (init && exit_) hipLaunchKernelGGL((k_col_pass<N, true, true>), g, b, 0, st, a);
-    else if (init) hipLaunchKernelGGL((k_col_pass<N, true, false>), g, b, 0, st, a);
-    else if (exit_) hipLaunchKernelGGL((k_col_pass<N, false, true>), g, b, 0, st, a);
-    else hipLaunchKernelGGL((k_col_pass<N, false, false>), g, b, 0, st, a);
+    dim3 b(CF::TW * CF::CW);
+    if (!h.panel) launch_col_w<N, CF, false, false>(g, b, init, exit_, h.detect, h.band.rows, a, st);
+    else if constexpr (CF::PANEL) launch_col_w<N, CF, false, true>(g, b, init, exit_, h.detect, h.band.rows, a, st);
   }
   return hipGetLastError();
 }
@@ -1360,34 +1275,45 @@ hipError_t launch_col_pass_n(int nwave, bool init, bool exit_, const ColArgsHost
 // long-column kernel)
 template <int N>
 hipError_t launch_col_pass_grp_n(int nx, int nwave, bool init, bool exit_, bool detect, long long part_dstride,
-                                 const float2* twy, const GrpArgs& ga, bool panel, hipStream_t st) {
+                                 const float2* twy, const GrpArgs& ga, bool panel, const BandHost& bd,
+                                 hipStream_t st) {
   using CF = Cfg<N>;
+  if (panel && (CF::XL || !CF::PANEL)) return hipErrorInvalidValue;
+  ColArgs a{};
+  a.nx = nx;
+  a.wave_stride = (long long)N * nx;
+  a.part_dstride = part_dstride;
+  a.twg = twy;
+  a.grp = ga;
+  a.tg0 = bd.x0 / CF::CC;
+  a.tgn = bd.on() ? (bd.x1 - bd.x0) / CF::CC : 0;
+  dim3 g((nx + CF::CC - 1) / CF::CC - a.tgn, nwave);
   if constexpr (CF::XL) {
-    if (panel) return hipErrorInvalidValue;
-    ColArgs a{};
-    a.nx = nx;
-    a.wave_stride = (long long)N * nx;
-    a.part_dstride = part_dstride;
-    a.twg = twy;
-    a.grp = ga;
-    dim3 g((nx + CF::XCT - 1) / CF::XCT, nwave), b(64 * CF::XCT);
-    launch_col_x<N, CF, false, true>(g, b, init, exit_, detect, a, st);
-    return hipGetLastError();
-  } else if constexpr (CF::WL) {
-    if (panel && !CF::PANEL) return hipErrorInvalidValue;
-    ColArgs a{};
-    a.nx = nx;
-    a.wave_stride = (long long)N * nx;
-    a.part_dstride = part_dstride;
-    a.twg = twy;
-    a.grp = ga;
-    dim3 g((nx + CF::CW - 1) / CF::CW, nwave), b(CF::TW * CF::CW);
-    if (!panel) launch_col_w<N, CF, true, false>(g, b, init, exit_, detect, a, st);
-    else if constexpr (CF::PANEL) launch_col_w<N, CF, true, true>(g, b, init, exit_, detect, a, st);
-    return hipGetLastError();
+    launch_col_x<N, CF, false, true>(g, dim3(64 * CF::XCT), init, exit_, detect, a, st);
   } else {
-    return hipErrorInvalidValue;
+    dim3 b(CF::TW * CF::CW);
+    if (!panel) launch_col_w<N, CF, true, false>(g, b, init, exit_, detect, bd.rows, a, st);
+    else if constexpr (CF::PANEL) launch_col_w<N, CF, true, true>(g, b, init, exit_, detect, bd.rows, a, st);
   }
+  return hipGetLastError();
+}
+
+// the part of a zero gap (columns [x0, x1), rows [y0, y1) where every
+// propagator vanishes) that the passes of an NX-point row / NY-point column
+// can leave out
+template <int NX>
+void band_row_n(int x0, int x1, int tile, BandHost& b) {
+  using BS = BandSlots<NX, radix_at<typename Cfg<NX>::P, false>(0)>;
+  const int g0 = (std::max(x0, BS::G0_MIN) + tile - 1) / tile * tile, g1 = std::min(x1, BS::G1_MAX) / tile * tile;
+  if (g0 < g1 && g0 <= BS::G0_MAX && g1 >= BS::G1_MIN) {
+    b.x0 = g0;
+    b.x1 = g1;
+  }
+}
+template <int NY>
+bool band_col_n(int y0, int y1) {
+  using BS = BandSlots<NY, radix_at<typename Cfg<NY>::PC, true>(0)>;
+  return BS::G0_MAX < BS::G1_MIN && y0 <= BS::G0_MAX && y1 >= BS::G1_MIN;
 }
 
 template <int N>

@@ -77,6 +77,16 @@ struct Bufs {
   int nw;
 };
 
+// the gap of band-limited waves (propagators zero beyond N/3) in column tiles
+// of CF; the variants are timed on such waves, as the slice loop runs them
+template <class CF>
+BandHost gap_of() {
+  BandHost b;
+  band_row_n<N>(N / 3 + 1, N - N / 3, CF::CC, b);
+  b.rows = band_col_n<N>(N / 3 + 1, N - N / 3);
+  return b;
+}
+
 template <class CF, bool PANEL = false>
 float time_row(const Bufs& b, int reps) {
   dim3 g((N + CF::LPB - 1) / CF::LPB, b.nw), bl(CF::T * CF::LPB);
@@ -85,9 +95,15 @@ float time_row(const Bufs& b, int reps) {
   (void)hipEventCreate(&e0);
   (void)hipEventCreate(&e1);
   (void)hipEventRecord(e0);
-  for (int i = 0; i < reps; ++i)
-    hipLaunchKernelGGL((k_row_pass<N, 0, CF, false, PANEL>), g, bl, 0, 0, b.w, N, (long long)N * N, b.pg, 0LL,
-                       (long long)N * N, b.var, 1, 0, b.tw, rc, GrpArgs{});
+  const BandHost bd = gap_of<CF>();
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, g, bl, 0, 0, b.w, N, (long long)N * N, b.pg, 0LL, (long long)N * N, b.var, 1, 0, b.tw,
+                       rc, GrpArgs{}, bd.x0, bd.x1);
+  };
+  for (int i = 0; i < reps; ++i) {
+    if (bd.on()) go(k_row_pass<N, 0, CF, false, PANEL, true>);
+    else go(k_row_pass<N, 0, CF, false, PANEL>);
+  }
   (void)hipEventRecord(e1);
   (void)hipEventSynchronize(e1);
   float ms = 0.f;
@@ -100,20 +116,22 @@ template <class CF, bool PANEL = false>
 float time_col(const Bufs& b, int reps) {
   ColArgs a{};
   a.wave = b.w; a.nx = N; a.wave_stride = (long long)N * N; a.pro = b.pro; a.pro_t = b.pro; a.twg = b.tw;
+  const BandHost bd = gap_of<CF>();
+  a.tg0 = bd.x0 / CF::CC;
+  a.tgn = bd.on() ? (bd.x1 - bd.x0) / CF::CC : 0;
+  const dim3 g((N + CF::CC - 1) / CF::CC - a.tgn, b.nw);
   hipEvent_t e0, e1;
   (void)hipEventCreate(&e0);
   (void)hipEventCreate(&e1);
   (void)hipEventRecord(e0);
   for (int i = 0; i < reps; ++i) {
     if constexpr (CF::XL) {
-      hipLaunchKernelGGL((k_col_pass_x<N, false, false, false, CF, PANEL>), dim3((N + CF::XCT - 1) / CF::XCT, b.nw),
-                         dim3(64 * CF::XCT), 0, 0, a);
-    } else if constexpr (CF::WL) {
-      hipLaunchKernelGGL((k_col_pass_w<N, false, false, false, CF, false, PANEL>), dim3((N + CF::CW - 1) / CF::CW, b.nw),
-                         dim3(CF::TW * CF::CW), 0, 0, a);
+      hipLaunchKernelGGL((k_col_pass_x<N, false, false, false, CF, PANEL>), g, dim3(64 * CF::XCT), 0, 0, a);
+    } else if (bd.rows) {
+      hipLaunchKernelGGL((k_col_pass_w<N, false, false, false, CF, false, PANEL, true>), g, dim3(CF::TW * CF::CW), 0,
+                         0, a);
     } else {
-      hipLaunchKernelGGL((k_col_pass<N, false, false, CF>), dim3((N + CF::C - 1) / CF::C, b.nw),
-                         dim3(CF::TC * CF::C), 0, 0, a);
+      hipLaunchKernelGGL((k_col_pass_w<N, false, false, false, CF, false, PANEL>), g, dim3(CF::TW * CF::CW), 0, 0, a);
     }
   }
   (void)hipEventRecord(e1);
