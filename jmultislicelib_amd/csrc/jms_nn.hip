@@ -273,8 +273,25 @@ __global__ __launch_bounds__(256) void k_loss(const float* __restrict__ y, const
   }
 }
 
+// the bf16 copy of parameter i in fragment order (nnmfma), for the weights that
+// have one
+__device__ __forceinline__ void store_packed(int i, uint16_t h, uint16_t* __restrict__ pack) {
+#pragma unroll
+  for (int l = 0; l < NCONV; ++l) {
+    const int e = i - off_cw(l), ci_n = CIN[l];
+    if (e >= 0 && e < conv_w(l)) {
+      const int co = e / (ci_n * 9), ci = e / 9 % ci_n, tap = e % 9;
+      pack[nnmfma::conv_pack(l, ci_n, co, ci, tap)] = h;
+      return;
+    }
+  }
+  const int e = i - OFF_D1W;
+  if (e >= 0 && e < HID * FLAT) pack[nnmfma::PACK_D1 + ((e % FLAT / 8) * HID + e / FLAT) * 8 + e % 8] = h;
+}
+
 __global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
-                       float* __restrict__ v, uint16_t* __restrict__ pbf, int np, float lr, float bc1, float bc2) {
+                       float* __restrict__ v, uint16_t* __restrict__ pbf, uint16_t* __restrict__ pack, int np,
+                       float lr, float bc1, float bc2) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= np) return;
   const float gi = g[i];
@@ -284,7 +301,9 @@ __global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float
   v[i] = vi;
   const float q = p[i] - lr * (mi / bc1) / (sqrtf(vi / bc2) + 1e-8f);
   p[i] = q;
-  pbf[i] = f2bf(q);
+  const uint16_t h = f2bf(q);
+  pbf[i] = h;
+  store_packed(i, h, pack);
 }
 
 __global__ void k_zero(float* __restrict__ p, int np) {
@@ -292,9 +311,13 @@ __global__ void k_zero(float* __restrict__ p, int np) {
   if (i < np) p[i] = 0.f;
 }
 
-__global__ void k_to_bf16(const float* __restrict__ p, uint16_t* __restrict__ q, int np) {
+__global__ void k_to_bf16(const float* __restrict__ p, uint16_t* __restrict__ q, uint16_t* __restrict__ pack,
+                          int np) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < np) q[i] = f2bf(p[i]);
+  if (i >= np) return;
+  const uint16_t h = f2bf(p[i]);
+  q[i] = h;
+  store_packed(i, h, pack);
 }
 
 // batch gather: xb[j] = X[idx[j]], tb[j] = T[idx[j]]
@@ -358,6 +381,12 @@ struct jms_nn {
   hipStream_t st = nullptr;
   float *p = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;
   uint16_t* pbf = nullptr;
+  uint16_t* pack = nullptr;       // bf16 weights in fragment order (nnmfma::PACK_SIZE)
+  int cus = 256;                  // compute units of the device
+  uint16_t* feat = nullptr;       // conv features of a prediction, capacity feat_cap samples
+  int feat_cap = 0;
+  float* pout = nullptr;          // outputs of a prediction, capacity pout_cap samples
+  int pout_cap = 0;
   uint16_t* act[NCONV + 2] = {};  // input, conv1..conv4, dense1
   float* out = nullptr;           // [maxb][3]
   float* gbuf[NCONV + 2] = {};    // gradient w.r.t. conv1..4 outputs, dense1 output, final output
@@ -394,6 +423,7 @@ hipError_t dalloc(T** p, size_t n) { return hipMalloc((void**)p, n * sizeof(T));
 void release(jms_nn* m) {
   if (!m) return;
   (void)hipFree(m->p); (void)hipFree(m->g); (void)hipFree(m->m); (void)hipFree(m->v); (void)hipFree(m->pbf);
+  (void)hipFree(m->pack); (void)hipFree(m->feat); (void)hipFree(m->pout);
   for (auto* a : m->act) (void)hipFree(a);
   for (auto* a : m->gbuf) (void)hipFree(a);
   (void)hipFree(m->out); (void)hipFree(m->tb); (void)hipFree(m->scale); (void)hipFree(m->loss_part);
@@ -445,9 +475,30 @@ void conv_bwd_mfma(jms_nn* m, int l, int n) {
   }
 }
 
-// forward over act[0] (n samples) -> out
-// forward pass of n samples: input act[0] (or in0: n windows in place),
-// output [n][3] into out (default m->out)
+// the dense head of n samples: hidden units (kept when hid is given), outputs
+void head_mfma(jms_nn* m, int n, const uint16_t* feat, uint16_t* hid, float* out) {
+  auto go = [&](auto kern, int ns) {
+    hipLaunchKernelGGL(kern, dim3(nblk(n, 16 * ns)), dim3(1024), 0, m->st, feat, m->pack + nnmfma::PACK_D1,
+                       m->p + OFF_D1B, m->pbf + OFF_D2W, m->p + OFF_D2B, n, hid, out);
+  };
+  // four samples share a weight read; one where four would leave CUs without
+  // a block
+  if (n >= 64 * m->cus) go(nnmfma::k_head<4>, 4);
+  else go(nnmfma::k_head<1>, 1);
+}
+
+// outputs [n][3] of n windows x on the matrix cores, without intermediates;
+// feat: n x 512 features
+hipError_t infer_mfma(jms_nn* m, int n, const uint16_t* x, uint16_t* feat, float* out) {
+  hipLaunchKernelGGL((nnmfma::k_net_fwd<false>), dim3(std::min(n, m->cus)), dim3(nnmfma::NET_THREADS), 0, m->st, x,
+                     m->pack, m->p + off_cb(0), m->p + off_cb(1), m->p + off_cb(2), m->p + off_cb(3), n, feat,
+                     (uint16_t*)nullptr, (uint16_t*)nullptr, (uint16_t*)nullptr);
+  head_mfma(m, n, feat, nullptr, out);
+  return hipGetLastError();
+}
+
+// forward pass of n samples with the activations kept: input act[0] (or in0:
+// n windows in place), output [n][3] into out (default m->out)
 hipError_t forward(jms_nn* m, int n, const uint16_t* in0 = nullptr, float* out = nullptr) {
   for (int l = 0; l < NCONV; ++l) {
     if (m->mfma) {
@@ -561,6 +612,12 @@ int jms_nn_create(jms_nn** out, int max_batch, unsigned int seed) {
   if (e == hipSuccess) e = dalloc(&m->m, NPARAM);
   if (e == hipSuccess) e = dalloc(&m->v, NPARAM);
   if (e == hipSuccess) e = dalloc(&m->pbf, NPARAM);
+  if (e == hipSuccess) e = dalloc(&m->pack, nnmfma::PACK_SIZE);
+  if (e == hipSuccess) e = hipMemsetAsync(m->pack, 0, nnmfma::PACK_SIZE * 2, m->st);  // unused K groups of conv 1
+  int dev = 0, cus = 0;
+  if (e == hipSuccess) e = hipGetDevice(&dev);
+  if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  if (cus > 0) m->cus = cus;
   for (int l = 0; l < NCONV + 2 && e == hipSuccess; ++l) e = dalloc(&m->act[l], (size_t)max_batch * act_size(l));
   const int gsz[NCONV + 2] = {act_size(1), act_size(2), act_size(3), act_size(4), HID, NOUT};
   for (int l = 0; l < NCONV + 2 && e == hipSuccess; ++l) e = dalloc(&m->gbuf[l], (size_t)max_batch * gsz[l]);
@@ -602,7 +659,7 @@ int jms_nn_set_params(jms_nn* m, const float* in) {
   if (e == hipSuccess) e = hipMemsetAsync(m->m, 0, NPARAM * sizeof(float), m->st);
   if (e == hipSuccess) e = hipMemsetAsync(m->v, 0, NPARAM * sizeof(float), m->st);
   if (e == hipSuccess) {
-    hipLaunchKernelGGL(k_to_bf16, dim3(nblk(NPARAM, 256)), dim3(256), 0, m->st, m->p, m->pbf, NPARAM);
+    hipLaunchKernelGGL(k_to_bf16, dim3(nblk(NPARAM, 256)), dim3(256), 0, m->st, m->p, m->pbf, m->pack, NPARAM);
     e = hipGetLastError();
   }
   if (e == hipSuccess) e = hipStreamSynchronize(m->st);
@@ -620,7 +677,7 @@ int jms_nn_get_params(jms_nn* m, float* out) {
 int jms_nn_forward(jms_nn* m, const uint16_t* x, int n, float* out) {
   if (!m || !x || !out || n < 1 || n > m->maxb) return 1;
   hipError_t e = hipMemcpyAsync(m->act[0], x, (size_t)n * IN_SIZE * 2, hipMemcpyHostToDevice, m->st);
-  if (e == hipSuccess) e = forward(m, n);
+  if (e == hipSuccess) e = m->mfma ? infer_mfma(m, n, m->act[0], m->act[NCONV], m->out) : forward(m, n);
   if (e == hipSuccess) e = hipMemcpyAsync(out, m->out, (size_t)n * NOUT * 4, hipMemcpyDeviceToHost, m->st);
   if (e == hipSuccess) e = hipStreamSynchronize(m->st);
   return e == hipSuccess ? 0 : 2;
@@ -762,7 +819,7 @@ int jms_nn_train_epoch(jms_nn* m, jms_nn_data* d, int batch, float lr, const flo
     ++m->step;
     const float bc1 = 1.f - std::pow(0.9f, (float)m->step), bc2 = 1.f - std::pow(0.999f, (float)m->step);
     hipLaunchKernelGGL(k_adam, dim3(nblk(NPARAM, 256)), dim3(256), 0, m->st, m->p, m->g, m->m, m->v, m->pbf,
-                       NPARAM, lr, bc1, bc2);
+                       m->pack, NPARAM, lr, bc1, bc2);
     e = hipGetLastError();
   }
   std::vector<float> bl(std::max(1, nbatch), 0.f);
@@ -778,21 +835,31 @@ int jms_nn_train_epoch(jms_nn* m, jms_nn_data* d, int batch, float lr, const flo
 int jms_nn_predict(jms_nn* m, jms_nn_data* d, float* out) {
   if (!m || !d || !out) return 1;
   if (d->n < 1) return 0;
-  // batches of up to max_batch windows read in place; every output goes to
-  // one device array, copied back once
-  float* dout = nullptr;
-  hipError_t e = dalloc(&dout, (size_t)d->n * NOUT);
-  for (int b0 = 0; b0 < d->n && e == hipSuccess; b0 += m->maxb) {
-    const int nb = std::min(m->maxb, d->n - b0);
-    e = forward(m, nb, d->x + (size_t)b0 * IN_SIZE, dout + (size_t)b0 * NOUT);
+  // windows read in place, every output in one device array, copied back
+  // once; the workspaces stay with the model.  Matrix cores: chunks of up to
+  // 16384 windows (16 MiB of features); FMA kernels: of up to max_batch.
+  constexpr int CHUNK = 16384;
+  auto grow = [](auto** p, int* cap, int want, int per) {
+    if (*cap >= want) return hipSuccess;
+    (void)hipFree(*p);
+    *p = nullptr;
+    *cap = 0;
+    const hipError_t e = dalloc(p, (size_t)want * per);
+    if (e == hipSuccess) *cap = want;
+    return e;
+  };
+  const int chunk = m->mfma ? CHUNK : m->maxb;
+  hipError_t e = grow(&m->pout, &m->pout_cap, d->n, NOUT);
+  if (e == hipSuccess && m->mfma) e = grow(&m->feat, &m->feat_cap, std::min(d->n, CHUNK), FLAT);
+  for (int b0 = 0; b0 < d->n && e == hipSuccess; b0 += chunk) {
+    const int nb = std::min(chunk, d->n - b0);
+    const uint16_t* x = d->x + (size_t)b0 * IN_SIZE;
+    float* y = m->pout + (size_t)b0 * NOUT;
+    e = m->mfma ? infer_mfma(m, nb, x, m->feat, y) : forward(m, nb, x, y);
   }
-  if (e == hipSuccess) e = hipMemcpyAsync(out, dout, (size_t)d->n * NOUT * 4, hipMemcpyDeviceToHost, m->st);
-  if (e == hipSuccess) e = hipStreamSynchronize(m->st);
-  if (dout) {
-    (void)hipStreamSynchronize(m->st);
-    (void)hipFree(dout);
-  }
-  return e == hipSuccess ? 0 : 2;
+  if (e == hipSuccess) e = hipMemcpyAsync(out, m->pout, (size_t)d->n * NOUT * 4, hipMemcpyDeviceToHost, m->st);
+  const hipError_t es = hipStreamSynchronize(m->st);
+  return e == hipSuccess && es == hipSuccess ? 0 : 2;
 }
 
 }  // extern "C"
