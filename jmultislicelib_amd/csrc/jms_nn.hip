@@ -10,6 +10,7 @@
 #include <cstdint>
 #include <cstring>
 #include <random>
+#include <type_traits>
 #include <vector>
 #include "jms_nn.h"
 
@@ -282,6 +283,7 @@ __device__ __forceinline__ void store_packed(int i, uint16_t h, uint16_t* __rest
     if (e >= 0 && e < conv_w(l)) {
       const int co = e / (ci_n * 9), ci = e / 9 % ci_n, tap = e % 9;
       pack[nnmfma::conv_pack(l, ci_n, co, ci, tap)] = h;
+      if (l > 0) pack[nnmfma::conv_pack_b(l, co, ci, tap)] = h;
       return;
     }
   }
@@ -289,12 +291,9 @@ __device__ __forceinline__ void store_packed(int i, uint16_t h, uint16_t* __rest
   if (e >= 0 && e < HID * FLAT) pack[nnmfma::PACK_D1 + ((e % FLAT / 8) * HID + e / FLAT) * 8 + e % 8] = h;
 }
 
-__global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
-                       float* __restrict__ v, uint16_t* __restrict__ pbf, uint16_t* __restrict__ pack, int np,
-                       float lr, float bc1, float bc2) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= np) return;
-  const float gi = g[i];
+__device__ __forceinline__ void adam_step(int i, float gi, float* __restrict__ p, float* __restrict__ m,
+                                          float* __restrict__ v, uint16_t* __restrict__ pbf,
+                                          uint16_t* __restrict__ pack, float lr, float bc1, float bc2) {
   const float mi = 0.9f * m[i] + 0.1f * gi;
   const float vi = 0.999f * v[i] + 0.001f * gi * gi;
   m[i] = mi;
@@ -304,6 +303,99 @@ __global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float
   const uint16_t h = f2bf(q);
   pbf[i] = h;
   store_packed(i, h, pack);
+}
+__global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
+                       float* __restrict__ v, uint16_t* __restrict__ pbf, uint16_t* __restrict__ pack, int np,
+                       float lr, float bc1, float bc2) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < np) adam_step(i, g[i], p, m, v, pbf, pack, lr, bc1, bc2);
+}
+
+// Gradients of a matrix-core training step and (ADAM) the update: 64 sums per
+// block, eight threads each, which share the shares of a sum.  Sums j:
+// [0, PART) the convolutions' positions of the nb blocks' parts; then the
+// dense layers, over the n samples, from the features and gh, hid and dy of
+// the head; the last stands for the loss (loss_sum: the sum of squares,
+// loss_mean: over the n x 3 outputs; either may be null).
+static_assert(nnmfma::PART % 64 == 0 && FLAT % 64 == 0, "a block's sums are of one kind, one hidden unit");
+constexpr int UPD_SUMS = nnmfma::PART + NPARAM - OFF_D1W + 1;
+template <bool ADAM>
+__global__ __launch_bounds__(512) void k_update(const float* __restrict__ part, int nb,
+                                                const uint16_t* __restrict__ feat, const float* __restrict__ gh,
+                                                const float* __restrict__ hid, const float* __restrict__ dy, int n,
+                                                float* __restrict__ g, float* __restrict__ p, float* __restrict__ m,
+                                                float* __restrict__ v, uint16_t* __restrict__ pbf,
+                                                uint16_t* __restrict__ pack, float lr, float bc1, float bc2,
+                                                float* __restrict__ loss_sum, float* __restrict__ loss_mean) {
+  __shared__ float red[32][64];
+  const int c = threadIdx.x & 63, q = threadIdx.x >> 6, j = blockIdx.x * 64 + c;
+  // at most 32 shares of 8 parts; for the head 16 shares of 16 samples
+  const int cs = max(1, min(nb / 8, 32)), ds = max(1, min(n / 16, 16));
+  const bool conv = j < nnmfma::PART;
+  static_assert(off_cw(3) == off_cw(1) + 2 * (conv_w(1) + CH), "convolutions 2..4 are alike");
+  auto cw = [](int l) { return l == 0 ? 0 : off_cw(1) + (l - 1) * (conv_w(1) + CH); };
+  int i = OFF_D1W + j - nnmfma::PART;  // parameter of the sum
+  if (conv) {
+    for (int y = q; y < cs; y += 8) {
+      const int k1 = nnmfma::share_begin(nb, y + 1, cs);
+      float s = 0.f;
+#pragma unroll 8
+      for (int k = nnmfma::share_begin(nb, y, cs); k < k1; ++k) s += part[(long long)k * nnmfma::PART + j];
+      red[y][c] = s;
+    }
+    if (j < nnmfma::PART_B) {
+      const nnmfma::PartIdx e = nnmfma::part_index(j);
+      i = e.tap < 9 ? cw(e.l) + (e.co * (e.l == 0 ? C0 : CH) + e.ci) * 9 + e.tap : -1;
+    } else {
+      const int l = (j - nnmfma::PART_B) / CH;
+      i = cw(l) + (l == 0 ? conv_w(0) : conv_w(1)) + (j - nnmfma::PART_B) % CH;
+    }
+  } else if (i < OFF_D1B) {  // 64 inputs of one hidden unit
+    const int o = __builtin_amdgcn_readfirstlane((i - OFF_D1W) / FLAT);
+    const uint16_t* f = feat + (i - OFF_D1W) % FLAT;
+    for (int y = q; y < ds; y += 8) {
+      const int k1 = nnmfma::share_begin(n, y + 1, ds);
+      float s = 0.f;
+#pragma unroll 8
+      for (int k = nnmfma::share_begin(n, y, ds); k < k1; ++k)
+        s = fmaf(gh[(long long)k * HID + o], bf2f(f[(long long)k * FLAT]), s);
+      red[y][c] = s;
+    }
+  } else if (i <= NPARAM) {
+    // output gradient o and hidden unit u of the parameter's products
+    const float *a = dy + 3, *b = nullptr;
+    int lda = 4;
+    if (i < OFF_D2W) {
+      a = gh + (i - OFF_D1B);
+      lda = HID;
+    } else if (i < OFF_D2B) {
+      a = dy + (i - OFF_D2W) / HID;
+      b = hid + (i - OFF_D2W) % HID;
+    } else if (i < NPARAM) {
+      a = dy + (i - OFF_D2B);
+    }
+    for (int y = q; y < ds; y += 8) {
+      const int k1 = nnmfma::share_begin(n, y + 1, ds);
+      float s = 0.f;
+#pragma unroll 4
+      for (int k = nnmfma::share_begin(n, y, ds); k < k1; ++k) {
+        const float av = a[(long long)k * lda];
+        s = b ? fmaf(av, b[(long long)k * HID], s) : s + av;
+      }
+      red[y][c] = s;
+    }
+  }
+  __syncthreads();
+  if (q != 0 || i < 0 || i > NPARAM) return;
+  float s = 0.f;
+  for (int y = 0; y < (conv ? cs : ds); ++y) s += red[y][c];
+  if (i == NPARAM) {
+    if (loss_sum) *loss_sum = s;
+    if (loss_mean) *loss_mean = s / (float)(n * NOUT);
+    return;
+  }
+  g[i] = s;
+  if constexpr (ADAM) adam_step(i, s, p, m, v, pbf, pack, lr, bc1, bc2);
 }
 
 __global__ void k_zero(float* __restrict__ p, int np) {
@@ -398,7 +490,9 @@ struct jms_nn {
   int perm_cap = 0;
   float* eloss = nullptr;    // per-batch losses of an epoch (device), capacity eloss_cap
   int eloss_cap = 0;
-  float* part = nullptr;     // per-sample weight-gradient partials of the matrix-core path
+  float* part = nullptr;     // convolution gradient sums per block of the matrix-core path
+  float* hid = nullptr;      // hidden units [maxb][64] and output gradients [maxb][4] of its head
+  float* dy = nullptr;
   bool mfma = true;          // convolutions on the matrix cores (else the FMA kernels)
   long long step = 0;
 };
@@ -428,58 +522,16 @@ void release(jms_nn* m) {
   for (auto* a : m->gbuf) (void)hipFree(a);
   (void)hipFree(m->out); (void)hipFree(m->tb); (void)hipFree(m->scale); (void)hipFree(m->loss_part);
   (void)hipFree(m->idx); (void)hipFree(m->perm); (void)hipFree(m->eloss); (void)hipFree(m->part);
+  (void)hipFree(m->hid); (void)hipFree(m->dy);
   if (m->st) (void)hipStreamDestroy(m->st);
   delete m;
 }
 
-// matrix-core convolution of layer l (one block per sample)
-void conv_fwd_mfma(jms_nn* m, int l, int n, const uint16_t* in0) {
-  const dim3 g(n), b(256);
-  const uint16_t* x = (l == 0 && in0) ? in0 : m->act[l];
-  const uint16_t* w = m->pbf + off_cw(l);
-  const float* bias = m->p + off_cb(l);
-  uint16_t* y = m->act[l + 1];
-  switch (l) {
-    case 0: hipLaunchKernelGGL((nnmfma::k_conv_fwd<1, C0, H0>), g, b, 0, m->st, x, w, bias, y); break;
-    case 1: hipLaunchKernelGGL((nnmfma::k_conv_fwd<2, CH, H0>), g, b, 0, m->st, x, w, bias, y); break;
-    case 2: hipLaunchKernelGGL((nnmfma::k_conv_fwd<2, CH, H0 / 2>), g, b, 0, m->st, x, w, bias, y); break;
-    default: hipLaunchKernelGGL((nnmfma::k_conv_fwd<2, CH, H0 / 4>), g, b, 0, m->st, x, w, bias, y); break;
-  }
-}
-
-// matrix-core gradients of layer l: weights (per-sample partials reduced in
-// a fixed order), bias, and for l > 0 the gradient w.r.t. its input
-void conv_bwd_mfma(jms_nn* m, int l, int n) {
-  const dim3 g(n), b(256);
-  const float* dy = m->gbuf[l];
-  const uint16_t* x = m->act[l];
-  switch (l) {
-    case 0: hipLaunchKernelGGL((nnmfma::k_conv_bwd_w<1, C0, H0>), g, b, 0, m->st, dy, x, m->part); break;
-    case 1: hipLaunchKernelGGL((nnmfma::k_conv_bwd_w<2, CH, H0>), g, b, 0, m->st, dy, x, m->part); break;
-    case 2: hipLaunchKernelGGL((nnmfma::k_conv_bwd_w<2, CH, H0 / 2>), g, b, 0, m->st, dy, x, m->part); break;
-    default: hipLaunchKernelGGL((nnmfma::k_conv_bwd_w<2, CH, H0 / 4>), g, b, 0, m->st, dy, x, m->part); break;
-  }
-  const int cnt = conv_w(l);
-  const unsigned shares = (unsigned)std::max(1, std::min(n / 8, 32));
-  hipLaunchKernelGGL(nnmfma::k_reduce_parts, dim3(nblk(cnt, 256), shares), dim3(256), 0, m->st, m->part, n, cnt,
-                     m->g + off_cw(l));
-  hipLaunchKernelGGL(nnmfma::k_bias_grad, dim3(CH, shares), dim3(256), 0, m->st, dy, n, HOUT[l] * HOUT[l],
-                     m->g + off_cb(l));
-  if (l == 0) return;
-  const uint16_t* w = m->pbf + off_cw(l);
-  float* dx = m->gbuf[l - 1];
-  switch (l) {
-    case 1: hipLaunchKernelGGL((nnmfma::k_conv_bwd_data<2, H0>), g, b, 0, m->st, dy, w, x, dx); break;
-    case 2: hipLaunchKernelGGL((nnmfma::k_conv_bwd_data<2, H0 / 2>), g, b, 0, m->st, dy, w, x, dx); break;
-    default: hipLaunchKernelGGL((nnmfma::k_conv_bwd_data<2, H0 / 4>), g, b, 0, m->st, dy, w, x, dx); break;
-  }
-}
-
-// the dense head of n samples: hidden units (kept when hid is given), outputs
-void head_mfma(jms_nn* m, int n, const uint16_t* feat, uint16_t* hid, float* out) {
+// outputs of the dense head of n samples
+void head_mfma(jms_nn* m, int n, const uint16_t* feat, float* out) {
   auto go = [&](auto kern, int ns) {
     hipLaunchKernelGGL(kern, dim3(nblk(n, 16 * ns)), dim3(1024), 0, m->st, feat, m->pack + nnmfma::PACK_D1,
-                       m->p + OFF_D1B, m->pbf + OFF_D2W, m->p + OFF_D2B, n, hid, out);
+                       m->p + OFF_D1B, m->pbf + OFF_D2W, m->p + OFF_D2B, n, out);
   };
   // four samples share a weight read; one where four would leave CUs without
   // a block
@@ -491,20 +543,41 @@ void head_mfma(jms_nn* m, int n, const uint16_t* feat, uint16_t* hid, float* out
 // feat: n x 512 features
 hipError_t infer_mfma(jms_nn* m, int n, const uint16_t* x, uint16_t* feat, float* out) {
   hipLaunchKernelGGL((nnmfma::k_net_fwd<false>), dim3(std::min(n, m->cus)), dim3(nnmfma::NET_THREADS), 0, m->st, x,
-                     m->pack, m->p + off_cb(0), m->p + off_cb(1), m->p + off_cb(2), m->p + off_cb(3), n, feat,
-                     (uint16_t*)nullptr, (uint16_t*)nullptr, (uint16_t*)nullptr);
-  head_mfma(m, n, feat, nullptr, out);
+                     (const int*)nullptr, m->pack, m->p + off_cb(0), m->p + off_cb(1), m->p + off_cb(2),
+                     m->p + off_cb(3), n, feat, (uint16_t*)nullptr, (uint16_t*)nullptr, (uint16_t*)nullptr);
+  head_mfma(m, n, feat, out);
   return hipGetLastError();
 }
 
-// forward pass of n samples with the activations kept: input act[0] (or in0:
-// n windows in place), output [n][3] into out (default m->out)
+// forward, loss and gradients of n samples on the matrix cores: sample s is
+// window idx[s] of x (idx null: window s) with targets t alike.  ADAM (bc1 >
+// 0): the update too; else the gradients into m->g.  The sum of squared
+// residuals goes to m->loss_part[0], the batch's mean loss to loss_mean.
+hipError_t step_mfma(jms_nn* m, int n, const uint16_t* x, const float* t, const int* idx, float lr, float bc1,
+                     float bc2, float* loss_mean) {
+  const int blocks = std::min(n, m->cus);
+  uint16_t *y1 = m->act[1], *y2 = m->act[2], *y3 = m->act[3], *feat = m->act[NCONV];
+  float *gh = m->gbuf[NCONV], *df = m->gbuf[NCONV - 1];
+  const dim3 nt(nnmfma::NET_THREADS);
+  hipLaunchKernelGGL((nnmfma::k_net_fwd<true>), dim3(blocks), nt, 0, m->st, x, idx, m->pack, m->p + off_cb(0),
+                     m->p + off_cb(1), m->p + off_cb(2), m->p + off_cb(3), n, feat, y1, y2, y3);
+  hipLaunchKernelGGL(nnmfma::k_head_train, dim3(nblk(n, 4)), dim3(256), 0, m->st, feat, m->pack + nnmfma::PACK_D1,
+                     m->p + OFF_D1B, m->pbf + OFF_D2W, m->p + OFF_D2B, t, idx, m->scale, n, gh, df, m->hid, m->dy);
+  hipLaunchKernelGGL(nnmfma::k_net_bwd, dim3(blocks), nt, 0, m->st, x, idx, m->pack, y1, y2, y3, df, n, m->part);
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(nblk(UPD_SUMS, 64)), dim3(512), 0, m->st, m->part, blocks, feat, gh, m->hid,
+                       m->dy, n, m->g, m->p, m->m, m->v, m->pbf, m->pack, lr, bc1, bc2, m->loss_part, loss_mean);
+  };
+  if (bc1 > 0.f) go(k_update<true>);
+  else go(k_update<false>);
+  return hipGetLastError();
+}
+
+// The FMA kernels (jms_nn_set_kernels(m, 0)).  Forward pass of n samples with
+// the activations kept: input act[0] (or in0: n windows in place), output
+// [n][3] into out (default m->out)
 hipError_t forward(jms_nn* m, int n, const uint16_t* in0 = nullptr, float* out = nullptr) {
   for (int l = 0; l < NCONV; ++l) {
-    if (m->mfma) {
-      conv_fwd_mfma(m, l, n, in0);
-      continue;
-    }
     const long long px = (long long)n * HOUT[l] * HOUT[l];
     const int gsz = group_size(px, CH);
     const dim3 g(nblk(px, 256), CH / gsz);
@@ -551,10 +624,6 @@ hipError_t backward(jms_nn* m, int n, float* loss_acc = nullptr) {
                      m->pbf + OFF_D1W, m->act[NCONV], n, FLAT, HID, m->gbuf[NCONV - 1]);
   // convolutions, last to first; gbuf[l] = gradient w.r.t. the output of conv l+1;
   // their weight gradients are accumulated atomically over shares of the batch
-  if (m->mfma) {
-    for (int l = NCONV - 1; l >= 0; --l) conv_bwd_mfma(m, l, n);
-    return hipGetLastError();
-  }
   for (int l = NCONV - 1; l >= 0; --l) {
     const float* dy = m->gbuf[l];
     const int nblk_w = CIN[l] * (CH / GMAX);
@@ -586,7 +655,7 @@ hipError_t backward(jms_nn* m, int n, float* loss_acc = nullptr) {
 }
 
 float sum_loss(jms_nn* m, int n) {
-  const unsigned nb = nblk((long long)n * NOUT, 256);
+  const unsigned nb = m->mfma ? 1u : nblk((long long)n * NOUT, 256);
   std::vector<float> h(nb);
   if (hipMemcpyAsync(h.data(), m->loss_part, nb * sizeof(float), hipMemcpyDeviceToHost, m->st) != hipSuccess) return NAN;
   if (hipStreamSynchronize(m->st) != hipSuccess) return NAN;
@@ -626,7 +695,9 @@ int jms_nn_create(jms_nn** out, int max_batch, unsigned int seed) {
   if (e == hipSuccess) e = dalloc(&m->scale, NOUT);
   if (e == hipSuccess) e = dalloc(&m->loss_part, nblk((long long)max_batch * NOUT, 256));
   if (e == hipSuccess) e = dalloc(&m->idx, max_batch);
-  if (e == hipSuccess) e = dalloc(&m->part, (size_t)max_batch * conv_w(1));  // the largest layer
+  if (e == hipSuccess) e = dalloc(&m->part, (size_t)std::min(max_batch, m->cus) * nnmfma::PART);
+  if (e == hipSuccess) e = dalloc(&m->hid, (size_t)max_batch * HID);
+  if (e == hipSuccess) e = dalloc(&m->dy, (size_t)max_batch * 4);
   if (e != hipSuccess) {
     release(m);
     return 2;
@@ -689,8 +760,9 @@ int jms_nn_gradients(jms_nn* m, const uint16_t* x, const float* t, const float* 
   hipError_t e = hipMemcpyAsync(m->act[0], x, (size_t)n * IN_SIZE * 2, hipMemcpyHostToDevice, m->st);
   if (e == hipSuccess) e = hipMemcpyAsync(m->tb, t, (size_t)n * NOUT * 4, hipMemcpyHostToDevice, m->st);
   if (e == hipSuccess) e = hipMemcpyAsync(m->scale, scale, NOUT * 4, hipMemcpyHostToDevice, m->st);
-  if (e == hipSuccess) e = forward(m, n);
-  if (e == hipSuccess) e = backward(m, n);
+  if (e == hipSuccess && m->mfma) e = step_mfma(m, n, m->act[0], m->tb, nullptr, 0.f, 0.f, 0.f, nullptr);
+  if (e == hipSuccess && !m->mfma) e = forward(m, n);
+  if (e == hipSuccess && !m->mfma) e = backward(m, n);
   if (e == hipSuccess) e = hipMemcpyAsync(grads, m->g, NPARAM * 4, hipMemcpyDeviceToHost, m->st);
   if (e != hipSuccess) return 2;
   const float l = sum_loss(m, n);
@@ -811,13 +883,18 @@ int jms_nn_train_epoch(jms_nn* m, jms_nn_data* d, int batch, float lr, const flo
     e = hipGetLastError();
   }
   for (int b = 0; b < nbatch && e == hipSuccess; ++b) {
-    hipLaunchKernelGGL(k_gather, dim3(nblk((long long)batch * IN_SIZE, 256)), dim3(256), 0, m->st, d->x, d->t,
-                       m->perm + (size_t)b * batch, batch, m->act[0], m->tb);
+    const int* idx = m->perm + (size_t)b * batch;
+    ++m->step;
+    const float bc1 = 1.f - std::pow(0.9f, (float)m->step), bc2 = 1.f - std::pow(0.999f, (float)m->step);
+    if (m->mfma) {
+      e = step_mfma(m, batch, d->x, d->t, idx, lr, bc1, bc2, m->eloss + b);
+      continue;
+    }
+    hipLaunchKernelGGL(k_gather, dim3(nblk((long long)batch * IN_SIZE, 256)), dim3(256), 0, m->st, d->x, d->t, idx,
+                       batch, m->act[0], m->tb);
     e = forward(m, batch);
     if (e == hipSuccess) e = backward(m, batch, m->eloss + b);
     if (e != hipSuccess) break;
-    ++m->step;
-    const float bc1 = 1.f - std::pow(0.9f, (float)m->step), bc2 = 1.f - std::pow(0.999f, (float)m->step);
     hipLaunchKernelGGL(k_adam, dim3(nblk(NPARAM, 256)), dim3(256), 0, m->st, m->p, m->g, m->m, m->v, m->pbf,
                        m->pack, NPARAM, lr, bc1, bc2);
     e = hipGetLastError();
