@@ -89,6 +89,7 @@ struct CfgP {
   // other's memory phase (N = 512: 1.35 -> 1.11 ms per 1024 waves on MI355X).
   static constexpr int WPE_COL = Tuned<N>::WPE;
   static constexpr int WPE_ROW = 1;
+  static constexpr bool PF = false;  // see Lat
 
   // nontemporal wave loads/stores in the row / column pass: the streamed
   // waves then leave the reused phase gratings and propagators in L2
@@ -131,6 +132,24 @@ struct CfgP {
 // the configuration the library is built with
 template <int N>
 struct Cfg : CfgP<N> {};
+
+// The shape for launches that leave most CUs without a block (a single wave,
+// a few small ones): what counts is the time of one block, so blocks are small
+// (one wavefront of rows; 8 columns), loads and stores ordinary (the next pass
+// reads the wave from cache), and the grating and propagator values are loaded
+// along with the wave.  The arithmetic is Cfg's.  One wave, a row and a column
+// pass on MI355X, this shape / Cfg's: 64^2 6.6 / 7.2 us, 128^2 7.3 / 8.7,
+// 256^2 9.2 / 11.2, 512^2 10.4 / 13.6, 720^2 16.6 / 17.9 (an empty kernel: 1.55).
+template <int N>
+struct Lat : CfgP<N> {
+  using B = CfgP<N>;
+  static constexpr int LPB = (64 / B::T) > 0 ? 64 / B::T : 1;
+  static constexpr int CW = (B::TW * 8) % 64 == 0 ? 8 : B::CW;
+  static constexpr int CC = CW;
+  static constexpr int WPE_COL = 1;
+  static constexpr bool NT_ROW = false, NT_COL = false;
+  static constexpr bool PF = true;
+};
 
 
 }  // namespace jms

@@ -146,7 +146,7 @@ struct jms_hip_engine {
   bool use_graph = false;
   std::map<std::array<int, 4>, hipGraphExec_t> graphs;
   std::array<const void*, 16> graph_bufs{};
-  std::array<int, 4> graph_band{};  // and to the band the launches were made for
+  std::array<int, 8> graph_band{};  // and to the band the launches were made for
   // this device's scratch of the allocation-free batch entry (resolved at create)
   float* scratch = nullptr;
   // staged batches keep their waves in 16-column panels (set with the grid)
@@ -179,11 +179,11 @@ struct jms_hip_engine {
     return {waves.p, partial.p, cur_ppar.p, cur_var.p, cur_res.p, s_weights.p, wav0.p, pgr.p,
             pro.p, pro_t.p, detw.p, detw_t.p, twx.p, twy.p, cppl.p, cppl_t.p};
   }
-  int ntiles_col() const { return jms::col_tiles(ny, nx); }
+  int ntiles_col(bool lat = false) const { return jms::col_tiles(ny, nx, lat); }
   // The columns and rows that the waves leave out: where the propagators of
   // all object slices vanish.  A detector weight that is not finite makes
   // 0 * weight count, so those keep every column.
-  jms::BandHost band() const {
+  jms::BandHost band(bool lat) const {
     Gap g{0, nx, 0, ny};
     if (nobjslc < 1) return jms::BandHost();
     for (char c : det_inf)
@@ -195,7 +195,7 @@ struct jms_hip_engine {
       g.y0 = std::max(g.y0, p.y0);
       g.y1 = std::min(g.y1, p.y1);
     }
-    return jms::band_of(nx, ny, g.x0, g.x1, g.y0, g.y1);
+    return jms::band_of(nx, ny, g.x0, g.x1, g.y0, g.y1, lat);
   }
   // the probe is zero there too, so the first passes leave the columns out as well
   static bool holds(const Gap& g, const jms::BandHost& b) { return g.x0 <= b.x0 && g.x1 >= b.x1; }
@@ -287,21 +287,26 @@ struct BatchChans {
 // (stride n); `ppar` (float4 per wave) and `var` (nobjslc ints per wave)
 // describe them; src/src_stride the INIT source.  Readout partial sums go to
 // `partial` ([wave][plane][detector][column tile]), combined into `res`
-// (npos results) when npass > 0; `ch` are the single-wave channels.  `bd`:
-// the columns left out from the first slice on, and with `src_in` (the source
-// is zero there) in the passes before it; `keep`: leave psi(k) of the exit
-// plane in the waves (batches only read the sums).
+// (npos results) when npass > 0; `ch` are the single-wave channels.  `lat`:
+// the small launch shapes (natural wave layout); `src_same`: the source is the
+// probe, else the single-wave path's wave; `keep`: leave psi(k) of the exit
+// plane in the waves (batches only read the sums).  The band's columns are
+// left out from the first slice on, and before it where the source is zero
+// there.
 int enqueue_batch(jms_hip_engine* e, void* waves, float* partial, int nwave, int islc0, const void* src,
                   long long src_stride, const void* ppar, const int* var, int npos, int npass,
                   const float* weights, float* res, int accumulate, const BatchChans& ch, bool timed,
-                  const jms::BandHost& bd, bool src_in, bool keep, bool panel = false) {
+                  bool lat, bool src_same, bool keep, bool panel) {
+  const jms::BandHost bd = e->band(lat);
+  const bool src_in = e->holds(src_same ? e->wav0_gap : e->wav_gap, bd);
   // panel waves (staged batches): integrated readouts only, the waves are internal
   if (panel && (ch.real_space() || ch.dif || ch.wff || ch.dif_avg || ch.wff_avg))
     return e->fail(135, "panel waves carry no readout channels");
   const int S = e->nobjslc;
-  const int ntc = e->ntiles_col();
+  const int ntc = e->ntiles_col(lat);
   const long long part_w = (long long)e->ndetslc * e->ndet * ntc;
   jms::ColArgsHost ca;
+  ca.lat = lat;
   ca.wave = waves;
   ca.nx = e->nx;
   ca.wave_stride = e->n;
@@ -366,7 +371,7 @@ int enqueue_batch(jms_hip_engine* e, void* waves, float* partial, int nwave, int
       err = jms::launch_row_pass(e->nx, e->ny, nwave, (float2*)waves, e->n,
                                  e->pgr.as<float2>(), e->slcoffset[js], (long long)e->npgx * e->npgy,
                                  var, S, j, e->twx.as<float2>(), rc, mode, panel,
-                                 j > islc0 || src_in ? bd : jms::BandHost(), e->st);
+                                 j > islc0 || src_in ? bd : jms::BandHost(), lat, e->st);
       if (err != hipSuccess) return e->fail(131, "row pass", err);
     }
     ca.pro = e->pro.as<float2>() + (long long)e->proidx[js] * e->n;
@@ -415,7 +420,7 @@ int enqueue_exit_real_readout(jms_hip_engine* e, int nwave, const BatchChans& ch
   hipError_t err = jms::launch_col_fft(e->nx, e->ny, nwave, e->waves.as<float2>(), +1, e->twy.as<float2>(), e->st);
   if (err == hipSuccess)
     err = jms::launch_row_pass(e->nx, e->ny, nwave, e->waves.as<float2>(), e->n, e->pgr.as<float2>(), 0, 0,
-                               nullptr, 0, 0, e->twx.as<float2>(), rc, 2, false, jms::BandHost(), e->st);
+                               nullptr, 0, 0, e->twx.as<float2>(), rc, 2, false, jms::BandHost(), false, e->st);
   if (err != hipSuccess) return e->fail(134, "exit-plane real-space readout", err);
   return 0;
 }
@@ -433,7 +438,7 @@ int ensure_batch(jms_hip_engine* e, int nwave) {
   hipError_t err = e->waves.ensure(sizeof(float) * 2 * (size_t)e->n * nwave);
   if (err != hipSuccess) return e->fail(110, "allocate wave batch", err);
   const size_t np = sizeof(float) * (size_t)nwave * std::max(1, e->ndetslc) *
-                    std::max(1, e->ndet) * (size_t)e->ntiles_col();
+                    std::max(1, e->ndet) * (size_t)std::max(e->ntiles_col(), e->ntiles_col(true));
   err = e->partial.ensure(np);
   if (err != hipSuccess) return e->fail(111, "allocate readout partials", err);
   return 0;
@@ -992,14 +997,13 @@ int jms_hip_run_staged(jms_hip_engine* e, int pos0, int npos, int islc0) {
   if (rc) return rc;
   const int S = e->nobjslc;
   const int per = e->ndetslc * std::max(1, e->ndet);
-  const jms::BandHost bd = e->band();
-  const bool src_in = e->probe_in(bd);
   for (int p = pos0; p < pos0 + npos; p += bpos) {
     const int np = std::min(bpos, pos0 + npos - p);
     const int nw = np * npass;
     const float4* ppar = e->s_ppar.as<float4>() + (long long)p * npass;
     const int* var = e->s_var.as<int>() + (long long)p * npass * S;
     float* res = e->s_res.as<float>() + (long long)p * per;
+    const bool lat = jms::lat_ok(e->nx, e->ny, nw), panel = e->panel && !lat;
     if (e->use_graph) {
       // the graph reads fixed "current batch" buffers, refreshed before replay
       hipError_t err = e->cur_ppar.ensure(sizeof(float4) * (size_t)bw);
@@ -1010,7 +1014,9 @@ int jms_hip_run_staged(jms_hip_engine* e, int pos0, int npos, int islc0) {
         err = hipMemcpyAsync(e->cur_var.p, var, sizeof(int) * (size_t)nw * S, hipMemcpyDeviceToDevice, e->st);
       if (err != hipSuccess) return e->fail(120, "stage batch", err);
       const auto bufs = e->batch_buffers();
-      const std::array<int, 4> gband{bd.x0, bd.x1, bd.rows, src_in};
+      // the band of the small and of the large launch shapes follow from one gap
+      const jms::BandHost b0 = e->band(false), b1 = e->band(true);
+      const std::array<int, 8> gband{b0.x0, b0.x1, b0.rows, e->probe_in(b0), b1.x0, b1.x1, b1.rows, e->probe_in(b1)};
       if (bufs != e->graph_bufs || gband != e->graph_band) {
         e->drop_graphs();
         e->graph_bufs = bufs;
@@ -1025,7 +1031,7 @@ int jms_hip_run_staged(jms_hip_engine* e, int pos0, int npos, int islc0) {
         rc = enqueue_batch(e, e->waves.p, e->partial.as<float>(), nw, islc0, e->wav0.p, 0, e->cur_ppar.p,
                            e->cur_var.as<int>(), np,
                            npass, e->s_weights.as<float>(), e->cur_res.as<float>(), 0, BatchChans(), false,
-                           bd, src_in, false, e->panel);
+                           lat, true, false, panel);
         hipError_t err2 = hipStreamEndCapture(e->st, &g);
         if (rc) { if (g) (void)hipGraphDestroy(g); return rc; }
         if (err2 != hipSuccess) return e->fail(122, "end capture", err2);
@@ -1045,7 +1051,7 @@ int jms_hip_run_staged(jms_hip_engine* e, int pos0, int npos, int islc0) {
     } else {
       rc = enqueue_batch(e, e->waves.p, e->partial.as<float>(), nw, islc0, e->wav0.p, 0, ppar, var, np, npass,
                          e->s_weights.as<float>(), res,
-                         0, BatchChans(), e->timing, bd, src_in, false, e->panel);
+                         0, BatchChans(), e->timing, lat, true, false, panel);
       if (rc) return rc;
     }
   }
@@ -1073,9 +1079,11 @@ int jms_hip_run_batch_noalloc(jms_hip_engine* e, int islc0, int nwave, void* wav
   if (!e->scratch) return e->fail(7, "no scratch address");
   islc0 = std::max(0, std::min(islc0, e->nobjslc));
   (void)hipSetDevice(e->device);
-  const jms::BandHost bd = e->band();
+  // the small launch shapes need up to twice the tiles: only where those fit too
+  const long long need_lat = (long long)nwave * std::max(1, e->ndetslc) * e->ndet * e->ntiles_col(true);
+  const bool lat = jms::lat_ok(e->nx, e->ny, nwave) && need_lat <= jms::kScratchFloats;
   return enqueue_batch(e, waves, e->scratch, nwave, islc0, e->wav0.p, 0, ppar, var, npos, npass, weights, res, 0,
-                       BatchChans(), false, bd, e->probe_in(bd), false, e->panel);
+                       BatchChans(), false, lat, true, false, e->panel && !lat);
 }
 
 // ---------------------------------------------------------------------------
@@ -1325,10 +1333,10 @@ int jms_hip_group_run(jms_hip_group* g) {
     g->host.swap(host);
   }
   // one band for all members: the columns and rows that every member leaves out
-  jms::BandHost bd = lead->band();
+  jms::BandHost bd = lead->band(false);
   for (auto* e : g->eng) {
     if (e->nobjslc < 1) continue;  // only its INIT pass, which covers its own columns
-    const jms::BandHost b = e->band();
+    const jms::BandHost b = e->band(false);
     bd.x0 = std::max(bd.x0, b.x0);
     bd.x1 = std::min(bd.x1, b.x1);
     bd.rows = bd.rows && b.rows;
@@ -1497,14 +1505,15 @@ int jms_hip_multislice(jms_hip_engine* e, int islc0, const int* var, float weigh
   if (fl & JMS_HIP_DETECT_IMAGE_AVG) ch.img_avg = e->img_avg.as<float>();
   if (fl & JMS_HIP_DETECT_WAVEF_AVG) ch.wff_avg = e->wff_avg.p;
   if (fl & JMS_HIP_DETECT_WAVER_AVG) ch.wfr_avg = e->wfr_avg.p;
-  const jms::BandHost bd = e->band();
-  const bool src_in = e->holds(e->wav_gap, bd);
-  if (islc0 < S) e->wav_gap = Gap();  // until the run is enqueued
+  const bool lat = jms::lat_ok(e->nx, e->ny, 1);
   rc = enqueue_batch(e, e->waves.p, e->partial.as<float>(), 1, islc0, e->wav.p, e->n, nullptr,
                      e->var1.as<int>(), 1, 1, e->w1.as<float>(),
-                     e->res1.as<float>(), 1, ch, e->timing, bd, src_in, true);
+                     e->res1.as<float>(), 1, ch, e->timing, lat, false, true, false);
+  if (islc0 < S) {  // the wave becomes psi(k) of the exit plane
+    const jms::BandHost bd = e->band(lat);
+    e->wav_gap = rc ? Gap() : Gap{bd.x0, bd.x1, 0, 0};
+  }
   if (rc) return rc;
-  if (islc0 < S) e->wav_gap = Gap{bd.x0, bd.x1, 0, 0};
   // the run leaves psi(k) of the exit plane in the batch slot; keep it as the wave
   err = hipMemcpyAsync(e->wav.p, e->waves.p, sizeof(float) * 2 * (size_t)e->n, hipMemcpyDeviceToDevice, e->st);
   if (err != hipSuccess) return e->fail(113, "multislice run", err);

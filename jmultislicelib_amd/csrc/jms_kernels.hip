@@ -16,7 +16,8 @@ template <int N>
 hipError_t launch_row_pass_n(int ny, int nwave, float2* wave, long long wave_stride,
                              const float2* pgr, long long slc_off, long long npg,
                              const int* var_tab, int var_ld, int jslc, const float2* twx,
-                             const RowChanHost& rc, int mode, bool panel, const BandHost& bd, hipStream_t st);
+                             const RowChanHost& rc, int mode, bool panel, const BandHost& bd, bool lat,
+                             hipStream_t st);
 template <int N>
 hipError_t launch_col_pass_n(int nwave, bool init, bool exit_, const ColArgsHost& h,
                              hipStream_t st);
@@ -358,20 +359,20 @@ int row_tiles(int nx, int ny) {
   }
 }
 
-int col_tiles(int ny, int nx) {
+int col_tiles(int ny, int nx, bool lat) {
   switch (ny) {
-#define JMS_CASE(N) case N: return (nx + Cfg<N>::CC - 1) / Cfg<N>::CC;
+#define JMS_CASE(N) case N: return lat ? (nx + Lat<N>::CC - 1) / Lat<N>::CC : (nx + Cfg<N>::CC - 1) / Cfg<N>::CC;
     JMS_SIZES(JMS_CASE)
 #undef JMS_CASE
     default: return 0;
   }
 }
 
-BandHost band_of(int nx, int ny, int gx0, int gx1, int gy0, int gy1) {
+BandHost band_of(int nx, int ny, int gx0, int gx1, int gy0, int gy1, bool lat) {
   BandHost b;
   int tile = 0;
   switch (ny) {
-#define JMS_CASE(N) case N: tile = Cfg<N>::CC; b.rows = band_col_n<N>(gy0, gy1); break;
+#define JMS_CASE(N) case N: tile = lat ? Lat<N>::CC : Cfg<N>::CC; b.rows = band_col_n<N>(gy0, gy1); break;
     JMS_SIZES(JMS_CASE)
 #undef JMS_CASE
     default: return b;
@@ -384,15 +385,22 @@ BandHost band_of(int nx, int ny, int gx0, int gx1, int gy0, int gy1) {
   return b;
 }
 
+bool lat_ok(int nx, int ny, int nwave) {
+  constexpr int kCUs = 256;  // MI355X
+  // the long-column kernel has one shape; its launches fill the device
+  const bool wl = ny != 1024 && ny != 2048;
+  return wl && nwave * col_tiles(ny, nx, false) < kCUs;
+}
+
 hipError_t launch_row_pass(int nx, int ny, int nwave, float2* wave, long long wave_stride,
                            const float2* pgr, long long slc_off, long long npg, const int* var_tab,
                            int var_ld, int jslc, const float2* twx, const RowChanHost& rc, int mode,
-                           bool panel, const BandHost& bd, hipStream_t st) {
+                           bool panel, const BandHost& bd, bool lat, hipStream_t st) {
   switch (nx) {
 #define JMS_CASE(N)                                                                         \
   case N:                                                                                   \
     return launch_row_pass_n<N>(ny, nwave, wave, wave_stride, pgr, slc_off, npg, var_tab, \
-                                var_ld, jslc, twx, rc, mode, panel, bd, st);
+                                var_ld, jslc, twx, rc, mode, panel, bd, lat, st);
     JMS_SIZES(JMS_CASE)
 #undef JMS_CASE
     default: return hipErrorInvalidValue;

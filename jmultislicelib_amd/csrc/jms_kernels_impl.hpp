@@ -243,6 +243,19 @@ __global__ __launch_bounds__(C_::T * C_::LPB) __attribute__((amdgpu_waves_per_eu
       }
     });
   }
+  // PF: the grating values are loaded along with the row, not when they are needed
+  float2 tg[C_::PF && MODE != 2 ? NREG : 1];
+  auto tptr = [&](int b, auto Q) { return at32(gblk + decltype(Q)::value * M1::NBF, line * N + b); };
+  if constexpr (C_::PF && MODE != 2) {
+    if (valid) {
+      static_for<0, M1::NB>([&](auto I) {
+        constexpr int i = decltype(I)::value;
+        const int b = t + i * T;
+        if (M1::FULL || b < M1::NBF)
+          static_for<0, M1::R0>([&](auto Q) { tg[i * M1::R0 + decltype(Q)::value] = *tptr(b, Q); });
+      });
+    }
+  }
   if constexpr (!C_::GTW_ROW) __syncthreads();  // twiddle table complete
   // rows lie inside one wavefront when T divides 64: wave-level barriers suffice
   using RowSync = std::conditional_t<(64 % T == 0), SyncWave, SyncBlock>;
@@ -277,7 +290,8 @@ __global__ __launch_bounds__(C_::T * C_::LPB) __attribute__((amdgpu_waves_per_eu
       if (M1::FULL || b < M1::NBF) {
         static_for<0, M1::R0>([&](auto Q) {
           constexpr int q = decltype(Q)::value;
-          v[i * M1::R0 + q] = cmul(v[i * M1::R0 + q], *at32(gblk + q * M1::NBF, line * N + b));
+          if constexpr (C_::PF) v[i * M1::R0 + q] = cmul(v[i * M1::R0 + q], tg[i * M1::R0 + q]);
+          else v[i * M1::R0 + q] = cmul(v[i * M1::R0 + q], *tptr(b, Q));
         });
       }
     });
@@ -449,9 +463,11 @@ struct ColTile {
 // BAND: the propagators vanish on the rows of the dead slots (BandSlots of
 // the transform's last radix): psi is zero there without the product, and the
 // butterflies on both sides of it are pruned.
-template <int N, bool INIT, bool EXIT, bool DET, class C_, bool FIN = false, bool FOUT = false, bool BAND = false>
+template <int N, bool INIT, bool EXIT, bool DET, class C_, bool FIN = false, bool FOUT = false, bool BAND = false,
+          int NPV = 1>
 __device__ __forceinline__ void col_body(const ColArgs& a, long long w, float2* s_buf, const float2* s_tw,
-                                         float* s_red, int c, int t, int x, int tile, bool valid) {
+                                         float* s_red, int c, int t, int x, int tile, bool valid,
+                                         const float2 (&pv)[NPV]) {
   static_assert(!INIT || !BAND, "the incident wave has no propagator");
   using P = typename C_::PC;
   constexpr int T = C_::TW;
@@ -524,6 +540,7 @@ __device__ __forceinline__ void col_body(const ColArgs& a, long long w, float2* 
         static_for<0, M1::R0>([&](auto Q) {
           constexpr int q = decltype(Q)::value;
           if constexpr (dead(q)) v[i * M1::R0 + q] = make_float2(0.f, 0.f);
+          else if constexpr (C_::PF) v[i * M1::R0 + q] = cmul(v[i * M1::R0 + q], pv[i * M1::R0 + q]);
           else v[i * M1::R0 + q] = cmul(v[i * M1::R0 + q], pcol[b + q * M1::NBF]);
         });
       }
@@ -712,6 +729,23 @@ __global__ __launch_bounds__(C_::TW * C_::CW) __attribute__((amdgpu_waves_per_eu
       return;
     }
   }
+  // PF: this thread's propagator values are loaded along with the tile
+  constexpr int NPV = C_::PF && !INIT ? NREG : 1;
+  float2 pv[NPV];
+  if constexpr (C_::PF && !INIT) {
+    using M1 = IOMap<N, T, P, true>;
+    using BSL = BandSlots<N, radix_at<P, true>(0)>;
+    const float2* pcol = a.pro_t + (long long)(c < ncol ? x0 + c : x0) * N;
+    static_for<0, M1::NB>([&](auto I) {
+      constexpr int i = decltype(I)::value;
+      const int b = t + i * T;
+      if (M1::FULL || b < M1::NBF)
+        static_for<0, M1::R0>([&](auto Q) {
+          constexpr int q = decltype(Q)::value;
+          if constexpr (!(BAND && BSL::dead(q))) pv[i * M1::R0 + q] = pcol[b + q * M1::NBF];
+        });
+    });
+  }
   {
     float2 st[TL::KST];
     TL::load(st, INIT ? (a.src + w * a.src_stride + x0) : wv_base, INIT ? nx : wrs, ncol, tid);
@@ -723,7 +757,8 @@ __global__ __launch_bounds__(C_::TW * C_::CW) __attribute__((amdgpu_waves_per_eu
     }
   }
   __syncthreads();
-  col_body<N, INIT, EXIT, DET, C_, FIN, FOUT, BAND && !INIT>(a, w, s_buf, s_tw, s_red, c, t, x0 + c, tile, c < ncol);
+  col_body<N, INIT, EXIT, DET, C_, FIN, FOUT, BAND && !INIT, NPV>(a, w, s_buf, s_tw, s_red, c, t, x0 + c, tile,
+                                                                 c < ncol, pv);
   if constexpr (EXIT) {
     if (!a.keep) return;
   }
@@ -1154,22 +1189,29 @@ template <int N>
 hipError_t launch_row_pass_n(int ny, int nwave, float2* wave, long long wave_stride,
                              const float2* pgr, long long slc_off, long long npg,
                              const int* var_tab, int var_ld, int jslc, const float2* twx,
-                             const RowChanHost& h, int mode, bool panel, const BandHost& bd, hipStream_t st) {
-  dim3 g((ny + Cfg<N>::LPB - 1) / Cfg<N>::LPB, nwave), b(Cfg<N>::T * Cfg<N>::LPB);
+                             const RowChanHost& h, int mode, bool panel, const BandHost& bd, bool lat,
+                             hipStream_t st) {
+  using CF = Cfg<N>;
+  using CL = Lat<N>;
   RowChan rc;
   rc.img = h.img; rc.img_avg = h.img_avg;
   rc.wfr = (float2*)h.wfr; rc.wfr_avg = (float2*)h.wfr_avg;
   rc.cwgt = h.cwgt; rc.chan_wstride = h.chan_wstride; rc.chan_off = h.chan_off;
-  if (panel && (mode != 0 || !Cfg<N>::PANEL)) return hipErrorInvalidValue;
+  if (panel && (mode != 0 || !CF::PANEL || lat)) return hipErrorInvalidValue;
+  const int lpb = lat && mode != 2 ? CL::LPB : CF::LPB;
+  const dim3 g((ny + lpb - 1) / lpb, nwave), b(CF::T * lpb);
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, g, b, 0, st, wave, ny, wave_stride, pgr, slc_off, npg, var_tab, var_ld, jslc, twx, rc,
                        GrpArgs{}, bd.x0, bd.x1);
   };
-  using CF = Cfg<N>;
   const bool band = bd.on();
   if (mode == 2) go(k_row_pass<N, 2>);
+  else if (mode == 1 && lat && band) go(k_row_pass<N, 1, CL, false, false, true>);
+  else if (mode == 1 && lat) go(k_row_pass<N, 1, CL>);
   else if (mode == 1 && band) go(k_row_pass<N, 1, CF, false, false, true>);
   else if (mode == 1) go(k_row_pass<N, 1>);
+  else if (lat && band) go(k_row_pass<N, 0, CL, false, false, true>);
+  else if (lat) go(k_row_pass<N, 0, CL>);
   else if (!panel && band) go(k_row_pass<N, 0, CF, false, false, true>);
   else if (!panel) go(k_row_pass<N, 0>);
   else if constexpr (CF::PANEL) {
@@ -1252,10 +1294,10 @@ hipError_t launch_col_pass_n(int nwave, bool init, bool exit_, const ColArgsHost
   a.cppl_t = h.cppl_t;
   using CF = Cfg<N>;
   static_assert(CF::XL || CF::WL, "every line length has a column kernel");
-  if (h.panel && !CF::PANEL) return hipErrorInvalidValue;
-  const int tiles = (h.nx + CF::CC - 1) / CF::CC;
-  a.tg0 = h.band.x0 / CF::CC;
-  a.tgn = h.band.on() ? (h.band.x1 - h.band.x0) / CF::CC : 0;
+  if (h.panel && (!CF::PANEL || h.lat)) return hipErrorInvalidValue;
+  const int cc = h.lat ? Lat<N>::CC : CF::CC, tiles = (h.nx + cc - 1) / cc;
+  a.tg0 = h.band.x0 / cc;
+  a.tgn = h.band.on() ? (h.band.x1 - h.band.x0) / cc : 0;
   a.keep = h.keep;
   a.tclr = exit_ && h.keep;
   dim3 g(a.tclr ? tiles : tiles - a.tgn, nwave);
@@ -1264,8 +1306,9 @@ hipError_t launch_col_pass_n(int nwave, bool init, bool exit_, const ColArgsHost
     if (!h.panel) launch_col_x<N, CF, false>(g, b, init, exit_, h.detect, a, st);
     else if constexpr (CF::PANEL) launch_col_x<N, CF, true>(g, b, init, exit_, h.detect, a, st);
   } else {
-    dim3 b(CF::TW * CF::CW);
-    if (!h.panel) launch_col_w<N, CF, false, false>(g, b, init, exit_, h.detect, h.band.rows, a, st);
+    dim3 b(CF::TW * cc);
+    if (h.lat) launch_col_w<N, Lat<N>, false, false>(g, b, init, exit_, h.detect, h.band.rows, a, st);
+    else if (!h.panel) launch_col_w<N, CF, false, false>(g, b, init, exit_, h.detect, h.band.rows, a, st);
     else if constexpr (CF::PANEL) launch_col_w<N, CF, false, true>(g, b, init, exit_, h.detect, h.band.rows, a, st);
   }
   return hipGetLastError();

@@ -127,3 +127,19 @@ def test_band_of_a_group():
         grp.close()
         for eng in engines:
             eng.close()
+
+
+@pytest.mark.parametrize("nx,ny", [(16, 32), (32, 16), (64, 64), (96, 128), (128, 96), (256, 256), (320, 360),
+                                   (384, 480), (512, 512), (625, 625), (640, 640), (720, 720), (768, 64), (64, 768)])
+def test_small_launches_equal_large_ones(nx, ny):
+    """A batch that leaves CUs without a block takes the small launch shapes
+    (natural layout, other column tiles), a larger one the shapes of the line
+    length (panels where it has them), with and without a band."""
+    sp = random_setup(nx, ny, nslices=4, nvar=(2, 2), ndetper=2, seed=nx + ny)
+    few, many = 3, 256 // max(1, nx // 16) + 3  # column tiles are at most 16 wide
+    var = np.resize(configs.variant_sequences(sp, few, seed=6), (many, 4))
+    x, y = np.array([0.0, 0.11, 0.3], np.float32), np.array([0.2, 0.0, 0.07], np.float32)
+    for s in (sp, _general(sp)):
+        small = _scan(s, var[:few], x, y)
+        large = _scan(s, var, np.resize(x, many), np.resize(y, many))
+        _close(large, small[np.resize(np.arange(few), many)], "large against small launches")
