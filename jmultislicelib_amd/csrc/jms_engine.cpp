@@ -113,6 +113,10 @@ struct jms_hip_engine {
   std::vector<int> proidx;
   DevBuf pro, pro_t;  // row-major and column-major ([x][y]) copies
   std::vector<Gap> pro_gap;  // zero gap of each propagator
+  // plane table of the one-launch slice loop (GrpPlane [nobjslc + 1]; sums of
+  // one tile), kept in step with the set-up calls
+  DevBuf loop_tab;
+  bool loop_ready = false;
   // object slices
   int nobjslc = 0;
   std::vector<int> objslc;
@@ -145,8 +149,8 @@ struct jms_hip_engine {
   // any of them moves, all graphs are dropped before the next capture.
   bool use_graph = false;
   std::map<std::array<int, 4>, hipGraphExec_t> graphs;
-  std::array<const void*, 16> graph_bufs{};
-  std::array<int, 8> graph_band{};  // and to the band the launches were made for
+  std::array<const void*, 17> graph_bufs{};
+  std::array<int, 12> graph_band{};  // and to the band the launches were made for
   // this device's scratch of the allocation-free batch entry (resolved at create)
   float* scratch = nullptr;
   // staged batches keep their waves in 16-column panels (set with the grid)
@@ -175,19 +179,19 @@ struct jms_hip_engine {
     graphs.clear();
   }
   // device addresses a captured batch depends on
-  std::array<const void*, 16> batch_buffers() const {
+  std::array<const void*, 17> batch_buffers() const {
     return {waves.p, partial.p, cur_ppar.p, cur_var.p, cur_res.p, s_weights.p, wav0.p, pgr.p,
-            pro.p, pro_t.p, detw.p, detw_t.p, twx.p, twy.p, cppl.p, cppl_t.p};
+            pro.p, pro_t.p, detw.p, detw_t.p, twx.p, twy.p, cppl.p, cppl_t.p, loop_tab.p};
   }
   int ntiles_col(bool lat = false) const { return jms::col_tiles(ny, nx, lat); }
   // The columns and rows that the waves leave out: where the propagators of
   // all object slices vanish.  A detector weight that is not finite makes
   // 0 * weight count, so those keep every column.
-  jms::BandHost band(bool lat) const {
+  Gap gap() const {
     Gap g{0, nx, 0, ny};
-    if (nobjslc < 1) return jms::BandHost();
+    if (nobjslc < 1) return Gap();
     for (char c : det_inf)
-      if (c) return jms::BandHost();
+      if (c) return Gap();
     for (int o : objslc) {
       const Gap& p = pro_gap[proidx[o % nscslc]];
       g.x0 = std::max(g.x0, p.x0);
@@ -195,6 +199,10 @@ struct jms_hip_engine {
       g.y0 = std::max(g.y0, p.y0);
       g.y1 = std::min(g.y1, p.y1);
     }
+    return g;
+  }
+  jms::BandHost band(bool lat) const {
+    const Gap g = gap();
     return jms::band_of(nx, ny, g.x0, g.x1, g.y0, g.y1, lat);
   }
   // the probe is zero there too, so the first passes leave the columns out as well
@@ -281,7 +289,39 @@ struct BatchChans {
   void* wfr_avg = nullptr;
   const float* cwgt = nullptr;
   bool real_space() const { return img || img_avg || wfr || wfr_avg; }
+  bool any() const { return real_space() || dif || dif_avg || wff || wff_avg; }
 };
+
+// The plane table of the one-launch slice loop, after a set-up call that it
+// depends on (the batch runs never allocate or copy it).
+void refresh_loop(jms_hip_engine* e) {
+  e->loop_ready = false;
+  const int S = e->nobjslc;
+  if (!jms::loop_ok(e->nx, e->ny, 256) || S < 1 || !e->pgr.p || !e->pro_t.p || e->npgx != e->nx || e->npgy != e->ny ||
+      e->nscslc < 1 || (int)e->proidx.size() < e->nscslc || (int)e->slcoffset.size() < e->nscslc ||
+      e->det_objslc.size() != (size_t)S + 1)
+    return;
+  std::vector<jms::GrpPlane> pl(S + 1);
+  for (int p = 0; p <= S; ++p) {
+    if (p < S) {
+      const int js = e->objslc[p] % e->nscslc;
+      pl[p].slc_off = e->slcoffset[js];
+      pl[p].pro_t = e->pro_t.as<float2>() + (long long)e->proidx[js] * e->n;
+    }
+    const int id = e->det_objslc[p];
+    pl[p].part_off = id >= 0 && (e->detflags & JMS_HIP_DETECT_INTEGRATED) ? (long long)id * e->ndet : -1;
+  }
+  (void)hipSetDevice(e->device);
+  (void)hipStreamSynchronize(e->st);  // launches already enqueued may still read the old table
+  const size_t nb = sizeof(jms::GrpPlane) * pl.size();
+  e->loop_ready = e->loop_tab.ensure(nb) == hipSuccess &&
+                  hipMemcpy(e->loop_tab.p, pl.data(), nb, hipMemcpyHostToDevice) == hipSuccess;
+}
+
+// whether a batch of nwave waves without channels runs as one launch
+bool use_loop(const jms_hip_engine* e, int nwave, int islc0) {
+  return e->loop_ready && islc0 < e->nobjslc && jms::loop_ok(e->nx, e->ny, nwave);
+}
 
 // Launch sequence of one batch.  `waves` holds the nwave working waves
 // (stride n); `ppar` (float4 per wave) and `var` (nobjslc ints per wave)
@@ -300,10 +340,11 @@ int enqueue_batch(jms_hip_engine* e, void* waves, float* partial, int nwave, int
   const jms::BandHost bd = e->band(lat);
   const bool src_in = e->holds(src_same ? e->wav0_gap : e->wav_gap, bd);
   // panel waves (staged batches): integrated readouts only, the waves are internal
-  if (panel && (ch.real_space() || ch.dif || ch.wff || ch.dif_avg || ch.wff_avg))
+  if (panel && ch.any())
     return e->fail(135, "panel waves carry no readout channels");
   const int S = e->nobjslc;
-  const int ntc = e->ntiles_col(lat);
+  const bool loop = use_loop(e, nwave, islc0) && !ch.any();
+  const int ntc = loop ? 1 : e->ntiles_col(lat);
   const long long part_w = (long long)e->ndetslc * e->ndet * ntc;
   jms::ColArgsHost ca;
   ca.lat = lat;
@@ -345,42 +386,76 @@ int enqueue_batch(jms_hip_engine* e, void* waves, float* partial, int nwave, int
     ca.part_off = id >= 0 ? (long long)id * e->ndet * ntc : 0;
     ca.chan_off = id >= 0 ? (long long)id * e->n : 0;
   };
-  // INIT column pass: plane islc0
-  {
-    ca.src = src;
-    ca.src_stride = src_stride;
-    ca.ppar = ppar;
-    ca.pro = nullptr;
-    plane_setup(islc0);
-    if (src_in && islc0 < S) ca.band = bd;
+  if (loop) {
+    jms::LoopArgs la;
+    la.wave = keep ? (float2*)waves : nullptr;
+    la.wave_stride = e->n;
+    la.src = (const float2*)src;
+    la.src_stride = src_stride;
+    la.ppar = (const float4*)ppar;
+    la.var = var;
+    la.var_ld = S;
+    la.pgr = e->pgr.as<float2>();
+    la.pl = e->loop_tab.as<jms::GrpPlane>();
+    la.islc0 = islc0;
+    la.nslc = S;
+    la.detw_t = ca.detw_t;
+    la.cppl_t = ca.cppl_t;
+    la.ndet = ca.ndet;
+    la.partial = partial;
+    la.part_wstride = part_w;
+    la.dsx = e->dsx;
+    la.dsy = e->dsy;
+    la.kscx = ca.kscx;
+    la.kscy = ca.kscy;
+    la.twx = e->twx.as<float2>();
+    la.twy = e->twy.as<float2>();
+    const Gap g = e->gap();
+    const jms::BandHost lb = jms::loop_band(e->nx, e->ny, g.x0, g.x1, g.y0, g.y1);
+    la.gx0 = lb.x0;
+    la.gx1 = lb.x1;
     TimedLaunch tl(e, 1, timed);
-    err = jms::launch_col_pass(e->ny, nwave, true, islc0 >= S, ca, e->st);
-    if (err != hipSuccess) return e->fail(130, "column pass (init)", err);
-  }
-  ca.src = nullptr;
-  ca.ppar = nullptr;
-  ca.band = bd;
-  for (int j = islc0; j < S; ++j) {
-    const int js = e->objslc[j] % e->nscslc;
+    err = jms::launch_loop(e->nx, e->ny, nwave, la, lb.on() && lb.rows && e->holds(src_same ? e->wav0_gap : e->wav_gap, lb),
+                           e->st);
+    if (err != hipSuccess) return e->fail(132, "slice loop", err);
+  } else {
+    // INIT column pass: plane islc0
     {
-      // real-space readout of plane j inside the row pass (ReadoutImgDet_d)
-      const int id = e->det_objslc[j];
-      const int mode = (id >= 0 && ch.real_space()) ? 1 : 0;
-      rc.chan_off = id >= 0 ? (long long)id * e->n : 0;
-      TimedLaunch tl(e, 0, timed);
-      err = jms::launch_row_pass(e->nx, e->ny, nwave, (float2*)waves, e->n,
-                                 e->pgr.as<float2>(), e->slcoffset[js], (long long)e->npgx * e->npgy,
-                                 var, S, j, e->twx.as<float2>(), rc, mode, panel,
-                                 j > islc0 || src_in ? bd : jms::BandHost(), lat, e->st);
-      if (err != hipSuccess) return e->fail(131, "row pass", err);
-    }
-    ca.pro = e->pro.as<float2>() + (long long)e->proidx[js] * e->n;
-    ca.pro_t = e->pro_t.as<float2>() + (long long)e->proidx[js] * e->n;
-    plane_setup(j + 1);
-    {
+      ca.src = src;
+      ca.src_stride = src_stride;
+      ca.ppar = ppar;
+      ca.pro = nullptr;
+      plane_setup(islc0);
+      if (src_in && islc0 < S) ca.band = bd;
       TimedLaunch tl(e, 1, timed);
-      err = jms::launch_col_pass(e->ny, nwave, false, j == S - 1, ca, e->st);
-      if (err != hipSuccess) return e->fail(132, "column pass", err);
+      err = jms::launch_col_pass(e->ny, nwave, true, islc0 >= S, ca, e->st);
+      if (err != hipSuccess) return e->fail(130, "column pass (init)", err);
+    }
+    ca.src = nullptr;
+    ca.ppar = nullptr;
+    ca.band = bd;
+    for (int j = islc0; j < S; ++j) {
+      const int js = e->objslc[j] % e->nscslc;
+      {
+        // real-space readout of plane j inside the row pass (ReadoutImgDet_d)
+        const int id = e->det_objslc[j];
+        const int mode = (id >= 0 && ch.real_space()) ? 1 : 0;
+        rc.chan_off = id >= 0 ? (long long)id * e->n : 0;
+        TimedLaunch tl(e, 0, timed);
+        err = jms::launch_row_pass(e->nx, e->ny, nwave, (float2*)waves, e->n,
+                                   e->pgr.as<float2>(), e->slcoffset[js], (long long)e->npgx * e->npgy,
+                                   var, S, j, e->twx.as<float2>(), rc, mode, panel,
+                                   j > islc0 || src_in ? bd : jms::BandHost(), lat, e->st);
+        if (err != hipSuccess) return e->fail(131, "row pass", err);
+      }
+      ca.pro = e->pro.as<float2>() + (long long)e->proidx[js] * e->n;
+      ca.pro_t = e->pro_t.as<float2>() + (long long)e->proidx[js] * e->n;
+      plane_setup(j + 1);
+      {
+        TimedLaunch tl(e, 1, timed);
+        err = jms::launch_col_pass(e->ny, nwave, false, j == S - 1, ca, e->st);
+        if (err != hipSuccess) return e->fail(132, "column pass", err);
+      }
     }
   }
   if (npass > 0 && res && ca.ndet > 0) {
@@ -485,7 +560,7 @@ void jms_hip_destroy(jms_hip_engine* e) {
   e->groups.clear();
   e->drop_graphs();
   for (auto ev : e->ev_pool) (void)hipEventDestroy(ev);
-  DevBuf* bufs[] = {&e->twx, &e->twy, &e->pgr, &e->pro, &e->pro_t, &e->detw, &e->detw_t, &e->wav0,
+  DevBuf* bufs[] = {&e->twx, &e->twy, &e->pgr, &e->pro, &e->pro_t, &e->loop_tab, &e->detw, &e->detw_t, &e->wav0,
                     &e->cppl, &e->cppl_t,
                     &e->s_ppar, &e->s_weights, &e->s_var, &e->s_res, &e->waves, &e->partial,
                     &e->cur_var, &e->cur_ppar, &e->cur_res, &e->wav, &e->var1, &e->res1,
@@ -512,6 +587,7 @@ int jms_hip_set_grid(jms_hip_engine* e, int nx, int ny, float a0x, float a0y, fl
   e->nx = nx; e->ny = ny; e->n = (long long)nx * ny;
   e->a0x = a0x; e->a0y = a0y; e->wl = wl;
   e->panel = jms::panel_ok(nx, ny);
+  e->loop_ready = false;
   e->pro_gap.assign(e->pro_gap.size(), Gap());
   e->wav0_gap = e->wav_gap = Gap();
   std::vector<float> tw;
@@ -547,6 +623,7 @@ int jms_hip_setup_gratings(jms_hip_engine* e, int npgx, int npgy, int nslc, cons
   if (err != hipSuccess) return e->fail(104, "allocate phase gratings", err);
   err = hipMemset(e->pgr.p, 0, sizeof(float) * 2 * (size_t)off);
   if (err != hipSuccess) return e->fail(105, "clear phase gratings", err);
+  refresh_loop(e);
   return 0;
 }
 
@@ -719,6 +796,7 @@ int jms_hip_setup_propagators(jms_hip_engine* e, int npro, int nslc, const int* 
   hipError_t err = e->pro.ensure(sizeof(float) * 2 * (size_t)npro * e->n);
   if (err == hipSuccess) err = e->pro_t.ensure(sizeof(float) * 2 * (size_t)npro * e->n);
   if (err != hipSuccess) return e->fail(102, "allocate propagators", err);
+  refresh_loop(e);
   return 0;
 }
 
@@ -747,6 +825,7 @@ int jms_hip_setup_objects(jms_hip_engine* e, int nobjslc, const int* objslc) {
   e->drop_graphs();
   e->nobjslc = nobjslc;
   e->objslc.assign(objslc, objslc + nobjslc);
+  refresh_loop(e);
   return 0;
 }
 
@@ -795,6 +874,7 @@ int jms_hip_setup_detection(jms_hip_engine* e, int ndetslc, const int* det_objsl
     if (err == hipSuccess) err = hipMemset(e->detw_t.p, 0, sizeof(float) * (size_t)ndet * e->n);
     if (err != hipSuccess) return e->fail(103, "allocate detector functions", err);
   }
+  refresh_loop(e);
   return 0;
 }
 
@@ -1016,7 +1096,9 @@ int jms_hip_run_staged(jms_hip_engine* e, int pos0, int npos, int islc0) {
       const auto bufs = e->batch_buffers();
       // the band of the small and of the large launch shapes follow from one gap
       const jms::BandHost b0 = e->band(false), b1 = e->band(true);
-      const std::array<int, 8> gband{b0.x0, b0.x1, b0.rows, e->probe_in(b0), b1.x0, b1.x1, b1.rows, e->probe_in(b1)};
+      const Gap g = e->gap();
+      const std::array<int, 12> gband{b0.x0, b0.x1, b0.rows, e->probe_in(b0), b1.x0, b1.x1, b1.rows, e->probe_in(b1),
+                                      g.x0, g.x1, e->wav0_gap.x0, e->wav0_gap.x1};
       if (bufs != e->graph_bufs || gband != e->graph_band) {
         e->drop_graphs();
         e->graph_bufs = bufs;

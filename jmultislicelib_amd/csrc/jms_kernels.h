@@ -19,8 +19,8 @@ struct BandHost {
 // rows [gy0, gy1) where every propagator of the run vanishes
 BandHost band_of(int nx, int ny, int gx0, int gx1, int gy0, int gy1, bool lat);
 // whether a batch of nwave waves takes the small launch shapes (Lat in
-// jms_cfg.hpp; natural wave layout): its column pass would have fewer blocks
-// than the device has CUs
+// jms_cfg.hpp; natural wave layout): its column pass would have fewer than 128
+// blocks
 bool lat_ok(int nx, int ny, int nwave);
 
 // Arguments of one column pass (see ColArgs in jms_kernels_impl.hpp).
@@ -143,6 +143,37 @@ struct GrpArgs {
   int w0 = 0;                     // first wave of the launch in the wave map
   int step = 0;                   // row pass: slice step; column pass: plane read out
 };
+// the whole slice loop of a batch of small waves (jms_loop_impl.hpp)
+struct LoopArgs {
+  float2* wave = nullptr;         // psi(k) of the exit plane (or nullptr: not kept)
+  long long wave_stride = 0;
+  const float2* src = nullptr;    // incident waves before the phase plate
+  long long src_stride = 0;       // 0: one shared source
+  const float4* ppar = nullptr;   // per wave (dx, dy, fz, 0) or nullptr
+  const int* var = nullptr;       // variant indices [wave][var_ld]
+  int var_ld = 0;
+  const float2* pgr = nullptr;    // phase gratings
+  const GrpPlane* pl = nullptr;   // plane table: slice offset, propagator and readout of each plane
+  int islc0 = 0, nslc = 0;        // slices [islc0, nslc)
+  const float* detw_t = nullptr;  // [ndet][nx][ny] detector weights
+  const float* cppl_t = nullptr;  // constant phase plate [x][y] or nullptr
+  int ndet = 0;
+  float* partial = nullptr;       // sums [wave][plane][detector] (one tile)
+  long long part_wstride = 0;
+  int dsx = 0, dsy = 0;           // diffraction de-scan [pixel]
+  float kscx = 0.f, kscy = 0.f;   // 1/a0x, 1/a0y [1/nm]
+  const float2* twx = nullptr;
+  const float2* twy = nullptr;
+  int gx0 = 0, gx1 = 0;           // columns left out (launch_loop's band)
+};
+// whether a batch of nwave waves runs as one launch
+bool loop_ok(int nx, int ny, int nwave);
+// band: columns [a.gx0, a.gx1) and the dead rows of the column transform are
+// zero in every propagator, the columns in the source
+hipError_t launch_loop(int nx, int ny, int nwave, const LoopArgs& a, bool band, hipStream_t st);
+// the band of the loop kernels: single columns instead of tiles
+BandHost loop_band(int nx, int ny, int gx0, int gx1, int gy0, int gy1);
+
 // grouped launches exist for grids whose column pass is the wave-local or
 // the long-column kernel
 bool grp_supported(int nx, int ny);

@@ -36,6 +36,8 @@ hipError_t launch_col_pass_grp_n(int nx, int nwave, bool init, bool exit_, bool 
                                  hipStream_t st);
 template <int NX>
 void band_row_n(int x0, int x1, int tile, BandHost& b);
+template <int NX, int NY>
+hipError_t launch_loop_n(int nwave, const LoopArgs& a, bool band, hipStream_t st);
 template <int NY>
 bool band_col_n(int y0, int y1);
 
@@ -368,6 +370,11 @@ int col_tiles(int ny, int nx, bool lat) {
   }
 }
 
+template <int NY>
+static bool band_loop_col_n(int y0, int y1) {
+  using BS = BandSlots<NY, radix_at<typename Cfg<NY>::PC, true>(0)>;
+  return BS::G0_MAX >= BS::G1_MIN || (y0 <= BS::G0_MAX && y1 >= BS::G1_MIN);
+}
 BandHost band_of(int nx, int ny, int gx0, int gx1, int gy0, int gy1, bool lat) {
   BandHost b;
   int tile = 0;
@@ -386,10 +393,54 @@ BandHost band_of(int nx, int ny, int gx0, int gx1, int gy0, int gy1, bool lat) {
 }
 
 bool lat_ok(int nx, int ny, int nwave) {
-  constexpr int kCUs = 256;  // MI355X
   // the long-column kernel has one shape; its launches fill the device
   const bool wl = ny != 1024 && ny != 2048;
-  return wl && nwave * col_tiles(ny, nx, false) < kCUs;
+  // a pair of passes in this shape / in Cfg's, us: 512^2 1 wave 10.8 / 13.2,
+  // 4 waves 17.0 / 16.2; 256^2 8 waves 12.4 / 12.7, 16 waves 16.8 / 15.3;
+  // 128^2 16 waves 8.8 / 9.3, 32 waves 11.8 / 11.0 (tiles: 32, 16, 8)
+  return wl && nwave * col_tiles(ny, nx, false) < 128;
+}
+
+// The slice loop in one launch takes one block per wave and CU (two at 64^2)
+// and is bound by arithmetic; two launches per slice are bound by latency for
+// few waves and by memory for many.  The measured lines (jms_loop_impl.hpp): a
+// wave of up to 4096 points is always faster in one launch; up to 9216 points
+// from about 32 waves on; up to 16384 points from about 112 waves on, as long
+// as the last round of 256 blocks is mostly full, and not beyond 1024 waves.
+bool loop_ok(int nx, int ny, int nwave) {
+  auto edge = [](int n) { return n == 64 || n == 96 || n == 128; };
+  if (!edge(nx) || !edge(ny)) return false;
+  const int n = nx * ny;
+  if (n <= 64 * 64) return true;
+  if (n <= 96 * 96) return nwave >= 32;
+  constexpr int kCUs = 256;
+  const int rounds = (nwave + kCUs - 1) / kCUs;
+  return nwave >= 112 && nwave <= 4 * kCUs && (rounds == 1 || nwave * 20 >= rounds * kCUs * 17);
+}
+BandHost loop_band(int nx, int ny, int gx0, int gx1, int gy0, int gy1) {
+  BandHost b;
+  switch (nx) {
+    case 64: band_row_n<64>(gx0, gx1, 1, b); break;
+    case 96: band_row_n<96>(gx0, gx1, 1, b); break;
+    case 128: band_row_n<128>(gx0, gx1, 1, b); break;
+  }
+  // the kernels' band has dead rows too; where the column plan has no slot
+  // that is dead, that asks for nothing
+  switch (ny) {
+    case 64: b.rows = band_loop_col_n<64>(gy0, gy1); break;
+    case 96: b.rows = band_loop_col_n<96>(gy0, gy1); break;
+    case 128: b.rows = band_loop_col_n<128>(gy0, gy1); break;
+  }
+  return b;
+}
+hipError_t launch_loop(int nx, int ny, int nwave, const LoopArgs& a, bool band, hipStream_t st) {
+  switch (nx * 1000 + ny) {
+#define JMS_LOOP(NX, NY) case NX * 1000 + NY: return launch_loop_n<NX, NY>(nwave, a, band, st);
+    JMS_LOOP(64, 64) JMS_LOOP(64, 96) JMS_LOOP(64, 128) JMS_LOOP(96, 64) JMS_LOOP(96, 96) JMS_LOOP(96, 128)
+    JMS_LOOP(128, 64) JMS_LOOP(128, 96) JMS_LOOP(128, 128)
+#undef JMS_LOOP
+    default: return hipErrorInvalidValue;
+  }
 }
 
 hipError_t launch_row_pass(int nx, int ny, int nwave, float2* wave, long long wave_stride,
