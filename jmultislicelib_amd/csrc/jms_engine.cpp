@@ -136,7 +136,13 @@ struct jms_hip_engine {
   int bcap_req = 0;
   DevBuf waves, partial, cur_var, cur_ppar, cur_res;
   // single-wave path: wave, variant sequence, results and channels
-  DevBuf wav, var1, res1, w1, dif1, wff1, img1, wfr1;
+  // in1: the run's weight and its variant sequence, one upload
+  DevBuf wav, in1, res1, dif1, wff1, img1, wfr1;
+  // pinned host side of a single-wave run: in1 as uploaded, and the integrated
+  // results as the run leaves them
+  float* pin = nullptr;
+  size_t pin_in = 0, pin_res = 0;  // capacities [items]
+  bool pin_valid = false;          // the results of the last run are in it
   // averaging channels (JMultiSlice.cpp:2489-2660): accumulated over runs until
   // reset, with the summed run weights of the image and wave groups
   DevBuf dif_avg, wff_avg, img_avg, wfr_avg;
@@ -332,11 +338,11 @@ bool use_loop(const jms_hip_engine* e, int nwave, int islc0) {
 // probe, else the single-wave path's wave; `keep`: leave psi(k) of the exit
 // plane in the waves (batches only read the sums).  The band's columns are
 // left out from the first slice on, and before it where the source is zero
-// there.
+// there.  `mirror` (or nullptr): host memory that gets the results too.
 int enqueue_batch(jms_hip_engine* e, void* waves, float* partial, int nwave, int islc0, const void* src,
                   long long src_stride, const void* ppar, const int* var, int npos, int npass,
                   const float* weights, float* res, int accumulate, const BatchChans& ch, bool timed,
-                  bool lat, bool src_same, bool keep, bool panel) {
+                  bool lat, bool src_same, bool keep, bool panel, float* mirror = nullptr) {
   const jms::BandHost bd = e->band(lat);
   const bool src_in = e->holds(src_same ? e->wav0_gap : e->wav_gap, bd);
   // panel waves (staged batches): integrated readouts only, the waves are internal
@@ -472,7 +478,7 @@ int enqueue_batch(jms_hip_engine* e, void* waves, float* partial, int nwave, int
     }
     TimedLaunch tl(e, 2, timed);
     err = jms::launch_combine(partial, ntc, e->ndet, e->ndetslc, npos, npass, weights,
-                              res, accumulate, e->st);
+                              res, accumulate, mirror, e->st);
     if (err != hipSuccess) return e->fail(133, "combine", err);
   }
   return 0;
@@ -484,6 +490,10 @@ int enqueue_batch(jms_hip_engine* e, void* waves, float* partial, int nwave, int
 int enqueue_exit_real_readout(jms_hip_engine* e, int nwave, const BatchChans& ch) {
   const int id = e->det_objslc[e->nobjslc];
   if (id < 0 || !ch.real_space()) return 0;
+  // works on a copy: the wave itself stays psi(k)
+  if (hipMemcpyAsync(e->waves.p, e->wav.p, sizeof(float) * 2 * (size_t)e->n * nwave, hipMemcpyDeviceToDevice, e->st) !=
+      hipSuccess)
+    return e->fail(134, "exit-plane wave copy");
   jms::RowChanHost rc;
   rc.img = ch.img;
   rc.img_avg = ch.img_avg;
@@ -563,10 +573,11 @@ void jms_hip_destroy(jms_hip_engine* e) {
   DevBuf* bufs[] = {&e->twx, &e->twy, &e->pgr, &e->pro, &e->pro_t, &e->loop_tab, &e->detw, &e->detw_t, &e->wav0,
                     &e->cppl, &e->cppl_t,
                     &e->s_ppar, &e->s_weights, &e->s_var, &e->s_res, &e->waves, &e->partial,
-                    &e->cur_var, &e->cur_ppar, &e->cur_res, &e->wav, &e->var1, &e->res1,
-                    &e->w1, &e->dif1, &e->wff1, &e->img1, &e->wfr1, &e->dif_avg, &e->wff_avg,
+                    &e->cur_var, &e->cur_ppar, &e->cur_res, &e->wav, &e->in1, &e->res1,
+                    &e->dif1, &e->wff1, &e->img1, &e->wfr1, &e->dif_avg, &e->wff_avg,
                     &e->img_avg, &e->wfr_avg};
   for (DevBuf* b : bufs) b->release();
+  if (e->pin) (void)hipHostFree(e->pin);
   if (e->st) (void)hipStreamDestroy(e->st);
   delete e;
 }
@@ -850,6 +861,7 @@ int jms_hip_setup_detection(jms_hip_engine* e, int ndetslc, const int* det_objsl
   e->detflags = flags;
   e->det_objslc.assign(det_objslc, det_objslc + e->nobjslc + 1);
   e->det_inf.assign(ndet, 0);
+  e->pin_valid = false;
   // averaging channels start empty (DetectorSetup, JMultiSlice.cpp:784-800)
   {
     const size_t nchan = (size_t)ndetslc * e->n;
@@ -1468,7 +1480,7 @@ int jms_hip_group_run(jms_hip_group* g) {
       TimedLaunch tl(lead, 2, lead->timing);
       err = jms::launch_combine(e->partial.as<float>(), ntc, e->ndet, e->ndetslc, nw / e->s_npass, e->s_npass,
                                 e->s_weights.as<float>(), e->s_res.as<float>() + (long long)rd.member_p0[k] * per, 0,
-                                st);
+                                nullptr, st);
       if (err != hipSuccess) return g->fail(133, "combine", err);
     }
   }
@@ -1513,7 +1525,6 @@ int jms_hip_wave_offset(jms_hip_engine* e, float dx, float dy, float dz, int ibt
   err = jms::launch_offset_wave(e->wav.as<float2>(), e->wav0.as<float2>(), e->nx, e->ny, 1.f / e->a0x,
                                 1.f / e->a0y, dx, dy, dz * e->wl * 0.5f,
                                 (use_cppl && e->have_cppl) ? e->cppl.as<float>() : nullptr, ish0, ish1, e->st);
-  if (err == hipSuccess) err = hipStreamSynchronize(e->st);
   if (err != hipSuccess) return e->fail(106, "offset incoming wave", err);
   return 0;
 }
@@ -1533,7 +1544,8 @@ int jms_hip_wave_get(jms_hip_engine* e, float* dst) {
   if (!e || !dst) return 1;
   if (!e->wav.p) return e->fail(2, "no wave");
   (void)hipSetDevice(e->device);
-  hipError_t err = hipMemcpy(dst, e->wav.p, sizeof(float) * 2 * (size_t)e->n, hipMemcpyDeviceToHost);
+  hipError_t err = hipStreamSynchronize(e->st);
+  if (err == hipSuccess) err = hipMemcpy(dst, e->wav.p, sizeof(float) * 2 * (size_t)e->n, hipMemcpyDeviceToHost);
   if (err != hipSuccess) return e->fail(102, "get wave", err);
   return 0;
 }
@@ -1555,9 +1567,20 @@ int jms_hip_multislice(jms_hip_engine* e, int islc0, const int* var, float weigh
   if (rc) return rc;
   const int per = e->ndetslc * std::max(1, e->ndet);
   const size_t nchan = (size_t)e->ndetslc * e->n;
+  const size_t nin = 1 + (size_t)S;
   hipError_t err = e->res1.ensure(sizeof(float) * per);
-  if (err == hipSuccess) err = e->w1.ensure(sizeof(float));
-  if (err == hipSuccess && S > 0) err = e->var1.ensure(sizeof(int) * S);
+  if (err == hipSuccess) err = e->in1.ensure(sizeof(float) * nin);
+  if (err == hipSuccess && (e->pin_in < nin || e->pin_res < (size_t)per)) {
+    if (e->pin) (void)hipHostFree(e->pin);
+    e->pin = nullptr;
+    e->pin_in = e->pin_res = 0;
+    err = hipHostMalloc((void**)&e->pin, sizeof(float) * (nin + per), hipHostMallocDefault);
+    if (err == hipSuccess) {
+      e->pin_in = nin;
+      e->pin_res = per;
+    }
+  }
+  e->pin_valid = false;
   const int fl = e->detflags;
   // per-run channels (cleared unless accumulating) and their buffers
   struct { DevBuf* b; int flag; size_t nb; } run[] = {
@@ -1568,17 +1591,21 @@ int jms_hip_multislice(jms_hip_engine* e, int islc0, const int* var, float weigh
   for (auto& r : run)
     if (err == hipSuccess && (fl & r.flag)) err = r.b->ensure(r.nb);
   if (err != hipSuccess) return e->fail(110, "allocate single-wave buffers", err);
+  const bool sums = (fl & JMS_HIP_DETECT_INTEGRATED) && e->ndet > 0;  // the combine writes every result
   if (!accumulate) {  // ClearDetMem_d (JMultiSlice.cpp:4054-4108); the averaging channels stay
-    err = hipMemsetAsync(e->res1.p, 0, sizeof(float) * per, e->st);
+    if (!sums) err = hipMemsetAsync(e->res1.p, 0, sizeof(float) * per, e->st);
     for (auto& r : run)
       if (err == hipSuccess && (fl & r.flag)) err = hipMemsetAsync(r.b->p, 0, r.nb, e->st);
     if (err != hipSuccess) return e->fail(111, "clear detector channels", err);
   }
-  err = hipMemcpyAsync(e->w1.p, &weight, sizeof(float), hipMemcpyHostToDevice, e->st);
-  if (err == hipSuccess && S > 0) err = hipMemcpyAsync(e->var1.p, var, sizeof(int) * S, hipMemcpyHostToDevice, e->st);
+  // every earlier run on the pinned buffer has been waited for
+  e->pin[0] = weight;
+  if (S > 0) memcpy(e->pin + 1, var, sizeof(int) * S);
+  err = hipMemcpyAsync(e->in1.p, e->pin, sizeof(float) * nin, hipMemcpyHostToDevice, e->st);
   if (err != hipSuccess) return e->fail(112, "stage single wave", err);
+  float* mirror = sums ? e->pin + e->pin_in : nullptr;
   BatchChans ch;
-  ch.cwgt = e->w1.as<float>();
+  ch.cwgt = e->in1.as<float>();
   if (fl & JMS_HIP_DETECT_DIFFRACTION) ch.dif = e->dif1.as<float>();
   if (fl & JMS_HIP_DETECT_IMAGE) ch.img = e->img1.as<float>();
   if (fl & JMS_HIP_DETECT_WAVEFOURIER) ch.wff = e->wff1.p;
@@ -1588,21 +1615,20 @@ int jms_hip_multislice(jms_hip_engine* e, int islc0, const int* var, float weigh
   if (fl & JMS_HIP_DETECT_WAVEF_AVG) ch.wff_avg = e->wff_avg.p;
   if (fl & JMS_HIP_DETECT_WAVER_AVG) ch.wfr_avg = e->wfr_avg.p;
   const bool lat = jms::lat_ok(e->nx, e->ny, 1);
-  rc = enqueue_batch(e, e->waves.p, e->partial.as<float>(), 1, islc0, e->wav.p, e->n, nullptr,
-                     e->var1.as<int>(), 1, 1, e->w1.as<float>(),
-                     e->res1.as<float>(), 1, ch, e->timing, lat, false, true, false);
+  // in place: every block of a pass reads its tile of the wave before it writes it
+  rc = enqueue_batch(e, e->wav.p, e->partial.as<float>(), 1, islc0, e->wav.p, e->n, nullptr, e->in1.as<int>() + 1, 1, 1,
+                     e->in1.as<float>(), e->res1.as<float>(), accumulate, ch, e->timing, lat, false, true, false,
+                     mirror);
   if (islc0 < S) {  // the wave becomes psi(k) of the exit plane
     const jms::BandHost bd = e->band(lat);
     e->wav_gap = rc ? Gap() : Gap{bd.x0, bd.x1, 0, 0};
   }
   if (rc) return rc;
-  // the run leaves psi(k) of the exit plane in the batch slot; keep it as the wave
-  err = hipMemcpyAsync(e->wav.p, e->waves.p, sizeof(float) * 2 * (size_t)e->n, hipMemcpyDeviceToDevice, e->st);
-  if (err != hipSuccess) return e->fail(113, "multislice run", err);
   rc = enqueue_exit_real_readout(e, 1, ch);
   if (rc) return rc;
   err = hipStreamSynchronize(e->st);
   if (err != hipSuccess) return e->fail(113, "multislice run", err);
+  e->pin_valid = mirror != nullptr;
   // averaging weights count the runs that fed the averaging channels (:4668-4673)
   if (fl & (JMS_HIP_DETECT_DIFFR_AVG | JMS_HIP_DETECT_IMAGE_AVG)) e->w_imgavg += weight;
   if (fl & (JMS_HIP_DETECT_WAVEF_AVG | JMS_HIP_DETECT_WAVER_AVG)) e->w_wavavg += weight;
@@ -1617,6 +1643,11 @@ int jms_hip_get_result(jms_hip_engine* e, int which, float* dst) {
   if (err != hipSuccess) return e->fail(101, "synchronize", err);
   if (which == JMS_HIP_DETECT_INTEGRATED) {
     if (!e->res1.p) return e->fail(2, "no result");
+    const size_t nr = (size_t)e->ndetslc * e->ndet;
+    if (e->pin_valid && nr <= e->pin_res) {  // the run was waited for
+      memcpy(dst, e->pin + e->pin_in, sizeof(float) * nr);
+      return 0;
+    }
     err = hipMemcpy(dst, e->res1.p, sizeof(float) * (size_t)e->ndetslc * e->ndet, hipMemcpyDeviceToHost);
   } else if (which == JMS_HIP_DETECT_DIFFRACTION) {
     if (!e->dif1.p) return e->fail(3, "diffraction channel not active");

@@ -218,7 +218,7 @@ hipError_t launch_fft2d(int nx, int ny, int nbatch, float2* data, int dir, const
 hipError_t launch_zero_partial(float* partial, long long part_w, long long off, int len, int nwave,
                                hipStream_t st);
 hipError_t launch_combine(const float* partial, int ntiles, int ndet, int ndetslc, int npos,
-                          int npass, const float* weights, float* out, int accumulate,
+                          int npass, const float* weights, float* out, int accumulate, float* mirror,
                           hipStream_t st);
 hipError_t launch_offset_wave(float2* out, const float2* in, int nx, int ny, float kscx,
                               float kscy, float dx, float dy, float fz, const float* cppl,

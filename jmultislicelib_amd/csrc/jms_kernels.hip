@@ -51,10 +51,12 @@ __device__ __forceinline__ int fidx(int i, int n) {
 // ---------------------------------------------------------------------------
 // combine partial detector sums of a batch into per-position results:
 //   out[(p0+p), idet, d] (+)= sum_r weight[r] * sum_tile partial[(p*npass+r), idet, d, tile]
+// mirror (or nullptr): the same values in host memory, for a caller that reads
+// them right after the run
 // ---------------------------------------------------------------------------
 __global__ void k_combine(const float* __restrict__ partial, int ntiles, int ndet, int ndetslc,
                           int npos, int npass, const float* __restrict__ weights,
-                          float* __restrict__ out, int accumulate) {
+                          float* __restrict__ out, int accumulate, float* __restrict__ mirror) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   const int per = ndetslc * ndet;
   if (i >= npos * per) return;
@@ -66,7 +68,9 @@ __global__ void k_combine(const float* __restrict__ partial, int ntiles, int nde
     for (int k = 0; k < ntiles; ++k) s += (double)src[k];
     acc += (double)weights[r] * s;
   }
-  out[i] = accumulate ? (float)((double)out[i] + acc) : (float)acc;
+  const float r = accumulate ? (float)((double)out[i] + acc) : (float)acc;
+  out[i] = r;
+  if (mirror) mirror[i] = r;
 }
 
 __global__ void k_zero_partial(float* __restrict__ partial, long long part_w, long long off, int len) {
@@ -549,12 +553,12 @@ hipError_t launch_fft2d(int nx, int ny, int nbatch, float2* data, int dir, const
 }
 
 hipError_t launch_combine(const float* partial, int ntiles, int ndet, int ndetslc, int npos,
-                          int npass, const float* weights, float* out, int accumulate,
+                          int npass, const float* weights, float* out, int accumulate, float* mirror,
                           hipStream_t st) {
   const int total = npos * ndetslc * ndet;
   if (total <= 0) return hipSuccess;
   hipLaunchKernelGGL(k_combine, dim3((total + 255) / 256), dim3(256), 0, st, partial, ntiles, ndet,
-                     ndetslc, npos, npass, weights, out, accumulate);
+                     ndetslc, npos, npass, weights, out, accumulate, mirror);
   return hipGetLastError();
 }
 
