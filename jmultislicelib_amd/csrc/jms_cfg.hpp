@@ -151,5 +151,20 @@ struct Lat : CfgP<N> {
   static constexpr bool PF = true;
 };
 
+// Cfg's shape for waves that stay in the 256 MB Infinity Cache from one pass
+// to the next (split_of in jms_engine.cpp): ordinary loads and stores, as
+// nontemporal ones make the cache drop the lines that the next pass reads, and
+// row blocks in block_xy's order, so the waves that meet a variant's grating
+// rows find them in one L2 (all variants of a slice exceed it: 16 MiB for eight
+// at 512^2; streamed waves want the order of their addresses instead).  A row
+// and a column pass with eight variants, 154 MiB of waves stored, on MI355X, ms
+// per 2 GiB of waves, this shape / the order of addresses / nontemporal (176
+// MiB): 256^2 0.99 / 0.99 / 1.18, 512^2 1.05 / 1.09 / 1.16, 640^2
+// 1.37 / 1.52 / 1.71, 720^2 1.49 / 1.58 / 1.76.
+template <int N>
+struct Near : CfgP<N> {
+  static constexpr bool NT_ROW = false, NT_COL = false;
+  static constexpr bool XCD_ROW = true;
+};
 
 }  // namespace jms

@@ -96,6 +96,10 @@ void group_member_gone(jms_hip_group* g, jms_hip_engine* e);
 struct jms_hip_engine {
   int device = 0;
   hipStream_t st = nullptr;
+  // second stream of staged batches, made by the first staged run, and the
+  // events that tie its work to st (SideBranch)
+  hipStream_t side = nullptr;
+  hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   std::string err;
   std::vector<jms_hip_group*> groups;  // grouped launches this engine is a member of
   // grid
@@ -154,7 +158,8 @@ struct jms_hip_engine {
   // addresses of every buffer the batch reads or writes (graph_bufs): when
   // any of them moves, all graphs are dropped before the next capture.
   bool use_graph = false;
-  std::map<std::array<int, 4>, hipGraphExec_t> graphs;
+  // (a batch that goes in two halves: one graph for each, the second for `side`)
+  std::map<std::array<int, 4>, std::array<hipGraphExec_t, 2>> graphs;
   std::array<const void*, 17> graph_bufs{};
   std::array<int, 12> graph_band{};  // and to the band the launches were made for
   // this device's scratch of the allocation-free batch entry (resolved at create)
@@ -181,7 +186,9 @@ struct jms_hip_engine {
     return code;
   }
   void drop_graphs() {
-    for (auto& kv : graphs) (void)hipGraphExecDestroy(kv.second);
+    for (auto& kv : graphs)
+      for (hipGraphExec_t g : kv.second)
+        if (g) (void)hipGraphExecDestroy(g);
     graphs.clear();
   }
   // device addresses a captured batch depends on
@@ -329,6 +336,89 @@ bool use_loop(const jms_hip_engine* e, int nwave, int islc0) {
   return e->loop_ready && islc0 < e->nobjslc && jms::loop_ok(e->nx, e->ny, nwave);
 }
 
+// How the passes of a batch go over its waves.  As one launch over all of them
+// per pass, every pass reads from memory what the last one wrote there.  Parts
+// whose stored waves fit the 256 MB Infinity Cache beside the gratings of two
+// slices go through all slices one after the other instead, so the waves come
+// from the cache, and each part goes in two halves on two streams, so the start
+// and end of a launch (about 5 us in which the device is partly empty) lie
+// beside the other half's work.  Eight variants, two slice types, ms per 2 GiB
+// of waves and pair of passes on MI355X, all 2 GiB per launch / parts of 143
+// MiB stored, one stream / two:
+//   160^2 1.46 / 1.31 / 1.20   256^2 1.10 / 1.05 / 1.02   360^2 1.70 / 1.67 / 1.58
+//   512^2 1.13 / 1.10 / 1.13   625^2 2.18 / 2.17 / 2.01   640^2 1.61 / 1.56 / 1.46
+//   720^2 1.74 / 1.71 / 1.60   1024^2 1.49 / 1.55 / 1.44
+// and a batch of that size as one streamed launch per pass: 256^2 1.21, 512^2
+// 1.20, 625^2 2.34, 720^2 1.78.  At 184 MiB stored 512^2 is back at 1.19.
+// Waves above kNearWave leave a part too few of them to fill the device (2048^2
+// 1.63, in parts 1.70); halves of less than kTwoBytes together are no faster
+// (256^2, 22 MiB stored: 1.66 on one stream, 1.73 on two; 44 MiB: 1.37, 1.32).
+constexpr long long kNearBytes = 184LL << 20, kNearWave = 8LL << 20, kTwoBytes = 40LL << 20;
+struct Split {
+  int rounds = 1;
+  bool near = false, two = false;
+};
+Split split_of(const jms_hip_engine* e, int nwave, const jms::BandHost& bd, bool lat, bool chans) {
+  Split s;
+  if (lat) return s;
+  int nvar = 1;
+  for (int v : e->nvarslc) nvar = std::max(nvar, v);
+  const long long per = 8LL * e->ny * (e->nx - (bd.x1 - bd.x0)), all = per * nwave;
+  // beside the waves: the variants of this slice and of the next
+  const long long room = std::max(kNearBytes - 16LL * nvar * e->npgx * e->npgy, kNearBytes / 2);
+  if (all > room && (per > kNearWave || chans)) return s;
+  s.near = true;
+  if (chans) return s;
+  s.rounds = (int)((all + room - 1) / room);
+  s.two = all >= kTwoBytes * s.rounds && nwave >= 2 * s.rounds;
+  return s;
+}
+// the second stream's work between two points of the engine's stream; also
+// inside a capture of the engine's stream
+struct SideBranch {
+  jms_hip_engine* e;
+  bool open = false;
+  hipError_t err = hipSuccess;
+  SideBranch(jms_hip_engine* e_, bool on) : e(e_) {
+    if (!on) return;
+    err = hipEventRecord(e->ev_fork, e->st);
+    if (err == hipSuccess) err = hipStreamWaitEvent(e->side, e->ev_fork, 0);
+    open = err == hipSuccess;
+  }
+  hipError_t join() {
+    if (!open) return hipSuccess;
+    open = false;
+    hipError_t r = hipEventRecord(e->ev_join, e->side);
+    if (r == hipSuccess) r = hipStreamWaitEvent(e->st, e->ev_join, 0);
+    return r;
+  }
+  ~SideBranch() { (void)join(); }
+};
+
+// the batch's partial sums combined into `res` (npos results)
+int enqueue_combine(jms_hip_engine* e, float* partial, int nwave, int islc0, int ntc, int npos, int npass,
+                    const float* weights, float* res, int accumulate, bool timed, float* mirror) {
+  const int ndet = (e->detflags & JMS_HIP_DETECT_INTEGRATED) ? e->ndet : 0, S = e->nobjslc;
+  if (npass < 1 || !res || ndet < 1) return 0;
+  const long long part_w = (long long)e->ndetslc * ndet * ntc;
+  hipError_t err;
+  // detection planes before islc0 are not read out in this batch: their
+  // partial sums hold nothing of it (GPUMultislice reads only the planes
+  // from islc0 on, JMultiSlice.cpp:4568-4590)
+  for (int p = 0; p < islc0 && p <= S; ++p) {
+    const int id = e->det_objslc[p];
+    bool later = false;
+    for (int q = islc0; q <= S && !later; ++q) later = e->det_objslc[q] == id;
+    if (id < 0 || later) continue;
+    err = jms::launch_zero_partial(partial, part_w, (long long)id * ndet * ntc, ndet * ntc, nwave, e->st);
+    if (err != hipSuccess) return e->fail(134, "clear unread planes", err);
+  }
+  TimedLaunch tl(e, 2, timed);
+  err = jms::launch_combine(partial, ntc, ndet, e->ndetslc, npos, npass, weights, res, accumulate, mirror, e->st);
+  if (err != hipSuccess) return e->fail(133, "combine", err);
+  return 0;
+}
+
 // Launch sequence of one batch.  `waves` holds the nwave working waves
 // (stride n); `ppar` (float4 per wave) and `var` (nobjslc ints per wave)
 // describe them; src/src_stride the INIT source.  Readout partial sums go to
@@ -338,11 +428,13 @@ bool use_loop(const jms_hip_engine* e, int nwave, int islc0) {
 // probe, else the single-wave path's wave; `keep`: leave psi(k) of the exit
 // plane in the waves (batches only read the sums).  The band's columns are
 // left out from the first slice on, and before it where the source is zero
-// there.  `mirror` (or nullptr): host memory that gets the results too.
+// there.  `mirror` (or nullptr): host memory that gets the results too.  `half`
+// 0 or 1: only the passes of the first or second halves of a batch that goes in
+// two (split_of), on the engine's stream, without the combination.
 int enqueue_batch(jms_hip_engine* e, void* waves, float* partial, int nwave, int islc0, const void* src,
                   long long src_stride, const void* ppar, const int* var, int npos, int npass,
                   const float* weights, float* res, int accumulate, const BatchChans& ch, bool timed,
-                  bool lat, bool src_same, bool keep, bool panel, float* mirror = nullptr) {
+                  bool lat, bool src_same, bool keep, bool panel, float* mirror = nullptr, int half = -1) {
   const jms::BandHost bd = e->band(lat);
   const bool src_in = e->holds(src_same ? e->wav0_gap : e->wav_gap, bd);
   // panel waves (staged batches): integrated readouts only, the waves are internal
@@ -353,7 +445,6 @@ int enqueue_batch(jms_hip_engine* e, void* waves, float* partial, int nwave, int
   const int ntc = loop ? 1 : e->ntiles_col(lat);
   const long long part_w = (long long)e->ndetslc * e->ndet * ntc;
   jms::ColArgsHost ca;
-  ca.lat = lat;
   ca.wave = waves;
   ca.nx = e->nx;
   ca.wave_stride = e->n;
@@ -425,63 +516,75 @@ int enqueue_batch(jms_hip_engine* e, void* waves, float* partial, int nwave, int
                            e->st);
     if (err != hipSuccess) return e->fail(132, "slice loop", err);
   } else {
-    // INIT column pass: plane islc0
-    {
-      ca.src = src;
-      ca.src_stride = src_stride;
-      ca.ppar = ppar;
-      ca.pro = nullptr;
-      plane_setup(islc0);
-      if (src_in && islc0 < S) ca.band = bd;
+    const Split sp = split_of(e, nwave, bd, lat, ch.any());
+    // one stream where each launch is timed
+    const bool two = half >= 0 || (sp.two && !timed && e->side);
+    const int parts = sp.rounds * (two ? 2 : 1);
+    const jms::Shape shape = lat ? jms::Shape::Small : sp.near ? jms::Shape::Near : jms::Shape::Stream;
+    ca.shape = shape;
+    SideBranch branch(e, two && half < 0);
+    if (branch.err != hipSuccess) return e->fail(129, "second stream", branch.err);
+    struct Part {
+      int w0, nw;
+      hipStream_t st;
+    };
+    // INIT column pass of a part: plane islc0
+    auto init = [&](const Part& q) {
+      jms::ColArgsHost c = ca;
+      c.wave = (float2*)waves + q.w0 * e->n;
+      c.partial = partial + q.w0 * part_w;
+      c.src = (const float2*)src + q.w0 * src_stride;
+      c.src_stride = src_stride;
+      c.ppar = ppar ? (const float4*)ppar + q.w0 : nullptr;
+      if (src_in && islc0 < S) c.band = bd;
       TimedLaunch tl(e, 1, timed);
-      err = jms::launch_col_pass(e->ny, nwave, true, islc0 >= S, ca, e->st);
-      if (err != hipSuccess) return e->fail(130, "column pass (init)", err);
-    }
-    ca.src = nullptr;
-    ca.ppar = nullptr;
-    ca.band = bd;
-    for (int j = islc0; j < S; ++j) {
-      const int js = e->objslc[j] % e->nscslc;
-      {
+      return jms::launch_col_pass(e->ny, q.nw, true, islc0 >= S, c, q.st);
+    };
+    auto row = [&](const Part& q, int j, int js, int mode) {
+      TimedLaunch tl(e, 0, timed);
+      return jms::launch_row_pass(e->nx, e->ny, q.nw, (float2*)waves + q.w0 * e->n, e->n, e->pgr.as<float2>(),
+                                  e->slcoffset[js], (long long)e->npgx * e->npgy, S > 0 ? var + (long long)q.w0 * S : var,
+                                  S, j, e->twx.as<float2>(), rc, mode, panel,
+                                  j > islc0 || src_in ? bd : jms::BandHost(), shape, q.st);
+    };
+    auto col = [&](const Part& q, int j, int js) {
+      jms::ColArgsHost c = ca;
+      c.wave = (float2*)waves + q.w0 * e->n;
+      c.partial = partial + q.w0 * part_w;
+      c.band = bd;
+      c.pro = e->pro.as<float2>() + (long long)e->proidx[js] * e->n;
+      c.pro_t = e->pro_t.as<float2>() + (long long)e->proidx[js] * e->n;
+      TimedLaunch tl(e, 1, timed);
+      return jms::launch_col_pass(e->ny, q.nw, false, j == S - 1, c, q.st);
+    };
+    for (int r = 0; r < sp.rounds; ++r) {
+      std::vector<Part> pt;
+      for (int h = 0; h < (two ? 2 : 1); ++h) {
+        if (half >= 0 && h != half) continue;
+        const int p = r * (two ? 2 : 1) + h;
+        const int w0 = (int)((long long)nwave * p / parts), w1 = (int)((long long)nwave * (p + 1) / parts);
+        pt.push_back({w0, w1 - w0, h && half < 0 ? e->side : e->st});
+      }
+      plane_setup(islc0);
+      for (const Part& q : pt)
+        if ((err = init(q)) != hipSuccess) return e->fail(130, "column pass (init)", err);
+      for (int j = islc0; j < S; ++j) {
+        const int js = e->objslc[j] % e->nscslc;
         // real-space readout of plane j inside the row pass (ReadoutImgDet_d)
         const int id = e->det_objslc[j];
         const int mode = (id >= 0 && ch.real_space()) ? 1 : 0;
         rc.chan_off = id >= 0 ? (long long)id * e->n : 0;
-        TimedLaunch tl(e, 0, timed);
-        err = jms::launch_row_pass(e->nx, e->ny, nwave, (float2*)waves, e->n,
-                                   e->pgr.as<float2>(), e->slcoffset[js], (long long)e->npgx * e->npgy,
-                                   var, S, j, e->twx.as<float2>(), rc, mode, panel,
-                                   j > islc0 || src_in ? bd : jms::BandHost(), lat, e->st);
-        if (err != hipSuccess) return e->fail(131, "row pass", err);
-      }
-      ca.pro = e->pro.as<float2>() + (long long)e->proidx[js] * e->n;
-      ca.pro_t = e->pro_t.as<float2>() + (long long)e->proidx[js] * e->n;
-      plane_setup(j + 1);
-      {
-        TimedLaunch tl(e, 1, timed);
-        err = jms::launch_col_pass(e->ny, nwave, false, j == S - 1, ca, e->st);
-        if (err != hipSuccess) return e->fail(132, "column pass", err);
+        plane_setup(j + 1);
+        for (const Part& q : pt) {
+          if ((err = row(q, j, js, mode)) != hipSuccess) return e->fail(131, "row pass", err);
+          if ((err = col(q, j, js)) != hipSuccess) return e->fail(132, "column pass", err);
+        }
       }
     }
+    if ((err = branch.join()) != hipSuccess) return e->fail(129, "second stream", err);
   }
-  if (npass > 0 && res && ca.ndet > 0) {
-    // detection planes before islc0 are not read out in this batch: their
-    // partial sums hold nothing of it (GPUMultislice reads only the planes
-    // from islc0 on, JMultiSlice.cpp:4568-4590)
-    for (int p = 0; p < islc0 && p <= S; ++p) {
-      const int id = e->det_objslc[p];
-      bool later = false;
-      for (int q = islc0; q <= S && !later; ++q) later = e->det_objslc[q] == id;
-      if (id < 0 || later) continue;
-      err = jms::launch_zero_partial(partial, part_w, (long long)id * e->ndet * ntc, e->ndet * ntc, nwave, e->st);
-      if (err != hipSuccess) return e->fail(134, "clear unread planes", err);
-    }
-    TimedLaunch tl(e, 2, timed);
-    err = jms::launch_combine(partial, ntc, e->ndet, e->ndetslc, npos, npass, weights,
-                              res, accumulate, mirror, e->st);
-    if (err != hipSuccess) return e->fail(133, "combine", err);
-  }
-  return 0;
+  if (half >= 0) return 0;
+  return enqueue_combine(e, partial, nwave, islc0, ntc, npos, npass, weights, res, accumulate, timed, mirror);
 }
 
 // exit-plane real-space readout (GPUMultislice :4662-4666): the column IFFT
@@ -505,7 +608,7 @@ int enqueue_exit_real_readout(jms_hip_engine* e, int nwave, const BatchChans& ch
   hipError_t err = jms::launch_col_fft(e->nx, e->ny, nwave, e->waves.as<float2>(), +1, e->twy.as<float2>(), e->st);
   if (err == hipSuccess)
     err = jms::launch_row_pass(e->nx, e->ny, nwave, e->waves.as<float2>(), e->n, e->pgr.as<float2>(), 0, 0,
-                               nullptr, 0, 0, e->twx.as<float2>(), rc, 2, false, jms::BandHost(), false, e->st);
+                               nullptr, 0, 0, e->twx.as<float2>(), rc, 2, false, jms::BandHost(), jms::Shape::Stream, e->st);
   if (err != hipSuccess) return e->fail(134, "exit-plane real-space readout", err);
   return 0;
 }
@@ -527,6 +630,16 @@ int ensure_batch(jms_hip_engine* e, int nwave) {
   err = e->partial.ensure(np);
   if (err != hipSuccess) return e->fail(111, "allocate readout partials", err);
   return 0;
+}
+
+// the second stream and its events (before a capture begins)
+int ensure_side(jms_hip_engine* e) {
+  if (e->side) return 0;
+  hipError_t err = hipSuccess;
+  if (!e->ev_fork) err = hipEventCreateWithFlags(&e->ev_fork, hipEventDisableTiming);
+  if (err == hipSuccess && !e->ev_join) err = hipEventCreateWithFlags(&e->ev_join, hipEventDisableTiming);
+  if (err == hipSuccess) err = hipStreamCreateWithFlags(&e->side, hipStreamNonBlocking);
+  return err == hipSuccess ? 0 : e->fail(112, "second stream", err);
 }
 
 // default batch: about 2 GiB of resident waves
@@ -578,6 +691,9 @@ void jms_hip_destroy(jms_hip_engine* e) {
                     &e->img_avg, &e->wfr_avg};
   for (DevBuf* b : bufs) b->release();
   if (e->pin) (void)hipHostFree(e->pin);
+  if (e->ev_fork) (void)hipEventDestroy(e->ev_fork);
+  if (e->ev_join) (void)hipEventDestroy(e->ev_join);
+  if (e->side) (void)hipStreamDestroy(e->side);
   if (e->st) (void)hipStreamDestroy(e->st);
   delete e;
 }
@@ -1087,6 +1203,8 @@ int jms_hip_run_staged(jms_hip_engine* e, int pos0, int npos, int islc0) {
   bw = bpos * npass;
   rc = ensure_batch(e, bw);
   if (rc) return rc;
+  rc = ensure_side(e);
+  if (rc) return rc;
   const int S = e->nobjslc;
   const int per = e->ndetslc * std::max(1, e->ndet);
   for (int p = pos0; p < pos0 + npos; p += bpos) {
@@ -1118,26 +1236,44 @@ int jms_hip_run_staged(jms_hip_engine* e, int pos0, int npos, int islc0) {
       }
       const std::array<int, 4> key{nw, islc0, np, npass};
       auto it = e->graphs.find(key);
+      const int ntc = e->ntiles_col(lat);
+      const bool two = !use_loop(e, nw, islc0) && split_of(e, nw, b0, lat, false).two;
       if (it == e->graphs.end()) {
-        hipGraph_t g = nullptr;
-        err = hipStreamBeginCapture(e->st, hipStreamCaptureModeThreadLocal);
-        if (err != hipSuccess) return e->fail(121, "begin capture", err);
-        rc = enqueue_batch(e, e->waves.p, e->partial.as<float>(), nw, islc0, e->wav0.p, 0, e->cur_ppar.p,
-                           e->cur_var.as<int>(), np,
-                           npass, e->s_weights.as<float>(), e->cur_res.as<float>(), 0, BatchChans(), false,
-                           lat, true, false, panel);
-        hipError_t err2 = hipStreamEndCapture(e->st, &g);
-        if (rc) { if (g) (void)hipGraphDestroy(g); return rc; }
-        if (err2 != hipSuccess) return e->fail(122, "end capture", err2);
-        hipGraphExec_t ge = nullptr;
-        err = hipGraphInstantiate(&ge, g, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(g);
-        if (err != hipSuccess) return e->fail(123, "instantiate graph", err);
+        std::array<hipGraphExec_t, 2> ge{};
+        for (int h = 0; h < (two ? 2 : 1); ++h) {
+          hipGraph_t g = nullptr;
+          err = hipStreamBeginCapture(e->st, hipStreamCaptureModeThreadLocal);
+          if (err != hipSuccess) rc = e->fail(121, "begin capture", err);
+          else {
+            rc = enqueue_batch(e, e->waves.p, e->partial.as<float>(), nw, islc0, e->wav0.p, 0, e->cur_ppar.p,
+                               e->cur_var.as<int>(), np, npass, e->s_weights.as<float>(), e->cur_res.as<float>(), 0,
+                               BatchChans(), false, lat, true, false, panel, nullptr, two ? h : -1);
+            err = hipStreamEndCapture(e->st, &g);
+            if (!rc && err != hipSuccess) rc = e->fail(122, "end capture", err);
+          }
+          if (!rc) {
+            err = hipGraphInstantiate(&ge[h], g, nullptr, nullptr, 0);
+            if (err != hipSuccess) rc = e->fail(123, "instantiate graph", err);
+          }
+          if (g) (void)hipGraphDestroy(g);
+          if (rc) {
+            if (ge[0]) (void)hipGraphExecDestroy(ge[0]);
+            return rc;
+          }
+        }
         it = e->graphs.emplace(key, ge).first;
       }
       {
         TimedLaunch tl(e, 3, e->timing);  // one replay = the batch's whole launch sequence
-        err = hipGraphLaunch(it->second, e->st);
+        SideBranch branch(e, two);
+        err = branch.err;
+        if (err == hipSuccess) err = hipGraphLaunch(it->second[0], e->st);
+        if (err == hipSuccess && two) err = hipGraphLaunch(it->second[1], e->side);
+        if (err == hipSuccess) err = branch.join();
+        if (err == hipSuccess && two)
+          rc = enqueue_combine(e, e->partial.as<float>(), nw, islc0, ntc, np, npass, e->s_weights.as<float>(),
+                               e->cur_res.as<float>(), 0, false, nullptr);
+        if (rc) return rc;
       }
       if (err == hipSuccess)
         err = hipMemcpyAsync(res, e->cur_res.p, sizeof(float) * (size_t)np * per, hipMemcpyDeviceToDevice, e->st);

@@ -18,6 +18,9 @@ struct BandHost {
 // the band the passes of an nx x ny grid use, given columns [gx0, gx1) and
 // rows [gy0, gy1) where every propagator of the run vanishes
 BandHost band_of(int nx, int ny, int gx0, int gx1, int gy0, int gy1, bool lat);
+// launch shapes of a batch's passes: waves streamed from memory (Cfg in
+// jms_cfg.hpp), few blocks (Lat; see lat_ok), waves in the Infinity Cache (Near)
+enum class Shape { Stream, Small, Near };
 // whether a batch of nwave waves takes the small launch shapes (Lat in
 // jms_cfg.hpp; natural wave layout): its column pass would have fewer than 128
 // blocks
@@ -57,7 +60,7 @@ struct ColArgsHost {
   bool panel = false;            // the waves are in 16-column panels (panel_ok)
   BandHost band;                 // columns and rows left out
   bool keep = false;             // EXIT: store psi(k), the columns left out cleared
-  bool lat = false;              // small launch shapes (lat_ok)
+  Shape shape = Shape::Stream;
 };
 
 // real-space readout channels of one detection plane for the row pass
@@ -201,7 +204,7 @@ int col_tiles(int ny, int nx, bool lat);
 hipError_t launch_row_pass(int nx, int ny, int nwave, float2* wave, long long wave_stride,
                            const float2* pgr, long long slc_off, long long npg, const int* var_tab,
                            int var_ld, int jslc, const float2* twx, const RowChanHost& rc, int mode,
-                           bool panel, const BandHost& bd, bool lat, hipStream_t st);
+                           bool panel, const BandHost& bd, Shape shape, hipStream_t st);
 // whether the staged batches of an nx x ny grid keep their waves in panels of
 // 16 columns: element (y, x) at (x / 16) * 16 ny + 16 y + x % 16 (column
 // tiles contiguous); chosen per line length where the passes run faster so

@@ -16,7 +16,7 @@ template <int N>
 hipError_t launch_row_pass_n(int ny, int nwave, float2* wave, long long wave_stride,
                              const float2* pgr, long long slc_off, long long npg,
                              const int* var_tab, int var_ld, int jslc, const float2* twx,
-                             const RowChanHost& rc, int mode, bool panel, const BandHost& bd, bool lat,
+                             const RowChanHost& rc, int mode, bool panel, const BandHost& bd, Shape shape,
                              hipStream_t st);
 template <int N>
 hipError_t launch_col_pass_n(int nwave, bool init, bool exit_, const ColArgsHost& h,
@@ -450,12 +450,12 @@ hipError_t launch_loop(int nx, int ny, int nwave, const LoopArgs& a, bool band, 
 hipError_t launch_row_pass(int nx, int ny, int nwave, float2* wave, long long wave_stride,
                            const float2* pgr, long long slc_off, long long npg, const int* var_tab,
                            int var_ld, int jslc, const float2* twx, const RowChanHost& rc, int mode,
-                           bool panel, const BandHost& bd, bool lat, hipStream_t st) {
+                           bool panel, const BandHost& bd, Shape shape, hipStream_t st) {
   switch (nx) {
 #define JMS_CASE(N)                                                                         \
   case N:                                                                                   \
     return launch_row_pass_n<N>(ny, nwave, wave, wave_stride, pgr, slc_off, npg, var_tab, \
-                                var_ld, jslc, twx, rc, mode, panel, bd, lat, st);
+                                var_ld, jslc, twx, rc, mode, panel, bd, shape, st);
     JMS_SIZES(JMS_CASE)
 #undef JMS_CASE
     default: return hipErrorInvalidValue;

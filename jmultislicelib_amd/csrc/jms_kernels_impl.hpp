@@ -1189,10 +1189,12 @@ template <int N>
 hipError_t launch_row_pass_n(int ny, int nwave, float2* wave, long long wave_stride,
                              const float2* pgr, long long slc_off, long long npg,
                              const int* var_tab, int var_ld, int jslc, const float2* twx,
-                             const RowChanHost& h, int mode, bool panel, const BandHost& bd, bool lat,
+                             const RowChanHost& h, int mode, bool panel, const BandHost& bd, Shape shape,
                              hipStream_t st) {
   using CF = Cfg<N>;
   using CL = Lat<N>;
+  using CN = std::conditional_t<CF::NT_ROW, Near<N>, CF>;  // where ordinary accesses make a difference
+  const bool lat = shape == Shape::Small;
   RowChan rc;
   rc.img = h.img; rc.img_avg = h.img_avg;
   rc.wfr = (float2*)h.wfr; rc.wfr_avg = (float2*)h.wfr_avg;
@@ -1212,11 +1214,18 @@ hipError_t launch_row_pass_n(int ny, int nwave, float2* wave, long long wave_str
   else if (mode == 1) go(k_row_pass<N, 1>);
   else if (lat && band) go(k_row_pass<N, 0, CL, false, false, true>);
   else if (lat) go(k_row_pass<N, 0, CL>);
-  else if (!panel && band) go(k_row_pass<N, 0, CF, false, false, true>);
-  else if (!panel) go(k_row_pass<N, 0>);
-  else if constexpr (CF::PANEL) {
-    if (band) go(k_row_pass<N, 0, CF, false, true, true>);
-    else go(k_row_pass<N, 0, CF, false, true>);
+  else {
+    auto pick = [&](auto c) {
+      using CS = decltype(c);
+      if (!panel && band) go(k_row_pass<N, 0, CS, false, false, true>);
+      else if (!panel) go(k_row_pass<N, 0, CS>);
+      else if constexpr (CF::PANEL) {
+        if (band) go(k_row_pass<N, 0, CS, false, true, true>);
+        else go(k_row_pass<N, 0, CS, false, true>);
+      }
+    };
+    if (shape == Shape::Near) pick(CN{});
+    else pick(CF{});
   }
   return hipGetLastError();
 }
@@ -1294,8 +1303,9 @@ hipError_t launch_col_pass_n(int nwave, bool init, bool exit_, const ColArgsHost
   a.cppl_t = h.cppl_t;
   using CF = Cfg<N>;
   static_assert(CF::XL || CF::WL, "every line length has a column kernel");
-  if (h.panel && (!CF::PANEL || h.lat)) return hipErrorInvalidValue;
-  const int cc = h.lat ? Lat<N>::CC : CF::CC, tiles = (h.nx + cc - 1) / cc;
+  const bool lat = h.shape == Shape::Small;
+  if (h.panel && (!CF::PANEL || lat)) return hipErrorInvalidValue;
+  const int cc = lat ? Lat<N>::CC : CF::CC, tiles = (h.nx + cc - 1) / cc;
   a.tg0 = h.band.x0 / cc;
   a.tgn = h.band.on() ? (h.band.x1 - h.band.x0) / cc : 0;
   a.keep = h.keep;
@@ -1307,9 +1317,15 @@ hipError_t launch_col_pass_n(int nwave, bool init, bool exit_, const ColArgsHost
     else if constexpr (CF::PANEL) launch_col_x<N, CF, true>(g, b, init, exit_, h.detect, a, st);
   } else {
     dim3 b(CF::TW * cc);
-    if (h.lat) launch_col_w<N, Lat<N>, false, false>(g, b, init, exit_, h.detect, h.band.rows, a, st);
-    else if (!h.panel) launch_col_w<N, CF, false, false>(g, b, init, exit_, h.detect, h.band.rows, a, st);
-    else if constexpr (CF::PANEL) launch_col_w<N, CF, false, true>(g, b, init, exit_, h.detect, h.band.rows, a, st);
+    using CN = std::conditional_t<CF::NT_COL, Near<N>, CF>;
+    auto pick = [&](auto c) {
+      using CS = decltype(c);
+      if (!h.panel) launch_col_w<N, CS, false, false>(g, b, init, exit_, h.detect, h.band.rows, a, st);
+      else if constexpr (CF::PANEL) launch_col_w<N, CS, false, true>(g, b, init, exit_, h.detect, h.band.rows, a, st);
+    };
+    if (lat) launch_col_w<N, Lat<N>, false, false>(g, b, init, exit_, h.detect, h.band.rows, a, st);
+    else if (h.shape == Shape::Near) pick(CN{});
+    else pick(CF{});
   }
   return hipGetLastError();
 }

@@ -9,7 +9,7 @@
 namespace jms {
 template hipError_t launch_row_pass_n<JMS_N>(int, int, float2*, long long, const float2*, long long,
                                              long long, const int*, int, int, const float2*,
-                                             const RowChanHost&, int, bool, const BandHost&, bool, hipStream_t);
+                                             const RowChanHost&, int, bool, const BandHost&, Shape, hipStream_t);
 template hipError_t launch_col_pass_n<JMS_N>(int, bool, bool, const ColArgsHost&, hipStream_t);
 template hipError_t launch_row_pass_grp_n<JMS_N>(int, int, long long, long long, const float2*, const GrpArgs&,
                                                  bool, const BandHost&, hipStream_t);
