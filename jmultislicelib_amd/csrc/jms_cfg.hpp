@@ -80,9 +80,12 @@ struct CfgP {
   // the same for the row pass's line exchanges
   static constexpr int PADSH_ROW = Tuned<N>::PADR > 0 ? Tuned<N>::PADR : PADSH;
   // waves of staged batches stored in panels of 16 columns (see panel_off):
-  // contiguous column tiles, rows in 128-byte segments; where the tuner found
-  // the pair of passes faster that way
-  static constexpr bool PANEL = Tuned<N>::PANEL && (N % 16 == 0);
+  // contiguous column tiles, rows in 128-byte segments; where the pair of
+  // passes was found faster that way.  A length that is no multiple of 16 has a
+  // partly filled last panel: 625 columns, whose rows are not aligned to
+  // 128-byte lines in the natural layout, 2.05 -> 1.65 ms per 2 GiB of waves
+  // and pair (streamed: 2.20 -> 1.68).
+  static constexpr bool PANEL = Tuned<N>::PANEL;
   // minimum waves per SIMD requested from the register allocator for the
   // wave-local column kernel (1 = no constraint; jms_tuned.h).  Eight waves
   // let two 1024-thread blocks share a CU, so one block's FFTs overlap the

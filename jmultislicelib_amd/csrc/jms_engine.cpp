@@ -166,6 +166,7 @@ struct jms_hip_engine {
   float* scratch = nullptr;
   // staged batches keep their waves in 16-column panels (set with the grid)
   bool panel = false;
+  long long wave_items(bool in_panels) const { return in_panels ? jms::panel_stride(nx, ny) : n; }
   // timing
   bool timing = false;
   Timer tm[4];  // row pass, column pass, combine, graph replay
@@ -446,8 +447,9 @@ int enqueue_batch(jms_hip_engine* e, void* waves, float* partial, int nwave, int
   const long long part_w = (long long)e->ndetslc * e->ndet * ntc;
   jms::ColArgsHost ca;
   ca.wave = waves;
+  const long long wst = e->wave_items(panel);
   ca.nx = e->nx;
-  ca.wave_stride = e->n;
+  ca.wave_stride = wst;
   ca.kscx = 1.f / e->a0x;
   ca.kscy = 1.f / e->a0y;
   ca.cppl = e->have_cppl ? e->cppl.as<float>() : nullptr;
@@ -531,7 +533,7 @@ int enqueue_batch(jms_hip_engine* e, void* waves, float* partial, int nwave, int
     // INIT column pass of a part: plane islc0
     auto init = [&](const Part& q) {
       jms::ColArgsHost c = ca;
-      c.wave = (float2*)waves + q.w0 * e->n;
+      c.wave = (float2*)waves + q.w0 * wst;
       c.partial = partial + q.w0 * part_w;
       c.src = (const float2*)src + q.w0 * src_stride;
       c.src_stride = src_stride;
@@ -542,14 +544,14 @@ int enqueue_batch(jms_hip_engine* e, void* waves, float* partial, int nwave, int
     };
     auto row = [&](const Part& q, int j, int js, int mode) {
       TimedLaunch tl(e, 0, timed);
-      return jms::launch_row_pass(e->nx, e->ny, q.nw, (float2*)waves + q.w0 * e->n, e->n, e->pgr.as<float2>(),
+      return jms::launch_row_pass(e->nx, e->ny, q.nw, (float2*)waves + q.w0 * wst, wst, e->pgr.as<float2>(),
                                   e->slcoffset[js], (long long)e->npgx * e->npgy, S > 0 ? var + (long long)q.w0 * S : var,
                                   S, j, e->twx.as<float2>(), rc, mode, panel,
                                   j > islc0 || src_in ? bd : jms::BandHost(), shape, q.st);
     };
     auto col = [&](const Part& q, int j, int js) {
       jms::ColArgsHost c = ca;
-      c.wave = (float2*)waves + q.w0 * e->n;
+      c.wave = (float2*)waves + q.w0 * wst;
       c.partial = partial + q.w0 * part_w;
       c.band = bd;
       c.pro = e->pro.as<float2>() + (long long)e->proidx[js] * e->n;
@@ -623,7 +625,7 @@ int check_ready(jms_hip_engine* e) {
 }
 
 int ensure_batch(jms_hip_engine* e, int nwave) {
-  hipError_t err = e->waves.ensure(sizeof(float) * 2 * (size_t)e->n * nwave);
+  hipError_t err = e->waves.ensure(sizeof(float) * 2 * (size_t)e->wave_items(e->panel) * nwave);
   if (err != hipSuccess) return e->fail(110, "allocate wave batch", err);
   const size_t np = sizeof(float) * (size_t)nwave * std::max(1, e->ndetslc) *
                     std::max(1, e->ndet) * (size_t)std::max(e->ntiles_col(), e->ntiles_col(true));
@@ -1312,8 +1314,10 @@ int jms_hip_run_batch_noalloc(jms_hip_engine* e, int islc0, int nwave, void* wav
   // the small launch shapes need up to twice the tiles: only where those fit too
   const long long need_lat = (long long)nwave * std::max(1, e->ndetslc) * e->ndet * e->ntiles_col(true);
   const bool lat = jms::lat_ok(e->nx, e->ny, nwave) && need_lat <= jms::kScratchFloats;
+  // the caller's waves have n items each: no partly filled panels
+  const bool panel = e->panel && !lat && e->wave_items(true) == e->n;
   return enqueue_batch(e, waves, e->scratch, nwave, islc0, e->wav0.p, 0, ppar, var, npos, npass, weights, res, 0,
-                       BatchChans(), false, lat, true, false, e->panel && !lat);
+                       BatchChans(), false, lat, true, false, panel);
 }
 
 // ---------------------------------------------------------------------------
@@ -1573,7 +1577,7 @@ int jms_hip_group_run(jms_hip_group* g) {
     if (!bd.on() || !b.on() || !e->probe_in(b)) bd.x0 = bd.x1 = 0;
   }
   const char* base = (const char*)g->tab.p;
-  const long long n = (long long)g->nx * g->ny;
+  const long long n = (long long)g->nx * g->ny, wst = lead->wave_items(lead->panel);
   const int ld = g->smax + 1;
   const int ntc = lead->ntiles_col();
   hipError_t err = hipSuccess;
@@ -1601,7 +1605,7 @@ int jms_hip_group_run(jms_hip_group* g) {
       ga.step = s;
       {
         TimedLaunch tl(lead, 0, lead->timing);
-        err = jms::launch_row_pass_grp(g->nx, g->ny, rd.active[s], n, n, lead->twx.as<float2>(), ga, lead->panel, bd,
+        err = jms::launch_row_pass_grp(g->nx, g->ny, rd.active[s], wst, n, lead->twx.as<float2>(), ga, lead->panel, bd,
                                        st);
       }
       if (err == hipSuccess) err = col(s + 1, false, 0, rd.active[s + 1], false);

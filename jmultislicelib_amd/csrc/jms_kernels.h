@@ -209,6 +209,8 @@ hipError_t launch_row_pass(int nx, int ny, int nwave, float2* wave, long long wa
 // 16 columns: element (y, x) at (x / 16) * 16 ny + 16 y + x % 16 (column
 // tiles contiguous); chosen per line length where the passes run faster so
 bool panel_ok(int nx, int ny);
+// items from one panel wave to the next (whole panels)
+inline long long panel_stride(int nx, int ny) { return (long long)((nx + 15) / 16 * 16) * ny; }
 // column transforms only (all columns of nbatch grids)
 hipError_t launch_col_fft(int nx, int ny, int nbatch, float2* data, int dir, const float2* twy,
                           hipStream_t st);

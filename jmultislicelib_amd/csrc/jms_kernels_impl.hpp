@@ -172,7 +172,7 @@ __global__ __launch_bounds__(C_::T * C_::LPB) __attribute__((amdgpu_waves_per_eu
     long long slc_off, long long npg, const int* __restrict__ var_tab, int var_ld, int jslc,
     const float2* __restrict__ twg, RowChan rc, GrpArgs ga, int gx0, int gx1) {
   static_assert(!GRP || MODE == 0, "grouped row passes carry no real-space readout");
-  static_assert(!PANEL || (MODE == 0 && N % kPanel == 0), "panel waves: whole panels, staged batches only");
+  static_assert(!PANEL || MODE == 0, "panel waves: staged batches only");
   static_assert(!BAND || MODE != 2, "the exit-plane readout reads whole rows");
   using P = typename C_::P;
   constexpr int T = C_::T, LPB = C_::LPB;
@@ -1340,7 +1340,7 @@ hipError_t launch_col_pass_grp_n(int nx, int nwave, bool init, bool exit_, bool 
   if (panel && (CF::XL || !CF::PANEL)) return hipErrorInvalidValue;
   ColArgs a{};
   a.nx = nx;
-  a.wave_stride = (long long)N * nx;
+  a.wave_stride = panel ? panel_stride(nx, N) : (long long)N * nx;
   a.part_dstride = part_dstride;
   a.twg = twy;
   a.grp = ga;

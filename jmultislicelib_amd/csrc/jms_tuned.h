@@ -1,5 +1,6 @@
 // jms_tuned.h -- launch shapes per line length chosen by the autotuner
-// (csrc/tune/tune.py) from measured kernel times on MI355X.  Generated:
+// (csrc/tune/tune.py) from measured kernel times on MI355X (some revised by the
+// time of pairs of passes, see REVISED there).  Generated:
 // edit by re-running the tuner.  Fields not given keep the defaults of
 // jms_cfg.hpp: LPB (rows per row-pass block; 0 = default), GTW (row-pass
 // twiddles from the global table with the product tree), CW (columns per
@@ -150,7 +151,7 @@ template <> struct Tuned<320> {
   static constexpr int CW = 16;
   static constexpr int WPE = 1;
   static constexpr int TW = 0;
-  static constexpr int PADC = 0;
+  static constexpr int PADC = 24;
   static constexpr int PADR = 0;
   static constexpr bool PANEL = false;
   static constexpr int TR = 0;
@@ -174,7 +175,7 @@ template <> struct Tuned<384> {
   static constexpr int CW = 16;
   static constexpr int WPE = 1;
   static constexpr int TW = 0;
-  static constexpr int PADC = 0;
+  static constexpr int PADC = 24;
   static constexpr int PADR = 0;
   static constexpr bool PANEL = true;
   static constexpr int TR = 0;
@@ -207,13 +208,13 @@ template <> struct Tuned<512> {
 template <> struct Tuned<625> {
   static constexpr int LPB = 4;
   static constexpr bool GTW = false;
-  static constexpr int CW = 16;
+  static constexpr int CW = 8;
   static constexpr int WPE = 1;
   static constexpr int TW = 0;
-  static constexpr int PADC = 0;
-  static constexpr int PADR = 0;
-  static constexpr bool PANEL = false;
-  static constexpr int TR = 0;
+  static constexpr int PADC = 24;
+  static constexpr int PADR = 24;
+  static constexpr bool PANEL = true;
+  static constexpr int TR = 64;
   static constexpr bool NTC = false;
 };
 template <> struct Tuned<640> {
@@ -222,11 +223,11 @@ template <> struct Tuned<640> {
   static constexpr int CW = 8;
   static constexpr int WPE = 1;
   static constexpr int TW = 0;
-  static constexpr int PADC = 0;
+  static constexpr int PADC = 24;
   static constexpr int PADR = 24;
   static constexpr bool PANEL = true;
   static constexpr int TR = 0;
-  static constexpr bool NTC = true;
+  static constexpr bool NTC = false;
 };
 template <> struct Tuned<720> {
   static constexpr int LPB = 2;
@@ -234,11 +235,11 @@ template <> struct Tuned<720> {
   static constexpr int CW = 8;
   static constexpr int WPE = 1;
   static constexpr int TW = 0;
-  static constexpr int PADC = 0;
+  static constexpr int PADC = 24;
   static constexpr int PADR = 24;
   static constexpr bool PANEL = false;
   static constexpr int TR = 0;
-  static constexpr bool NTC = true;
+  static constexpr bool NTC = false;
 };
 template <> struct Tuned<768> {
   static constexpr int LPB = 2;
@@ -246,11 +247,11 @@ template <> struct Tuned<768> {
   static constexpr int CW = 8;
   static constexpr int WPE = 1;
   static constexpr int TW = 0;
-  static constexpr int PADC = 0;
+  static constexpr int PADC = 24;
   static constexpr int PADR = 0;
   static constexpr bool PANEL = true;
   static constexpr int TR = 0;
-  static constexpr bool NTC = true;
+  static constexpr bool NTC = false;
 };
 template <> struct Tuned<1024> {
   static constexpr int LPB = 2;
