@@ -250,58 +250,99 @@ __device__ __forceinline__ float ff_gmag(float qx, float qy) {
 // grouped by type, ascending atom order inside a type):
 //   pot(q) = sum_t ff_t(q) ap(q) sum_{atoms of t} occ exp(-2 pi i (x qx + y qy))
 // ap(q) = 1/2 - 1/2 tanh(30 (|q|/kmax - 0.9)) with the potential band limit,
-// else 1 (JEElaSca.cpp:592-595).  The atoms pass through LDS 256 at a time;
-// every thread walks the same list, so the type switches are uniform.
-// grid: (ceil(nx*ny/256), nvar), block: 256
+// else 1 (JEElaSca.cpp:592-595).  The phase factor is one of x times one of y,
+// so the sum over the atoms of a type is a product of two thin matrices: a
+// block of (16 P)^2 pixels takes kFFChunk atoms at a time, computes their
+// factors once per column and row (the phase in turns in double, reduced, sine
+// and cosine in double, rounded: the product is then no further from exact
+// than one float sine and cosine of the whole phase) and adds outer products,
+// P x P pixels a thread from 2 P values in LDS.  Bound by the float FMAs (four
+// per atom and pixel) where one sine and cosine per atom and pixel was: 8
+// variants of 512^2, 160 atoms each, 364 -> 99 us on MI355X (34 of them the FMAs
+// at 80 TFLOP/s; the rest mostly the double sines and cosines of the factors).
+// Every thread walks the same list, so the type switches are uniform.
+// grid: (ceil(nx / 16 P), ceil(ny / 16 P), nvar), block: 256
+constexpr int kFFChunk = 32;
+template <int P>
 __global__ __launch_bounds__(256) void k_ff_sum(float2* __restrict__ out, const float2* __restrict__ ff,
                                                 const FFAtom* __restrict__ atoms, const int* __restrict__ off,
                                                 int nx, int ny, float itogx, float itogy, float kmax,
                                                 int bwl_pot) {
-  __shared__ FFAtom s_at[256];
+  constexpr int TILE = 16 * P;
+  __shared__ float2 s_x[kFFChunk][TILE], s_y[kFFChunk][TILE];
+  __shared__ int s_type[kFFChunk];
   const long long n = (long long)nx * ny;
-  const int v = blockIdx.y;
-  const long long p = (long long)blockIdx.x * 256 + threadIdx.x;
-  const bool valid = p < n;
-  const int ix = valid ? (int)(p % nx) : 0, iy = valid ? (int)(p / nx) : 0;
-  const float qx = ff_freq(ix, nx, itogx), qy = ff_freq(iy, ny, itogy);
-  float ap = 1.f;
-  if (bwl_pot) ap = 0.5f - 0.5f * tanhf((ff_gmag(qx, qy) / kmax - 0.9f) * 30.f);
-  const int a0 = off[v], a1 = off[v + 1];
-  float2 pot = make_float2(0.f, 0.f), s = make_float2(0.f, 0.f);
-  int cur = -1;  // type of the running sum s
-  for (int c0 = a0; c0 < a1; c0 += 256) {
-    const int m = (a1 - c0 < 256) ? (a1 - c0) : 256;
+  const int v = blockIdx.z, tx = threadIdx.x % 16, ty = threadIdx.x / 16;
+  const int x0 = blockIdx.x * TILE, y0 = blockIdx.y * TILE;
+  float2 pot[P][P], s[P][P];
+#pragma unroll
+  for (int j = 0; j < P; ++j)
+#pragma unroll
+    for (int i = 0; i < P; ++i) pot[j][i] = s[j][i] = make_float2(0.f, 0.f);
+  int cur = -1;  // type of the running sums s
+  auto flush = [&]() {
+#pragma unroll
+    for (int j = 0; j < P; ++j)
+#pragma unroll
+      for (int i = 0; i < P; ++i) {
+        const int x = x0 + tx + 16 * i, y = y0 + ty + 16 * j;
+        if (x < nx && y < ny) {
+          float ap = 1.f;
+          if (bwl_pot)
+            ap = 0.5f - 0.5f * tanhf((ff_gmag(ff_freq(x, nx, itogx), ff_freq(y, ny, itogy)) / kmax - 0.9f) * 30.f);
+          const float2 f = ff[(long long)cur * n + (long long)y * nx + x], z = s[j][i];
+          pot[j][i].x += ap * (f.x * z.x - f.y * z.y);
+          pot[j][i].y += ap * (f.x * z.y + f.y * z.x);
+        }
+        s[j][i] = make_float2(0.f, 0.f);
+      }
+  };
+  const int a1 = off[v + 1];
+  for (int c0 = off[v]; c0 < a1; c0 += kFFChunk) {
+    const int m = (a1 - c0 < kFFChunk) ? (a1 - c0) : kFFChunk;
     __syncthreads();  // the previous chunk's reads are done
-    if ((int)threadIdx.x < m) s_at[threadIdx.x] = atoms[c0 + threadIdx.x];
+    for (int e = threadIdx.x; e < m * 2 * TILE; e += 256) {
+      const int k = e / (2 * TILE), r = e % (2 * TILE), c = r % TILE;
+      const FFAtom at = atoms[c0 + k];
+      const bool isx = r < TILE;
+      const float q = isx ? ff_freq(min(x0 + c, nx - 1), nx, itogx) : ff_freq(min(y0 + c, ny - 1), ny, itogy);
+      double ud = (double)(isx ? at.x : at.y) * (double)q;
+      ud -= rint(ud);
+      double sn, cs;
+      sincospi(2.0 * ud, &sn, &cs);
+      const double o = isx ? 1.0 : (double)at.occ;
+      (isx ? s_x : s_y)[k][c] = make_float2((float)(o * cs), (float)(-o * sn));
+    }
+    if ((int)threadIdx.x < m) s_type[threadIdx.x] = atoms[c0 + threadIdx.x].type;
     __syncthreads();
     for (int k = 0; k < m; ++k) {
-      const FFAtom at = s_at[k];
-      if (at.type != cur) {
-        if (cur >= 0 && valid) {
-          const float2 f = ff[(long long)cur * n + p];
-          pot.x += ap * (f.x * s.x - f.y * s.y);
-          pot.y += ap * (f.x * s.y + f.y * s.x);
-        }
-        s = make_float2(0.f, 0.f);
-        cur = at.type;
+      if (s_type[k] != cur) {
+        if (cur >= 0) flush();
+        cur = s_type[k];
       }
-      // phase in turns, formed in double (x q reaches ~100 turns) and
-      // reduced before the float sine and cosine
-      double ud = (double)at.x * (double)qx + (double)at.y * (double)qy;
-      ud -= rint(ud);
-      float sn, cs;
-      sincospif(2.f * (float)ud, &sn, &cs);
-      s.x += at.occ * cs;
-      s.y -= at.occ * sn;
+      float2 ex[P], ey[P];
+#pragma unroll
+      for (int i = 0; i < P; ++i) {
+        ex[i] = s_x[k][tx + 16 * i];
+        ey[i] = s_y[k][ty + 16 * i];
+      }
+#pragma unroll
+      for (int j = 0; j < P; ++j)
+#pragma unroll
+        for (int i = 0; i < P; ++i) {
+          s[j][i].x = fmaf(ey[j].x, ex[i].x, fmaf(-ey[j].y, ex[i].y, s[j][i].x));
+          s[j][i].y = fmaf(ey[j].x, ex[i].y, fmaf(ey[j].y, ex[i].x, s[j][i].y));
+        }
     }
   }
-  if (!valid) return;
-  if (cur >= 0) {
-    const float2 f = ff[(long long)cur * n + p];
-    pot.x += ap * (f.x * s.x - f.y * s.y);
-    pot.y += ap * (f.x * s.y + f.y * s.x);
-  }
-  out[(long long)v * n + p] = pot;
+  if (cur >= 0) flush();
+#pragma unroll
+  for (int j = 0; j < P; ++j)
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+      const int x = x0 + tx + 16 * i, y = y0 + ty + 16 * j;
+      if (x < nx && y < ny) out[(long long)v * n + (long long)y * nx + x] = pot[j][i];
+    }
 }
 
 // a <- exp(i sg sc a): real-space potential (complex: the imaginary part
@@ -592,8 +633,13 @@ hipError_t launch_ff_gratings(float2* out, int nx, int ny, int nvar, const float
                               float sg, int bwl_pgr, float kthr, float ftrn, const float2* twx,
                               const float2* twy, hipStream_t st) {
   const long long n = (long long)nx * ny, total = n * nvar;
-  hipLaunchKernelGGL(k_ff_sum, dim3((unsigned)((n + 255) / 256), nvar), dim3(256), 0, st, out, ff, atoms, off, nx,
-                     ny, itogx, itogy, kmax, bwl_pot);
+  // tiles of 64 x 64 pixels where they give every CU two blocks, else of 32 x 32
+  auto sum = [&](auto kern, int tile) {
+    hipLaunchKernelGGL(kern, dim3((nx + tile - 1) / tile, (ny + tile - 1) / tile, nvar), dim3(256), 0, st, out, ff,
+                       atoms, off, nx, ny, itogx, itogy, kmax, bwl_pot);
+  };
+  if ((long long)((nx + 63) / 64) * ((ny + 63) / 64) * nvar >= 512) sum(k_ff_sum<4>, 64);
+  else sum(k_ff_sum<2>, 32);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) e = launch_fft2d(nx, ny, nvar, out, +1, twx, twy, st);
   if (e != hipSuccess) return e;
