@@ -158,8 +158,8 @@ struct jms_hip_engine {
   // addresses of every buffer the batch reads or writes (graph_bufs): when
   // any of them moves, all graphs are dropped before the next capture.
   bool use_graph = false;
-  // (a batch that goes in two halves: one graph for each, the second for `side`)
-  std::map<std::array<int, 4>, std::array<hipGraphExec_t, 2>> graphs;
+  // (one graph for each part of a batch that goes in several; see split_of)
+  std::map<std::array<int, 4>, std::vector<hipGraphExec_t>> graphs;
   std::array<const void*, 17> graph_bufs{};
   std::array<int, 12> graph_band{};  // and to the band the launches were made for
   // this device's scratch of the allocation-free batch entry (resolved at create)
@@ -188,8 +188,7 @@ struct jms_hip_engine {
   }
   void drop_graphs() {
     for (auto& kv : graphs)
-      for (hipGraphExec_t g : kv.second)
-        if (g) (void)hipGraphExecDestroy(g);
+      for (hipGraphExec_t g : kv.second) (void)hipGraphExecDestroy(g);
     graphs.clear();
   }
   // device addresses a captured batch depends on
@@ -358,6 +357,7 @@ constexpr long long kNearBytes = 184LL << 20, kNearWave = 8LL << 20, kTwoBytes =
 struct Split {
   int rounds = 1;
   bool near = false, two = false;
+  int parts() const { return rounds * (two ? 2 : 1); }
 };
 Split split_of(const jms_hip_engine* e, int nwave, const jms::BandHost& bd, bool lat, bool chans) {
   Split s;
@@ -429,13 +429,13 @@ int enqueue_combine(jms_hip_engine* e, float* partial, int nwave, int islc0, int
 // probe, else the single-wave path's wave; `keep`: leave psi(k) of the exit
 // plane in the waves (batches only read the sums).  The band's columns are
 // left out from the first slice on, and before it where the source is zero
-// there.  `mirror` (or nullptr): host memory that gets the results too.  `half`
-// 0 or 1: only the passes of the first or second halves of a batch that goes in
-// two (split_of), on the engine's stream, without the combination.
+// there.  `mirror` (or nullptr): host memory that gets the results too.  `part`
+// (or -1): only the passes of this part of a batch that goes in several
+// (split_of), on the engine's stream, without the combination.
 int enqueue_batch(jms_hip_engine* e, void* waves, float* partial, int nwave, int islc0, const void* src,
                   long long src_stride, const void* ppar, const int* var, int npos, int npass,
                   const float* weights, float* res, int accumulate, const BatchChans& ch, bool timed,
-                  bool lat, bool src_same, bool keep, bool panel, float* mirror = nullptr, int half = -1) {
+                  bool lat, bool src_same, bool keep, bool panel, float* mirror = nullptr, int part = -1) {
   const jms::BandHost bd = e->band(lat);
   const bool src_in = e->holds(src_same ? e->wav0_gap : e->wav_gap, bd);
   // panel waves (staged batches): integrated readouts only, the waves are internal
@@ -520,11 +520,11 @@ int enqueue_batch(jms_hip_engine* e, void* waves, float* partial, int nwave, int
   } else {
     const Split sp = split_of(e, nwave, bd, lat, ch.any());
     // one stream where each launch is timed
-    const bool two = half >= 0 || (sp.two && !timed && e->side);
-    const int parts = sp.rounds * (two ? 2 : 1);
+    const bool two = sp.two && (part >= 0 || (!timed && e->side));
+    const int parts = two ? sp.parts() : sp.rounds;
     const jms::Shape shape = lat ? jms::Shape::Small : sp.near ? jms::Shape::Near : jms::Shape::Stream;
     ca.shape = shape;
-    SideBranch branch(e, two && half < 0);
+    SideBranch branch(e, two && part < 0);
     if (branch.err != hipSuccess) return e->fail(129, "second stream", branch.err);
     struct Part {
       int w0, nw;
@@ -562,11 +562,12 @@ int enqueue_batch(jms_hip_engine* e, void* waves, float* partial, int nwave, int
     for (int r = 0; r < sp.rounds; ++r) {
       std::vector<Part> pt;
       for (int h = 0; h < (two ? 2 : 1); ++h) {
-        if (half >= 0 && h != half) continue;
         const int p = r * (two ? 2 : 1) + h;
+        if (part >= 0 && p != part) continue;
         const int w0 = (int)((long long)nwave * p / parts), w1 = (int)((long long)nwave * (p + 1) / parts);
-        pt.push_back({w0, w1 - w0, h && half < 0 ? e->side : e->st});
+        pt.push_back({w0, w1 - w0, h && part < 0 ? e->side : e->st});
       }
+      if (pt.empty()) continue;
       plane_setup(islc0);
       for (const Part& q : pt)
         if ((err = init(q)) != hipSuccess) return e->fail(130, "column pass (init)", err);
@@ -585,7 +586,7 @@ int enqueue_batch(jms_hip_engine* e, void* waves, float* partial, int nwave, int
     }
     if ((err = branch.join()) != hipSuccess) return e->fail(129, "second stream", err);
   }
-  if (half >= 0) return 0;
+  if (part >= 0) return 0;
   return enqueue_combine(e, partial, nwave, islc0, ntc, npos, npass, weights, res, accumulate, timed, mirror);
 }
 
@@ -1239,40 +1240,44 @@ int jms_hip_run_staged(jms_hip_engine* e, int pos0, int npos, int islc0) {
       const std::array<int, 4> key{nw, islc0, np, npass};
       auto it = e->graphs.find(key);
       const int ntc = e->ntiles_col(lat);
-      const bool two = !use_loop(e, nw, islc0) && split_of(e, nw, b0, lat, false).two;
+      const Split sp = use_loop(e, nw, islc0) ? Split() : split_of(e, nw, b0, lat, false);
+      const int parts = sp.parts();
       if (it == e->graphs.end()) {
-        std::array<hipGraphExec_t, 2> ge{};
-        for (int h = 0; h < (two ? 2 : 1); ++h) {
-          hipGraph_t g = nullptr;
+        std::vector<hipGraphExec_t> ge;
+        for (int q = 0; q < parts && !rc; ++q) {
+          hipGraph_t gr = nullptr;
+          hipGraphExec_t x = nullptr;
           err = hipStreamBeginCapture(e->st, hipStreamCaptureModeThreadLocal);
-          if (err != hipSuccess) rc = e->fail(121, "begin capture", err);
-          else {
-            rc = enqueue_batch(e, e->waves.p, e->partial.as<float>(), nw, islc0, e->wav0.p, 0, e->cur_ppar.p,
-                               e->cur_var.as<int>(), np, npass, e->s_weights.as<float>(), e->cur_res.as<float>(), 0,
-                               BatchChans(), false, lat, true, false, panel, nullptr, two ? h : -1);
-            err = hipStreamEndCapture(e->st, &g);
-            if (!rc && err != hipSuccess) rc = e->fail(122, "end capture", err);
+          if (err != hipSuccess) {
+            rc = e->fail(121, "begin capture", err);
+            break;
           }
+          rc = enqueue_batch(e, e->waves.p, e->partial.as<float>(), nw, islc0, e->wav0.p, 0, e->cur_ppar.p,
+                             e->cur_var.as<int>(), np, npass, e->s_weights.as<float>(), e->cur_res.as<float>(), 0,
+                             BatchChans(), false, lat, true, false, panel, nullptr, parts > 1 ? q : -1);
+          err = hipStreamEndCapture(e->st, &gr);
+          if (!rc && err != hipSuccess) rc = e->fail(122, "end capture", err);
           if (!rc) {
-            err = hipGraphInstantiate(&ge[h], g, nullptr, nullptr, 0);
+            err = hipGraphInstantiate(&x, gr, nullptr, nullptr, 0);
             if (err != hipSuccess) rc = e->fail(123, "instantiate graph", err);
+            else ge.push_back(x);
           }
-          if (g) (void)hipGraphDestroy(g);
-          if (rc) {
-            if (ge[0]) (void)hipGraphExecDestroy(ge[0]);
-            return rc;
-          }
+          if (gr) (void)hipGraphDestroy(gr);
+        }
+        if (rc) {
+          for (hipGraphExec_t x : ge) (void)hipGraphExecDestroy(x);
+          return rc;
         }
         it = e->graphs.emplace(key, ge).first;
       }
       {
         TimedLaunch tl(e, 3, e->timing);  // one replay = the batch's whole launch sequence
-        SideBranch branch(e, two);
+        SideBranch branch(e, sp.two);
         err = branch.err;
-        if (err == hipSuccess) err = hipGraphLaunch(it->second[0], e->st);
-        if (err == hipSuccess && two) err = hipGraphLaunch(it->second[1], e->side);
+        for (int q = 0; q < parts && err == hipSuccess; ++q)
+          err = hipGraphLaunch(it->second[q], sp.two && q % 2 ? e->side : e->st);
         if (err == hipSuccess) err = branch.join();
-        if (err == hipSuccess && two)
+        if (err == hipSuccess && parts > 1)
           rc = enqueue_combine(e, e->partial.as<float>(), nw, islc0, ntc, np, npass, e->s_weights.as<float>(),
                                e->cur_res.as<float>(), 0, false, nullptr);
         if (rc) return rc;
