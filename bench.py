@@ -15,13 +15,17 @@ graph (the batch's whole launch sequence; --no-graph: eager launches), with
 HIP events around every replay.  A second pass over the same steps with eager
 launches and HIP events around every kernel launch (on the engine's stream)
 gives the per-kernel durations behind `roofline`: the dominant kernel's
-algorithmic bytes per launch (16 n per wave: one read and one write of the
-complex64 wave; 8 n for the initial column pass, which reads the shared
-probe) over its average launch duration, against MI355X's 8 TB/s HBM peak.
-Its `traffic` is the HBM bytes per launch measured with rocprofv3
-FETCH_SIZE / WRITE_SIZE (scaled by a plain copy of known size) and committed
-in profiles/hbm_traffic_stem_scan_512.md, per wave times the waves per
-launch.  `fft_rate` is 10 n log2 n flops per probe pass and slice over the
+algorithmic bytes per launch (16 n f per wave: one read and one write of the
+complex64 wave, of which the fraction f of column tiles inside the
+propagators' band limit is stored; 8 n f for the initial column pass, which
+reads the shared probe) over its average launch duration, against MI355X's 8
+TB/s HBM peak (the waves of a part come from the Infinity Cache, so this is a
+rate of the memory system, not of HBM alone).  Its `traffic` is the bytes per
+launch beyond the L2 caches measured with rocprofv3 FETCH_SIZE / WRITE_SIZE
+(scaled by a plain copy of known size) and committed in
+profiles/hbm_traffic_stem_scan_512.md, per wave times the waves per launch.
+The eager pass runs each part's halves one after the other, the replay side
+by side.  `fft_rate` is 10 n log2 n flops per probe pass and slice over the
 timed region against the FP32 vector peak.  Outside the timed region,
 `accuracy` compares a subset of the scan (8 positions x 8 passes) with the
 CPU oracle's float32 run and its FP64 twin, detector by detector, and
@@ -63,6 +67,16 @@ def measured_traffic_per_wave(kernel):
         return None
     m = re.search(r"traffic_bytes_per_wave\[" + re.escape(kernel) + r"\]\s*=\s*([0-9.]+)", txt)
     return float(m.group(1)) if m else None
+
+
+def stored_fraction(sp) -> float:
+    """Part of a wave that the slice loop keeps between its passes: the
+    16-column tiles that reach into the band of some propagator."""
+    live = np.zeros(sp.nx, bool)
+    for p in sp.propagators:
+        live |= (np.asarray(p) != 0).any(axis=0)
+    starts = range(0, sp.nx, 16)
+    return sum(min(16, sp.nx - x) for x in starts if live[x:x + 16].any()) / sp.nx
 
 
 def cpu_model() -> str:
@@ -163,7 +177,8 @@ def run_thick2048(args):
         log(f"kernel {kinds[k]}: {cnt} launches, {ms:.1f} ms total, {ms / max(cnt, 1):.3f} ms avg")
     n = sp.nx * sp.ny
     positions = args.steps * npos
-    slice_bytes = 32.0 * n * positions * len(sp.objslc)
+    frac = stored_fraction(sp)
+    slice_bytes = 32.0 * n * frac * positions * len(sp.objslc)
     # the plane wave of each batch (single-wave path)
     pw = np.zeros((sp.ny, sp.nx), np.complex64)
     pw[0, 0] = 1.0
@@ -179,7 +194,7 @@ def run_thick2048(args):
     dom = max((0, 1), key=lambda k: tm[k][0])
     ms, cnt = tm[dom]
     waves_per_launch = npos
-    achieved = 16.0 * n * waves_per_launch / (ms / cnt * 1e-3) / 1e9
+    achieved = 16.0 * n * frac * waves_per_launch / (ms / cnt * 1e-3) / 1e9
     out = {"metric": "STEM probe-positions/s at 2048^2 x 1000 distinct slices (large thick specimen)",
            "value": round(positions / wall, 3), "unit": "positions/s", "n_gpus": 1, "steps": args.steps,
            "warmup": 0, "ms_per_step": round(wall / args.steps * 1e3, 1), "higher_is_better": True,
@@ -225,7 +240,8 @@ def run_jobs64(args):
         for e in sorted(set(j.setup.nx for j in jobs)):
             groups.append(Group([eng for eng, j in zip(engines, jobs) if j.setup.nx == e]))
     positions = sum(len(j.dx) for j in jobs)
-    work = sum(len(j.dx) * len(j.setup.objslc) * 32.0 * j.setup.nx * j.setup.ny for j in jobs)
+    work = sum(len(j.dx) * len(j.setup.objslc) * 32.0 * j.setup.nx * j.setup.ny * stored_fraction(j.setup)
+               for j in jobs)
     log(f"setup {time.perf_counter() - t0:.1f} s: {len(jobs)} jobs, {positions} positions, "
         f"edges {sorted(set(j.setup.nx for j in jobs))}, slices {min(len(j.setup.objslc) for j in jobs)}-"
         f"{max(len(j.setup.objslc) for j in jobs)}")
@@ -264,7 +280,8 @@ def run_jobs64(args):
                       "jobs": len(jobs), "positions_per_step": positions, "grouped": grouped},
            "roofline": {"bound": "hbm", "achieved": round(rate, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                         "frac": round(rate / HBM_PEAK_GBS, 4), "traffic": None,
-                        "kernel": "whole slice loop over all jobs (32 n bytes per position and slice)"},
+                        "kernel": "whole slice loop over all jobs (32 n bytes per position and slice, of the stored part of "
+                                  "a wave)"},
            "cpu_baseline": None}
     for g in groups:
         g.close()
@@ -430,10 +447,11 @@ def run_stem512(args):
     dom = max((0, 1), key=lambda k: tm[k][0])
     ms, cnt = tm[dom]
     passes = positions * npass
-    if dom == 0:  # S row passes per wave, 16 n bytes each
-        total_bytes = 16.0 * n * passes * S
-    else:  # S column passes of 16 n bytes plus the initial one: probe read shared, 8 n written
-        total_bytes = (16.0 * n * S + 8.0 * n) * passes
+    nf = n * stored_fraction(sp)
+    if dom == 0:  # S row passes per wave, 16 n bytes of its stored part each
+        total_bytes = 16.0 * nf * passes * S
+    else:  # S column passes plus the initial one: probe read shared, 8 n written
+        total_bytes = (16.0 * nf * S + 8.0 * nf) * passes
     bytes_per_launch = total_bytes / max(cnt, 1)
     achieved = bytes_per_launch / (ms / cnt * 1e-3) / 1e9
     nwave_avg = passes * (S + (1 if dom == 1 else 0)) / max(cnt, 1)
@@ -447,8 +465,8 @@ def run_stem512(args):
             "timing": "HIP events on the engine stream around every eager launch"}
     total_kernel_ms = sum(v[0] for v in tm.values())
     log(f"kernel time {total_kernel_ms / 1e3:.2f} s of {wall_eager:.2f} s wall (eager pass)")
-    # whole-slice view: 32 n bytes per probe pass per slice
-    slice_bytes = 32.0 * n * passes * S
+    # whole-slice view: 32 n bytes of the stored part per probe pass per slice
+    slice_bytes = 32.0 * nf * passes * S
     flops = 10.0 * n * np.log2(n) * passes * S  # two 2-D FFTs of 5 n log2 n per probe pass and slice
     log(f"scan: {positions} positions in {wall:.2f} s -> {value:.1f} positions/s; "
         f"slice-loop HBM rate {slice_bytes / wall / 1e9:.0f} GB/s ({slice_bytes / wall / 1e9 / HBM_PEAK_GBS:.1%} of peak); "
