@@ -127,7 +127,8 @@ struct jms_hip_engine {
   // detection
   int ndetslc = 0, ndet = 0, detflags = 0;
   std::vector<int> det_objslc;
-  DevBuf detw, detw_t;
+  DevBuf detw, detw_t, det_cols;
+  std::vector<unsigned> det_cols_h;  // bit d of entry x: detector d has a weight in column x
   std::vector<char> det_inf;  // detectors with weights that are not finite
   // incident wave
   DevBuf wav0, cppl, cppl_t;
@@ -160,7 +161,7 @@ struct jms_hip_engine {
   bool use_graph = false;
   // (one graph for each part of a batch that goes in several; see split_of)
   std::map<std::array<int, 4>, std::vector<hipGraphExec_t>> graphs;
-  std::array<const void*, 17> graph_bufs{};
+  std::array<const void*, 18> graph_bufs{};
   std::array<int, 12> graph_band{};  // and to the band the launches were made for
   // this device's scratch of the allocation-free batch entry (resolved at create)
   float* scratch = nullptr;
@@ -192,9 +193,9 @@ struct jms_hip_engine {
     graphs.clear();
   }
   // device addresses a captured batch depends on
-  std::array<const void*, 17> batch_buffers() const {
+  std::array<const void*, 18> batch_buffers() const {
     return {waves.p, partial.p, cur_ppar.p, cur_var.p, cur_res.p, s_weights.p, wav0.p, pgr.p,
-            pro.p, pro_t.p, detw.p, detw_t.p, twx.p, twy.p, cppl.p, cppl_t.p, loop_tab.p};
+            pro.p, pro_t.p, detw.p, detw_t.p, det_cols.p, twx.p, twy.p, cppl.p, cppl_t.p, loop_tab.p};
   }
   int ntiles_col(bool lat = false) const { return jms::col_tiles(ny, nx, lat); }
   // The columns and rows that the waves leave out: where the propagators of
@@ -455,6 +456,7 @@ int enqueue_batch(jms_hip_engine* e, void* waves, float* partial, int nwave, int
   ca.cppl = e->have_cppl ? e->cppl.as<float>() : nullptr;
   ca.cppl_t = e->have_cppl ? e->cppl_t.as<float>() : nullptr;
   ca.detw_t = e->detw_t.as<float>();
+  ca.det_cols = e->det_cols.as<unsigned>();
   ca.ndet = (e->detflags & JMS_HIP_DETECT_INTEGRATED) ? e->ndet : 0;
   ca.detw = e->detw.as<float>();
   ca.partial = partial;
@@ -686,7 +688,7 @@ void jms_hip_destroy(jms_hip_engine* e) {
   e->groups.clear();
   e->drop_graphs();
   for (auto ev : e->ev_pool) (void)hipEventDestroy(ev);
-  DevBuf* bufs[] = {&e->twx, &e->twy, &e->pgr, &e->pro, &e->pro_t, &e->loop_tab, &e->detw, &e->detw_t, &e->wav0,
+  DevBuf* bufs[] = {&e->twx, &e->twy, &e->pgr, &e->pro, &e->pro_t, &e->loop_tab, &e->detw, &e->detw_t, &e->det_cols, &e->wav0,
                     &e->cppl, &e->cppl_t,
                     &e->s_ppar, &e->s_weights, &e->s_var, &e->s_res, &e->waves, &e->partial,
                     &e->cur_var, &e->cur_ppar, &e->cur_res, &e->wav, &e->in1, &e->res1,
@@ -729,6 +731,11 @@ int jms_hip_set_grid(jms_hip_engine* e, int nx, int ny, float a0x, float a0y, fl
   err = e->twy.ensure(tw.size() * sizeof(float));
   if (err == hipSuccess) err = hipMemcpy(e->twy.p, tw.data(), tw.size() * sizeof(float), hipMemcpyHostToDevice);
   if (err != hipSuccess) return e->fail(102, "twiddles y", err);
+  e->det_cols_h.assign(nx, ~0u);  // until the detection is set up for this grid
+  err = e->det_cols.ensure(sizeof(unsigned) * (size_t)nx);
+  if (err == hipSuccess)
+    err = hipMemcpy(e->det_cols.p, e->det_cols_h.data(), sizeof(unsigned) * (size_t)nx, hipMemcpyHostToDevice);
+  if (err != hipSuccess) return e->fail(102, "detector columns", err);
   return 0;
 }
 
@@ -1003,6 +1010,8 @@ int jms_hip_setup_detection(jms_hip_engine* e, int ndetslc, const int* det_objsl
     if (err == hipSuccess) err = hipMemset(e->detw.p, 0, sizeof(float) * (size_t)ndet * e->n);
     if (err == hipSuccess) err = e->detw_t.ensure(sizeof(float) * (size_t)ndet * e->n);
     if (err == hipSuccess) err = hipMemset(e->detw_t.p, 0, sizeof(float) * (size_t)ndet * e->n);
+    e->det_cols_h.assign(e->nx, 0u);
+    if (err == hipSuccess) err = hipMemset(e->det_cols.p, 0, sizeof(unsigned) * (size_t)e->nx);
     if (err != hipSuccess) return e->fail(103, "allocate detector functions", err);
   }
   refresh_loop(e);
@@ -1037,6 +1046,14 @@ int jms_hip_upload_detector(jms_hip_engine* e, int idet, const float* det, int m
   hipError_t err = hipMemcpy(e->detw.as<float>() + (long long)idet * e->n, wgt.data(), nb, hipMemcpyHostToDevice);
   if (err == hipSuccess)
     err = hipMemcpy(e->detw_t.as<float>() + (long long)idet * e->n, wt.data(), nb, hipMemcpyHostToDevice);
+  if (idet < 32)
+    for (int x = 0; x < e->nx; ++x) {
+      const float* col = wt.data() + (size_t)x * e->ny;
+      const bool any = std::any_of(col, col + e->ny, [](float v) { return !(v == 0.f); });
+      e->det_cols_h[x] = (e->det_cols_h[x] & ~(1u << idet)) | (any ? 1u << idet : 0u);
+    }
+  if (err == hipSuccess)
+    err = hipMemcpy(e->det_cols.p, e->det_cols_h.data(), sizeof(unsigned) * (size_t)e->nx, hipMemcpyHostToDevice);
   if (err != hipSuccess) return e->fail(104, "upload detector", err);
   return 0;
 }
@@ -1438,6 +1455,7 @@ int group_build(jms_hip_group* g, std::vector<char>& host) {
       jb.partial = e->partial.as<float>();
       jb.pgr = e->pgr.p;
       jb.detw_t = e->detw_t.as<float>();
+      jb.det_cols = e->det_cols.as<unsigned>();
       jb.cppl_t = e->have_cppl ? e->cppl_t.as<float>() : nullptr;
       jb.detw = e->detw.as<float>();
       jb.cppl = e->have_cppl ? e->cppl.as<float>() : nullptr;

@@ -56,6 +56,7 @@ struct ColArgsHost {
   // column-major ([x][y]) copies for the wave-local column kernel
   const void* pro_t = nullptr;   // propagator of this slice (float2)
   const float* detw_t = nullptr; // [ndet][nx][ny] detector weights
+  const unsigned* det_cols = nullptr;  // [nx]: bit d set where detector d has a weight in the column
   const float* cppl_t = nullptr; // constant phase plate or nullptr
   bool panel = false;            // the waves are in 16-column panels (panel_ok)
   BandHost band;                 // columns and rows left out
@@ -118,6 +119,7 @@ struct GrpJob {
   float* partial = nullptr;       // readout partial sums [wave][plane][detector][tile]
   const void* pgr = nullptr;      // phase gratings (float2)
   const float* detw_t = nullptr;  // [ndet][nx][ny] detector weights
+  const unsigned* det_cols = nullptr;  // [nx], see ColArgsHost
   const float* cppl_t = nullptr;  // constant phase plate [x][y] or nullptr
   const float* detw = nullptr;    // the same row-major [ndet][ny][nx] (long-column kernel)
   const float* cppl = nullptr;    // the same row-major [y][x] or nullptr

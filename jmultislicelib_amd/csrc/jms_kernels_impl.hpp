@@ -385,6 +385,7 @@ struct ColArgs {
   // column-major copies used by the wave-local column kernel: [x][y]
   const float2* pro_t;      // propagator of this slice
   const float* detw_t;      // [ndet][nx][ny] detector weights
+  const unsigned* det_cols; // [nx]: bit d set where detector d has a weight in the column
   const float* cppl_t;      // constant phase plate
   GrpArgs grp;              // grouped launch: wave map and job / plane tables
   // band-limited waves: tiles [tg0, tg0 + tgn) hold only columns where every
@@ -483,6 +484,12 @@ __device__ __forceinline__ void col_body(const ColArgs& a, long long w, float2* 
   const int nx = a.nx;
   const long long n = (long long)N * nx;
   const long long colb = (long long)(valid ? x : x - c) * N;  // column-major offset
+  // the detectors with a weight in this (de-scanned) column: small ones have
+  // none in most columns, and each detector's weights are one more round of
+  // dependent loads (625^2, 32 waves, three ring detectors: 118 -> 108 us for
+  // the launch of a detection plane, 75 without one)
+  [[maybe_unused]] unsigned dets = 0;
+  if (DET && a.detect && valid && a.ndet > 0) dets = a.det_cols[wrap_sub(x, a.dsx, nx)];
   float2 v[NREG];
   if constexpr (INIT) {
     float dx = 0.f, dy = 0.f, fz = 0.f;
@@ -566,6 +573,7 @@ __device__ __forceinline__ void col_body(const ColArgs& a, long long w, float2* 
       // with det(i - d)
       const long long colbs = (long long)wrap_sub(x, a.dsx, nx) * N;
       for (int d = 0; d < a.ndet && d < kMaxDet; ++d) {  // uniform loop over detectors
+        if (!(dets >> d & 1u)) continue;
         const float* dw = a.detw_t + d * n + colbs;
         float wt[NREG];
         static_for<0, M1::NB>([&](auto I) {  // all weight loads of this detector first
@@ -692,6 +700,7 @@ __global__ __launch_bounds__(C_::TW * C_::CW) __attribute__((amdgpu_waves_per_eu
     a.cppl_t = jb.cppl_t;
     a.ndet = jb.ndet;
     a.detw_t = jb.detw_t;
+    a.det_cols = jb.det_cols;
     a.partial = jb.partial;
     a.part_wstride = jb.part_wstride;
     const long long po = pl[a0.grp.step].part_off;
@@ -1300,6 +1309,7 @@ hipError_t launch_col_pass_n(int nwave, bool init, bool exit_, const ColArgsHost
   a.twg = (const float2*)h.twy;
   a.pro_t = (const float2*)h.pro_t;
   a.detw_t = h.detw_t;
+  a.det_cols = h.det_cols;
   a.cppl_t = h.cppl_t;
   using CF = Cfg<N>;
   static_assert(CF::XL || CF::WL, "every line length has a column kernel");

@@ -3,15 +3,13 @@ multiple of 16): staged and grouped batches keep whole panels in their own
 buffers, the allocation-free entry works in the caller's, one grid a wave, and
 must leave what lies behind it alone.  All compute the same sums (1e-6 of the
 largest value: instantiations may contract products differently)."""
-import ctypes as C
-
 import numpy as np
 import pytest
-import torch
 
 from jmultislicelib_amd import Engine, Group, configs
 
 from helpers import random_setup
+from test_zz_no_alloc import _Hip
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-6
@@ -38,17 +36,19 @@ def test_partly_filled_panels(nx, ny):
     grp.close()
     ppar = np.zeros((nwave, 4), np.float32)
     ppar[:, 0], ppar[:, 1] = dx, dy
-    dev = [torch.from_numpy(a).cuda() for a in (ppar, np.asarray(var, np.int32), w)]
-    waves = torch.full((2 * nx * ny * nwave + 64 * ny,), 7.0, device="cuda")
-    res = torch.zeros(staged.size, device="cuda")
-    torch.cuda.synchronize()
-    p = [C.c_void_p(t.data_ptr()) for t in (waves, *dev, res)]
+    hip = _Hip()
+    nw = 2 * nx * ny * nwave
+    waves = hip.put(np.full(nw + 64 * ny, 7.0, np.float32))
+    res = hip.put(np.zeros(staged.size, np.float32))
     eng = engines[1]
-    rc = eng.L.jms_hip_run_batch_noalloc(eng.h, 0, nwave, p[0], p[1], p[2], nwave, 1, p[3], p[4])
+    rc = eng.L.jms_hip_run_batch_noalloc(eng.h, 0, nwave, waves, hip.put(ppar), hip.put(np.asarray(var, np.int32)),
+                                         nwave, 1, hip.put(w), res)
     assert rc == 0, eng.L.jms_hip_last_error(eng.h)
     eng.sync()
-    got["caller's buffers"] = res.cpu().numpy().reshape(staged.shape)
-    assert bool((waves[2 * nx * ny * nwave:] == 7.0).all()), "written behind the caller's waves"
+    got["caller's buffers"] = hip.get(res, staged.shape, np.float32)
+    behind = hip.get(waves, (nw + 64 * ny,), np.float32)[nw:]
+    hip.free()
+    assert (behind == 7.0).all(), "written behind the caller's waves"
     for eng in engines:
         eng.close()
     for what, r in got.items():
