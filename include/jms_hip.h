@@ -174,12 +174,14 @@ int jms_hip_get_scan_results(jms_hip_engine* e, float* out);
 /* batch size in probe passes (waves resident at once, at most 65535); 0 =
  * automatic (about 2 GiB of waves, at most 8192) */
 int jms_hip_set_batch(jms_hip_engine* e, int nwave_max);
-/* 1: capture the per-batch launch sequence in a HIP graph and replay it */
+/* 1: capture the per-batch launch sequence in HIP graphs (one for each part
+ * of a batch larger than the Infinity Cache) and replay them */
 int jms_hip_set_graph(jms_hip_engine* e, int use_graph);
 
 /* single-wave path (CJMultiSlice::GPUMultislice) --------------------------- */
 /* wave <- probe * exp(-i[2pi(kx dx + ky dy + k^2 dz wl/2) + cppl]), with a
- * cyclic beam-tilt shift (ibtx, ibty) pixels -- OffsetIncomingWave :1961 */
+ * cyclic beam-tilt shift (ibtx, ibty) pixels -- OffsetIncomingWave :1961
+ * (asynchronous; reading the wave or a result waits) */
 int jms_hip_wave_offset(jms_hip_engine* e, float dx, float dy, float dz, int ibtx, int ibty,
                         int use_cppl);
 /* wave <- host data (Fourier space) -- SetIncomingWaveGPU :4468 */
