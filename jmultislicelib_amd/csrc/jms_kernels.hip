@@ -259,7 +259,8 @@ __device__ __forceinline__ float ff_gmag(float qx, float qy) {
 // P x P pixels a thread from 2 P values in LDS.  Bound by the float FMAs (four
 // per atom and pixel) where one sine and cosine per atom and pixel was: 8
 // variants of 512^2, 160 atoms each, 364 -> 99 us on MI355X (34 of them the FMAs
-// at 80 TFLOP/s; the rest mostly the double sines and cosines of the factors).
+// at 80 TFLOP/s; with float sines and cosines 94; in tiles of 32 or 48 pixels
+// 125 and 150, as the factors are computed more often).
 // Every thread walks the same list, so the type switches are uniform.
 // grid: (ceil(nx / 16 P), ceil(ny / 16 P), nvar), block: 256
 constexpr int kFFChunk = 32;
