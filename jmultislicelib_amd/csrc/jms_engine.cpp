@@ -128,7 +128,13 @@ struct jms_hip_engine {
   int ndetslc = 0, ndet = 0, detflags = 0;
   std::vector<int> det_objslc;
   DevBuf detw, detw_t, det_cols;
-  std::vector<unsigned> det_cols_h;  // bit d of entry x: detector d has a weight in column x
+  // bit d of entry x: detector d has a weight in column x; in use (columns())
+  // once every detector of the set-up has been uploaded (det_seen)
+  std::vector<unsigned> det_cols_h;
+  unsigned det_seen = 0;
+  const unsigned* columns() const {
+    return ndet > 0 && det_seen == (1u << ndet) - 1 ? (const unsigned*)det_cols.p : nullptr;
+  }
   std::vector<char> det_inf;  // detectors with weights that are not finite
   // incident wave
   DevBuf wav0, cppl, cppl_t;
@@ -195,7 +201,7 @@ struct jms_hip_engine {
   // device addresses a captured batch depends on
   std::array<const void*, 18> batch_buffers() const {
     return {waves.p, partial.p, cur_ppar.p, cur_var.p, cur_res.p, s_weights.p, wav0.p, pgr.p,
-            pro.p, pro_t.p, detw.p, detw_t.p, det_cols.p, twx.p, twy.p, cppl.p, cppl_t.p, loop_tab.p};
+            pro.p, pro_t.p, detw.p, detw_t.p, columns(), twx.p, twy.p, cppl.p, cppl_t.p, loop_tab.p};
   }
   int ntiles_col(bool lat = false) const { return jms::col_tiles(ny, nx, lat); }
   // The columns and rows that the waves leave out: where the propagators of
@@ -456,7 +462,7 @@ int enqueue_batch(jms_hip_engine* e, void* waves, float* partial, int nwave, int
   ca.cppl = e->have_cppl ? e->cppl.as<float>() : nullptr;
   ca.cppl_t = e->have_cppl ? e->cppl_t.as<float>() : nullptr;
   ca.detw_t = e->detw_t.as<float>();
-  ca.det_cols = e->det_cols.as<unsigned>();
+  ca.det_cols = e->columns();
   ca.ndet = (e->detflags & JMS_HIP_DETECT_INTEGRATED) ? e->ndet : 0;
   ca.detw = e->detw.as<float>();
   ca.partial = partial;
@@ -731,11 +737,7 @@ int jms_hip_set_grid(jms_hip_engine* e, int nx, int ny, float a0x, float a0y, fl
   err = e->twy.ensure(tw.size() * sizeof(float));
   if (err == hipSuccess) err = hipMemcpy(e->twy.p, tw.data(), tw.size() * sizeof(float), hipMemcpyHostToDevice);
   if (err != hipSuccess) return e->fail(102, "twiddles y", err);
-  e->det_cols_h.assign(nx, ~0u);  // until the detection is set up for this grid
-  err = e->det_cols.ensure(sizeof(unsigned) * (size_t)nx);
-  if (err == hipSuccess)
-    err = hipMemcpy(e->det_cols.p, e->det_cols_h.data(), sizeof(unsigned) * (size_t)nx, hipMemcpyHostToDevice);
-  if (err != hipSuccess) return e->fail(102, "detector columns", err);
+  e->det_seen = 0;  // the columns are those of another grid
   return 0;
 }
 
@@ -987,6 +989,8 @@ int jms_hip_setup_detection(jms_hip_engine* e, int ndetslc, const int* det_objsl
   e->detflags = flags;
   e->det_objslc.assign(det_objslc, det_objslc + e->nobjslc + 1);
   e->det_inf.assign(ndet, 0);
+  e->det_cols_h.assign(e->nx, 0u);
+  e->det_seen = 0;
   e->pin_valid = false;
   // averaging channels start empty (DetectorSetup, JMultiSlice.cpp:784-800)
   {
@@ -1010,8 +1014,6 @@ int jms_hip_setup_detection(jms_hip_engine* e, int ndetslc, const int* det_objsl
     if (err == hipSuccess) err = hipMemset(e->detw.p, 0, sizeof(float) * (size_t)ndet * e->n);
     if (err == hipSuccess) err = e->detw_t.ensure(sizeof(float) * (size_t)ndet * e->n);
     if (err == hipSuccess) err = hipMemset(e->detw_t.p, 0, sizeof(float) * (size_t)ndet * e->n);
-    e->det_cols_h.assign(e->nx, 0u);
-    if (err == hipSuccess) err = hipMemset(e->det_cols.p, 0, sizeof(unsigned) * (size_t)e->nx);
     if (err != hipSuccess) return e->fail(103, "allocate detector functions", err);
   }
   refresh_loop(e);
@@ -1046,14 +1048,19 @@ int jms_hip_upload_detector(jms_hip_engine* e, int idet, const float* det, int m
   hipError_t err = hipMemcpy(e->detw.as<float>() + (long long)idet * e->n, wgt.data(), nb, hipMemcpyHostToDevice);
   if (err == hipSuccess)
     err = hipMemcpy(e->detw_t.as<float>() + (long long)idet * e->n, wt.data(), nb, hipMemcpyHostToDevice);
-  if (idet < 32)
-    for (int x = 0; x < e->nx; ++x) {
-      const float* col = wt.data() + (size_t)x * e->ny;
-      const bool any = std::any_of(col, col + e->ny, [](float v) { return !(v == 0.f); });
-      e->det_cols_h[x] = (e->det_cols_h[x] & ~(1u << idet)) | (any ? 1u << idet : 0u);
-    }
-  if (err == hipSuccess)
-    err = hipMemcpy(e->det_cols.p, e->det_cols_h.data(), sizeof(unsigned) * (size_t)e->nx, hipMemcpyHostToDevice);
+  e->det_cols_h.resize(e->nx, ~0u);
+  for (int x = 0; x < e->nx; ++x) {
+    const float* col = wt.data() + (size_t)x * e->ny;
+    const bool any = std::any_of(col, col + e->ny, [](float v) { return !(v == 0.f); });
+    e->det_cols_h[x] = (e->det_cols_h[x] & ~(1u << idet)) | (any ? 1u << idet : 0u);
+  }
+  e->det_seen |= 1u << idet;
+  if (e->det_seen == (1u << e->ndet) - 1) {
+    const size_t nc = sizeof(unsigned) * (size_t)e->nx;
+    if (err == hipSuccess) err = e->det_cols.ensure(nc);
+    if (err == hipSuccess) err = hipMemcpy(e->det_cols.p, e->det_cols_h.data(), nc, hipMemcpyHostToDevice);
+    if (err != hipSuccess) e->det_seen = 0;
+  }
   if (err != hipSuccess) return e->fail(104, "upload detector", err);
   return 0;
 }
@@ -1455,7 +1462,7 @@ int group_build(jms_hip_group* g, std::vector<char>& host) {
       jb.partial = e->partial.as<float>();
       jb.pgr = e->pgr.p;
       jb.detw_t = e->detw_t.as<float>();
-      jb.det_cols = e->det_cols.as<unsigned>();
+      jb.det_cols = e->columns();
       jb.cppl_t = e->have_cppl ? e->cppl_t.as<float>() : nullptr;
       jb.detw = e->detw.as<float>();
       jb.cppl = e->have_cppl ? e->cppl.as<float>() : nullptr;

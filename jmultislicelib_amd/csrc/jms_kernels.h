@@ -56,7 +56,7 @@ struct ColArgsHost {
   // column-major ([x][y]) copies for the wave-local column kernel
   const void* pro_t = nullptr;   // propagator of this slice (float2)
   const float* detw_t = nullptr; // [ndet][nx][ny] detector weights
-  const unsigned* det_cols = nullptr;  // [nx]: bit d set where detector d has a weight in the column
+  const unsigned* det_cols = nullptr;  // [nx]: bit d set where detector d has a weight in the column; nullptr: all
   const float* cppl_t = nullptr; // constant phase plate or nullptr
   bool panel = false;            // the waves are in 16-column panels (panel_ok)
   BandHost band;                 // columns and rows left out

@@ -385,7 +385,7 @@ struct ColArgs {
   // column-major copies used by the wave-local column kernel: [x][y]
   const float2* pro_t;      // propagator of this slice
   const float* detw_t;      // [ndet][nx][ny] detector weights
-  const unsigned* det_cols; // [nx]: bit d set where detector d has a weight in the column
+  const unsigned* det_cols; // [nx]: bit d set where detector d has a weight in the column, or nullptr: all
   const float* cppl_t;      // constant phase plate
   GrpArgs grp;              // grouped launch: wave map and job / plane tables
   // band-limited waves: tiles [tg0, tg0 + tgn) hold only columns where every
@@ -489,7 +489,7 @@ __device__ __forceinline__ void col_body(const ColArgs& a, long long w, float2* 
   // dependent loads (625^2, 32 waves, three ring detectors: 118 -> 108 us for
   // the launch of a detection plane, 75 without one)
   [[maybe_unused]] unsigned dets = 0;
-  if (DET && a.detect && valid && a.ndet > 0) dets = a.det_cols[wrap_sub(x, a.dsx, nx)];
+  if (DET && a.detect && valid) dets = a.det_cols ? a.det_cols[wrap_sub(x, a.dsx, nx)] : ~0u;
   float2 v[NREG];
   if constexpr (INIT) {
     float dx = 0.f, dy = 0.f, fz = 0.f;
