@@ -39,7 +39,8 @@ struct LoopCol {
 
 // BAND: columns [gx0, gx1) and the dead row slots are zero in every
 // propagator and the columns in the source: their LDS columns stay zero and
-// are not transformed.
+// are not transformed.  The source may hold anything in the dead rows: the
+// incident plane's readout and the first transform take them all.
 // The same loop in two launches per slice / here, us per slice on MI355X:
 // 64^2 with 1, 64, 256, 1024 waves 6.7 / 4.8, 8.0 / 4.9, 14.8 / 5.2, 25 / 16.8;
 // 96^2 with 1, 64, 256, 1024 waves 8.2 / 10.5, 14.8 / 10.8, 26.6 / 11.6,
@@ -92,8 +93,9 @@ __global__ __launch_bounds__((loop_block<NX, NY>())) void k_loop(LoopArgs a) {
   float2 v[RX > RY ? RX : RY];
   float2 (&vx)[RX] = reinterpret_cast<float2 (&)[RX]>(v);
   float2 (&vy)[RY] = reinterpret_cast<float2 (&)[RY]>(v);
-  // readout of plane p from the columns in registers
-  auto readout = [&](int p) {
+  // readout of plane p from the columns in registers; INC: the incident wave,
+  // which no propagator has made zero in the dead rows
+  auto readout = [&](int p, auto INC) {
     const long long off = a.pl[p].part_off;
     if (off < 0) return;  // uniform
     float acc[kMaxDet];
@@ -105,7 +107,7 @@ __global__ __launch_bounds__((loop_block<NX, NY>())) void k_loop(LoopArgs a) {
         const float* dw = a.detw_t + (long long)d * NX * NY + xs * NY;
         float s = 0.f;
         each_y1([&](auto K, int ky, auto Q) {
-          if constexpr (dead_y(decltype(Q)::value)) return;
+          if constexpr (!decltype(INC)::value && dead_y(decltype(Q)::value)) return;
           const float2 z = vy[decltype(K)::value];
           s += (z.x * z.x + z.y * z.y) * dw[wrap_sub(ky, a.dsy, NY)];
         });
@@ -154,7 +156,7 @@ __global__ __launch_bounds__((loop_block<NX, NY>())) void k_loop(LoopArgs a) {
     });
   }
   __syncthreads();  // tables and zeros in place
-  readout(a.islc0);
+  readout(a.islc0, std::true_type{});
   if (col_on) down();
   const int* var = a.var + w * a.var_ld;
 #pragma unroll 1
@@ -244,7 +246,7 @@ __global__ __launch_bounds__((loop_block<NX, NY>())) void k_loop(LoopArgs a) {
         else vy[k] = cmul(vy[k], pv[k]);
       });
     }
-    readout(j + 1);
+    readout(j + 1, std::false_type{});
     if (j + 1 < a.nslc && col_on) {
       SyncWave{}();
       down();
