@@ -154,6 +154,20 @@ struct Lat : CfgP<N> {
   static constexpr bool PF = true;
 };
 
+// The allocation-free entry's column tiles at a length that got 8-column ones
+// for its panels with a partly filled last one (625): 16 columns in the natural
+// layout, as the caller's waves cannot hold such panels, and half as many
+// readout sums per wave in that entry's fixed scratch.  Cfg's tiles at all other
+// lengths.
+template <int N>
+struct Wide : CfgP<N> {
+  using B = CfgP<N>;
+  static constexpr bool OWN = !(B::PANEL && N % 16 != 0);
+  static constexpr int CW = OWN ? B::CW : 16;
+  static constexpr int CC = OWN ? B::CC : CW;
+  static constexpr int PADSH_COL = OWN ? B::PADSH_COL : B::PADSH;
+};
+
 // Cfg's shape for waves that stay in the 256 MB Infinity Cache from one pass
 // to the next (split_of in jms_engine.cpp): ordinary loads and stores, as
 // nontemporal ones make the cache drop the lines that the next pass reads, and

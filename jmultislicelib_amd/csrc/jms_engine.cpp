@@ -203,7 +203,7 @@ struct jms_hip_engine {
     return {waves.p, partial.p, cur_ppar.p, cur_var.p, cur_res.p, s_weights.p, wav0.p, pgr.p,
             pro.p, pro_t.p, detw.p, detw_t.p, columns(), twx.p, twy.p, cppl.p, cppl_t.p, loop_tab.p};
   }
-  int ntiles_col(bool lat = false) const { return jms::col_tiles(ny, nx, lat); }
+  int ntiles_col(jms::Tile t = jms::Tile::Own) const { return jms::col_tiles(ny, nx, t); }
   // The columns and rows that the waves leave out: where the propagators of
   // all object slices vanish.  A detector weight that is not finite makes
   // 0 * weight count, so those keep every column.
@@ -221,9 +221,9 @@ struct jms_hip_engine {
     }
     return g;
   }
-  jms::BandHost band(bool lat) const {
+  jms::BandHost band(jms::Tile t) const {
     const Gap g = gap();
-    return jms::band_of(nx, ny, g.x0, g.x1, g.y0, g.y1, lat);
+    return jms::band_of(nx, ny, g.x0, g.x1, g.y0, g.y1, t);
   }
   // the probe is zero there too, so the first passes leave the columns out as well
   static bool holds(const Gap& g, const jms::BandHost& b) { return g.x0 <= b.x0 && g.x1 >= b.x1; }
@@ -431,26 +431,29 @@ int enqueue_combine(jms_hip_engine* e, float* partial, int nwave, int islc0, int
 // (stride n); `ppar` (float4 per wave) and `var` (nobjslc ints per wave)
 // describe them; src/src_stride the INIT source.  Readout partial sums go to
 // `partial` ([wave][plane][detector][column tile]), combined into `res`
-// (npos results) when npass > 0; `ch` are the single-wave channels.  `lat`:
-// the small launch shapes (natural wave layout); `src_same`: the source is the
-// probe, else the single-wave path's wave; `keep`: leave psi(k) of the exit
-// plane in the waves (batches only read the sums).  The band's columns are
-// left out from the first slice on, and before it where the source is zero
-// there.  `mirror` (or nullptr): host memory that gets the results too.  `part`
+// (npos results) when npass > 0; `ch` are the single-wave channels.  `tile`:
+// Small for the small launch shapes (natural wave layout), Wide for the
+// allocation-free entry (natural layout where jms_cfg.hpp has such tiles);
+// `src_same`: the source is the probe, else the single-wave path's wave;
+// `keep`: leave psi(k) of the exit plane in the waves (batches only read the
+// sums).  The band's columns are left out from the first slice on, and before
+// it where the source is zero there.  `mirror` (or nullptr): host memory that
+// gets the results too.  `part`
 // (or -1): only the passes of this part of a batch that goes in several
 // (split_of), on the engine's stream, without the combination.
 int enqueue_batch(jms_hip_engine* e, void* waves, float* partial, int nwave, int islc0, const void* src,
                   long long src_stride, const void* ppar, const int* var, int npos, int npass,
                   const float* weights, float* res, int accumulate, const BatchChans& ch, bool timed,
-                  bool lat, bool src_same, bool keep, bool panel, float* mirror = nullptr, int part = -1) {
-  const jms::BandHost bd = e->band(lat);
+                  jms::Tile tile, bool src_same, bool keep, bool panel, float* mirror = nullptr, int part = -1) {
+  const bool lat = tile == jms::Tile::Small;
+  const jms::BandHost bd = e->band(tile);
   const bool src_in = e->holds(src_same ? e->wav0_gap : e->wav_gap, bd);
   // panel waves (staged batches): integrated readouts only, the waves are internal
   if (panel && ch.any())
     return e->fail(135, "panel waves carry no readout channels");
   const int S = e->nobjslc;
   const bool loop = use_loop(e, nwave, islc0) && !ch.any();
-  const int ntc = loop ? 1 : e->ntiles_col(lat);
+  const int ntc = loop ? 1 : e->ntiles_col(tile);
   const long long part_w = (long long)e->ndetslc * e->ndet * ntc;
   jms::ColArgsHost ca;
   ca.wave = waves;
@@ -532,6 +535,7 @@ int enqueue_batch(jms_hip_engine* e, void* waves, float* partial, int nwave, int
     const int parts = two ? sp.parts() : sp.rounds;
     const jms::Shape shape = lat ? jms::Shape::Small : sp.near ? jms::Shape::Near : jms::Shape::Stream;
     ca.shape = shape;
+    ca.tile = tile;
     SideBranch branch(e, two && part < 0);
     if (branch.err != hipSuccess) return e->fail(129, "second stream", branch.err);
     struct Part {
@@ -637,7 +641,7 @@ int ensure_batch(jms_hip_engine* e, int nwave) {
   hipError_t err = e->waves.ensure(sizeof(float) * 2 * (size_t)e->wave_items(e->panel) * nwave);
   if (err != hipSuccess) return e->fail(110, "allocate wave batch", err);
   const size_t np = sizeof(float) * (size_t)nwave * std::max(1, e->ndetslc) *
-                    std::max(1, e->ndet) * (size_t)std::max(e->ntiles_col(), e->ntiles_col(true));
+                    std::max(1, e->ndet) * (size_t)std::max(e->ntiles_col(), e->ntiles_col(jms::Tile::Small));
   err = e->partial.ensure(np);
   if (err != hipSuccess) return e->fail(111, "allocate readout partials", err);
   return 0;
@@ -1241,6 +1245,7 @@ int jms_hip_run_staged(jms_hip_engine* e, int pos0, int npos, int islc0) {
     const int* var = e->s_var.as<int>() + (long long)p * npass * S;
     float* res = e->s_res.as<float>() + (long long)p * per;
     const bool lat = jms::lat_ok(e->nx, e->ny, nw), panel = e->panel && !lat;
+    const jms::Tile tile = lat ? jms::Tile::Small : jms::Tile::Own;
     if (e->use_graph) {
       // the graph reads fixed "current batch" buffers, refreshed before replay
       hipError_t err = e->cur_ppar.ensure(sizeof(float4) * (size_t)bw);
@@ -1252,7 +1257,7 @@ int jms_hip_run_staged(jms_hip_engine* e, int pos0, int npos, int islc0) {
       if (err != hipSuccess) return e->fail(120, "stage batch", err);
       const auto bufs = e->batch_buffers();
       // the band of the small and of the large launch shapes follow from one gap
-      const jms::BandHost b0 = e->band(false), b1 = e->band(true);
+      const jms::BandHost b0 = e->band(jms::Tile::Own), b1 = e->band(jms::Tile::Small);
       const Gap g = e->gap();
       const std::array<int, 12> gband{b0.x0, b0.x1, b0.rows, e->probe_in(b0), b1.x0, b1.x1, b1.rows, e->probe_in(b1),
                                       g.x0, g.x1, e->wav0_gap.x0, e->wav0_gap.x1};
@@ -1263,7 +1268,7 @@ int jms_hip_run_staged(jms_hip_engine* e, int pos0, int npos, int islc0) {
       }
       const std::array<int, 4> key{nw, islc0, np, npass};
       auto it = e->graphs.find(key);
-      const int ntc = e->ntiles_col(lat);
+      const int ntc = e->ntiles_col(tile);
       const Split sp = use_loop(e, nw, islc0) ? Split() : split_of(e, nw, b0, lat, false);
       const int parts = sp.parts();
       if (it == e->graphs.end()) {
@@ -1278,7 +1283,7 @@ int jms_hip_run_staged(jms_hip_engine* e, int pos0, int npos, int islc0) {
           }
           rc = enqueue_batch(e, e->waves.p, e->partial.as<float>(), nw, islc0, e->wav0.p, 0, e->cur_ppar.p,
                              e->cur_var.as<int>(), np, npass, e->s_weights.as<float>(), e->cur_res.as<float>(), 0,
-                             BatchChans(), false, lat, true, false, panel, nullptr, parts > 1 ? q : -1);
+                             BatchChans(), false, tile, true, false, panel, nullptr, parts > 1 ? q : -1);
           err = hipStreamEndCapture(e->st, &gr);
           if (!rc && err != hipSuccess) rc = e->fail(122, "end capture", err);
           if (!rc) {
@@ -1312,7 +1317,7 @@ int jms_hip_run_staged(jms_hip_engine* e, int pos0, int npos, int islc0) {
     } else {
       rc = enqueue_batch(e, e->waves.p, e->partial.as<float>(), nw, islc0, e->wav0.p, 0, ppar, var, np, npass,
                          e->s_weights.as<float>(), res,
-                         0, BatchChans(), e->timing, lat, true, false, panel);
+                         0, BatchChans(), e->timing, tile, true, false, panel);
       if (rc) return rc;
     }
   }
@@ -1330,7 +1335,7 @@ int jms_hip_run_batch_noalloc(jms_hip_engine* e, int islc0, int nwave, void* wav
   if (!waves || !ppar || !weights || !res || (e->nobjslc > 0 && !var)) return e->fail(3, "missing buffer");
   if (!(e->detflags & JMS_HIP_DETECT_INTEGRATED) || e->ndet < 1)
     return e->fail(4, "no integrating detectors set up");
-  const long long need = (long long)nwave * std::max(1, e->ndetslc) * e->ndet * e->ntiles_col();
+  const long long need = (long long)nwave * std::max(1, e->ndetslc) * e->ndet * e->ntiles_col(jms::Tile::Wide);
   if (need > jms::kScratchFloats) {
     char msg[200];
     snprintf(msg, sizeof(msg), "batch needs %lld floats of readout scratch, more than the %lld available "
@@ -1341,12 +1346,14 @@ int jms_hip_run_batch_noalloc(jms_hip_engine* e, int islc0, int nwave, void* wav
   islc0 = std::max(0, std::min(islc0, e->nobjslc));
   (void)hipSetDevice(e->device);
   // the small launch shapes need up to twice the tiles: only where those fit too
-  const long long need_lat = (long long)nwave * std::max(1, e->ndetslc) * e->ndet * e->ntiles_col(true);
+  const long long need_lat = (long long)nwave * std::max(1, e->ndetslc) * e->ndet * e->ntiles_col(jms::Tile::Small);
   const bool lat = jms::lat_ok(e->nx, e->ny, nwave) && need_lat <= jms::kScratchFloats;
-  // the caller's waves have n items each: no partly filled panels
-  const bool panel = e->panel && !lat && e->wave_items(true) == e->n;
+  // the caller's waves have n items each: no partly filled panels, and none
+  // where the columns take tiles for the natural layout
+  const bool own = e->ntiles_col(jms::Tile::Wide) == e->ntiles_col();
+  const bool panel = e->panel && !lat && own && e->wave_items(true) == e->n;
   return enqueue_batch(e, waves, e->scratch, nwave, islc0, e->wav0.p, 0, ppar, var, npos, npass, weights, res, 0,
-                       BatchChans(), false, lat, true, false, panel);
+                       BatchChans(), false, lat ? jms::Tile::Small : jms::Tile::Wide, true, false, panel);
 }
 
 // ---------------------------------------------------------------------------
@@ -1597,10 +1604,10 @@ int jms_hip_group_run(jms_hip_group* g) {
     g->host.swap(host);
   }
   // one band for all members: the columns and rows that every member leaves out
-  jms::BandHost bd = lead->band(false);
+  jms::BandHost bd = lead->band(jms::Tile::Own);
   for (auto* e : g->eng) {
     if (e->nobjslc < 1) continue;  // only its INIT pass, which covers its own columns
-    const jms::BandHost b = e->band(false);
+    const jms::BandHost b = e->band(jms::Tile::Own);
     bd.x0 = std::max(bd.x0, b.x0);
     bd.x1 = std::min(bd.x1, b.x1);
     bd.rows = bd.rows && b.rows;
@@ -1784,13 +1791,13 @@ int jms_hip_multislice(jms_hip_engine* e, int islc0, const int* var, float weigh
   if (fl & JMS_HIP_DETECT_IMAGE_AVG) ch.img_avg = e->img_avg.as<float>();
   if (fl & JMS_HIP_DETECT_WAVEF_AVG) ch.wff_avg = e->wff_avg.p;
   if (fl & JMS_HIP_DETECT_WAVER_AVG) ch.wfr_avg = e->wfr_avg.p;
-  const bool lat = jms::lat_ok(e->nx, e->ny, 1);
+  const jms::Tile tile = jms::lat_ok(e->nx, e->ny, 1) ? jms::Tile::Small : jms::Tile::Own;
   // in place: every block of a pass reads its tile of the wave before it writes it
   rc = enqueue_batch(e, e->wav.p, e->partial.as<float>(), 1, islc0, e->wav.p, e->n, nullptr, e->in1.as<int>() + 1, 1, 1,
-                     e->in1.as<float>(), e->res1.as<float>(), accumulate, ch, e->timing, lat, false, true, false,
+                     e->in1.as<float>(), e->res1.as<float>(), accumulate, ch, e->timing, tile, false, true, false,
                      mirror);
   if (islc0 < S) {  // the wave becomes psi(k) of the exit plane
-    const jms::BandHost bd = e->band(lat);
+    const jms::BandHost bd = e->band(tile);
     e->wav_gap = rc ? Gap() : Gap{bd.x0, bd.x1, 0, 0};
   }
   if (rc) return rc;

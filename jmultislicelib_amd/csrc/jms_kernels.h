@@ -16,8 +16,10 @@ struct BandHost {
   bool on() const { return x1 > x0; }
 };
 // the band the passes of an nx x ny grid use, given columns [gx0, gx1) and
-// rows [gy0, gy1) where every propagator of the run vanishes
-BandHost band_of(int nx, int ny, int gx0, int gx1, int gy0, int gy1, bool lat);
+// rows [gy0, gy1) where every propagator of the run vanishes; tile: the column
+// tiles of Cfg, Lat or Wide (jms_cfg.hpp)
+enum class Tile { Own, Small, Wide };
+BandHost band_of(int nx, int ny, int gx0, int gx1, int gy0, int gy1, Tile tile);
 // launch shapes of a batch's passes: waves streamed from memory (Cfg in
 // jms_cfg.hpp), few blocks (Lat; see lat_ok), waves in the Infinity Cache (Near)
 enum class Shape { Stream, Small, Near };
@@ -62,6 +64,7 @@ struct ColArgsHost {
   BandHost band;                 // columns and rows left out
   bool keep = false;             // EXIT: store psi(k), the columns left out cleared
   Shape shape = Shape::Stream;
+  Tile tile = Tile::Own;         // Small with Shape::Small; Wide: natural layout
 };
 
 // real-space readout channels of one detection plane for the row pass
@@ -197,7 +200,7 @@ constexpr int kMaxDetPerSweep = 8;
 
 bool size_supported(int n);
 int row_tiles(int nx, int ny);
-int col_tiles(int ny, int nx, bool lat);
+int col_tiles(int ny, int nx, Tile tile);
 
 // mode 0: slice; 1: slice with the real-space readout of `rc` first;
 // 2: inverse x-transform and readout only (exit plane, after a column IFFT).

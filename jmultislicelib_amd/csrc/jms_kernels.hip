@@ -407,9 +407,13 @@ int row_tiles(int nx, int ny) {
   }
 }
 
-int col_tiles(int ny, int nx, bool lat) {
+template <int N>
+static constexpr int tile_width(Tile tile) {
+  return tile == Tile::Small ? Lat<N>::CC : tile == Tile::Wide ? Wide<N>::CC : Cfg<N>::CC;
+}
+int col_tiles(int ny, int nx, Tile tile) {
   switch (ny) {
-#define JMS_CASE(N) case N: return lat ? (nx + Lat<N>::CC - 1) / Lat<N>::CC : (nx + Cfg<N>::CC - 1) / Cfg<N>::CC;
+#define JMS_CASE(N) case N: return (nx + tile_width<N>(tile) - 1) / tile_width<N>(tile);
     JMS_SIZES(JMS_CASE)
 #undef JMS_CASE
     default: return 0;
@@ -421,11 +425,11 @@ static bool band_loop_col_n(int y0, int y1) {
   using BS = BandSlots<NY, radix_at<typename Cfg<NY>::PC, true>(0)>;
   return BS::G0_MAX >= BS::G1_MIN || (y0 <= BS::G0_MAX && y1 >= BS::G1_MIN);
 }
-BandHost band_of(int nx, int ny, int gx0, int gx1, int gy0, int gy1, bool lat) {
+BandHost band_of(int nx, int ny, int gx0, int gx1, int gy0, int gy1, Tile tl) {
   BandHost b;
   int tile = 0;
   switch (ny) {
-#define JMS_CASE(N) case N: tile = lat ? Lat<N>::CC : Cfg<N>::CC; b.rows = band_col_n<N>(gy0, gy1); break;
+#define JMS_CASE(N) case N: tile = tile_width<N>(tl); b.rows = band_col_n<N>(gy0, gy1); break;
     JMS_SIZES(JMS_CASE)
 #undef JMS_CASE
     default: return b;
@@ -444,7 +448,7 @@ bool lat_ok(int nx, int ny, int nwave) {
   // a pair of passes in this shape / in Cfg's, us: 512^2 1 wave 10.8 / 13.2,
   // 4 waves 17.0 / 16.2; 256^2 8 waves 12.4 / 12.7, 16 waves 16.8 / 15.3;
   // 128^2 16 waves 8.8 / 9.3, 32 waves 11.8 / 11.0 (tiles: 32, 16, 8)
-  return wl && nwave * col_tiles(ny, nx, false) < 128;
+  return wl && nwave * col_tiles(ny, nx, Tile::Own) < 128;
 }
 
 // The slice loop in one launch takes one block per wave and CU (two at 64^2)

@@ -1313,9 +1313,9 @@ hipError_t launch_col_pass_n(int nwave, bool init, bool exit_, const ColArgsHost
   a.cppl_t = h.cppl_t;
   using CF = Cfg<N>;
   static_assert(CF::XL || CF::WL, "every line length has a column kernel");
-  const bool lat = h.shape == Shape::Small;
-  if (h.panel && (!CF::PANEL || lat)) return hipErrorInvalidValue;
-  const int cc = lat ? Lat<N>::CC : CF::CC, tiles = (h.nx + cc - 1) / cc;
+  const bool lat = h.tile == Tile::Small, wide = h.tile == Tile::Wide && !Wide<N>::OWN;
+  if (h.panel && (!CF::PANEL || lat || wide)) return hipErrorInvalidValue;
+  const int cc = lat ? Lat<N>::CC : wide ? Wide<N>::CC : CF::CC, tiles = (h.nx + cc - 1) / cc;
   a.tg0 = h.band.x0 / cc;
   a.tgn = h.band.on() ? (h.band.x1 - h.band.x0) / cc : 0;
   a.keep = h.keep;
@@ -1334,7 +1334,9 @@ hipError_t launch_col_pass_n(int nwave, bool init, bool exit_, const ColArgsHost
       else if constexpr (CF::PANEL) launch_col_w<N, CS, false, true>(g, b, init, exit_, h.detect, h.band.rows, a, st);
     };
     if (lat) launch_col_w<N, Lat<N>, false, false>(g, b, init, exit_, h.detect, h.band.rows, a, st);
-    else if (h.shape == Shape::Near) pick(CN{});
+    else if (wide) {
+      if constexpr (!Wide<N>::OWN) launch_col_w<N, Wide<N>, false, false>(g, b, init, exit_, h.detect, h.band.rows, a, st);
+    } else if (h.shape == Shape::Near) pick(CN{});
     else pick(CF{});
   }
   return hipGetLastError();
