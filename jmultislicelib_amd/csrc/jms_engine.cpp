@@ -1775,7 +1775,15 @@ int jms_hip_multislice(jms_hip_engine* e, int islc0, const int* var, float weigh
       if (err == hipSuccess && (fl & r.flag)) err = hipMemsetAsync(r.b->p, 0, r.nb, e->st);
     if (err != hipSuccess) return e->fail(111, "clear detector channels", err);
   }
-  // every earlier run on the pinned buffer has been waited for
+  // every earlier run on the pinned buffer has been waited for, and this one is
+  // wherever it returns from here on
+  struct Waits {
+    hipStream_t st;
+    bool on = true;
+    ~Waits() {
+      if (on) (void)hipStreamSynchronize(st);
+    }
+  } waits{e->st};
   e->pin[0] = weight;
   if (S > 0) memcpy(e->pin + 1, var, sizeof(int) * S);
   err = hipMemcpyAsync(e->in1.p, e->pin, sizeof(float) * nin, hipMemcpyHostToDevice, e->st);
@@ -1803,6 +1811,7 @@ int jms_hip_multislice(jms_hip_engine* e, int islc0, const int* var, float weigh
   if (rc) return rc;
   rc = enqueue_exit_real_readout(e, 1, ch);
   if (rc) return rc;
+  waits.on = false;
   err = hipStreamSynchronize(e->st);
   if (err != hipSuccess) return e->fail(113, "multislice run", err);
   e->pin_valid = mirror != nullptr;
