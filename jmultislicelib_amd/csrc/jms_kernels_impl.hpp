@@ -569,6 +569,15 @@ __device__ __forceinline__ void col_body(const ColArgs& a, long long w, float2* 
           pw[i * M1::R0 + q] = z.x * z.x + z.y * z.y;
         });
       });
+      // a value that is not finite makes every sum so (0 * inf), also those of
+      // the detectors without a weight here
+      float top = 0.f;
+      static_for<0, M1::NB>([&](auto I) {
+        constexpr int i = decltype(I)::value;
+        if (M1::FULL || t + i * T < M1::NBF)
+          static_for<0, M1::R0>([&](auto Q) { top += pw[i * M1::R0 + decltype(Q)::value]; });
+      });
+      if (!(top < __builtin_huge_valf())) dets = ~0u;
       // de-scan (DescanDifN, JMultiSlice.cpp:2184-2275): pixel i is weighted
       // with det(i - d)
       const long long colbs = (long long)wrap_sub(x, a.dsx, nx) * N;
