@@ -64,6 +64,15 @@ bool zeros(const float* row, int i0, int i1) {
   }
   return (any & 0x7fffffffu) == 0;
 }
+bool finite(const float* a, size_t n) {
+  uint32_t inf = 0;
+  for (size_t k = 0; k < n; ++k) {
+    uint32_t u;
+    std::memcpy(&u, a + k, 4);
+    inf |= ((u & 0x7f800000u) == 0x7f800000u);
+  }
+  return inf == 0;
+}
 Gap zero_gap(const float* a, int nx, int ny, bool rows) {
   Gap g{0, nx, 0, 0};
   auto row = [&](int y) { return a + 2 * (size_t)y * nx; };
@@ -139,7 +148,7 @@ struct jms_hip_engine {
   // incident wave
   DevBuf wav0, cppl, cppl_t;
   Gap wav0_gap, wav_gap;  // zero gap (columns) of the probe and of the single-wave path's wave
-  bool have_cppl = false;
+  bool have_cppl = false, cppl_inf = false;  // cppl_inf: some phase not finite
   // staged scan
   int s_npos = 0, s_npass = 0;
   DevBuf s_ppar, s_weights, s_var, s_res;
@@ -205,11 +214,12 @@ struct jms_hip_engine {
   }
   int ntiles_col(jms::Tile t = jms::Tile::Own) const { return jms::col_tiles(ny, nx, t); }
   // The columns and rows that the waves leave out: where the propagators of
-  // all object slices vanish.  A detector weight that is not finite makes
-  // 0 * weight count, so those keep every column.
+  // all object slices vanish.  A detector weight or a phase of the constant
+  // plate that is not finite makes 0 * weight (0 * exp(i phase)) count, so those
+  // keep every column.
   Gap gap() const {
     Gap g{0, nx, 0, ny};
-    if (nobjslc < 1) return Gap();
+    if (nobjslc < 1 || (have_cppl && cppl_inf)) return Gap();
     for (char c : det_inf)
       if (c) return Gap();
     for (int o : objslc) {
@@ -1040,13 +1050,7 @@ int jms_hip_upload_detector(jms_hip_engine* e, int idet, const float* det, int m
   } else {
     std::memcpy(wgt.data(), det, sizeof(float) * (size_t)e->n);
   }
-  uint32_t inf = 0;  // some weight not finite
-  for (float x : wgt) {
-    uint32_t u;
-    std::memcpy(&u, &x, 4);
-    inf |= ((u & 0x7f800000u) == 0x7f800000u);
-  }
-  e->det_inf[idet] = inf != 0;
+  e->det_inf[idet] = !finite(wgt.data(), wgt.size());
   std::vector<float> wt = to_colmajor(wgt.data(), e->nx, e->ny);
   const size_t nb = sizeof(float) * (size_t)e->n;
   hipError_t err = hipMemcpy(e->detw.as<float>() + (long long)idet * e->n, wgt.data(), nb, hipMemcpyHostToDevice);
@@ -1147,6 +1151,7 @@ int jms_hip_set_phaseplate(jms_hip_engine* e, const float* cppl) {
   if (err == hipSuccess) err = hipMemcpy(e->cppl_t.p, t.data(), nb, hipMemcpyHostToDevice);
   if (err != hipSuccess) return e->fail(102, "upload phase plate", err);
   e->have_cppl = true;
+  e->cppl_inf = !finite(cppl, (size_t)e->n);
   return 0;
 }
 
@@ -1698,10 +1703,11 @@ int jms_hip_wave_offset(jms_hip_engine* e, float dx, float dy, float dz, int ibt
   if (err != hipSuccess) return e->fail(103, "allocate wave", err);
   int ish0 = ibtx % e->nx; if (ish0 < 0) ish0 += e->nx;  // JMultiSlice.cpp:1990-1991
   int ish1 = ibty % e->ny; if (ish1 < 0) ish1 += e->ny;
-  e->wav_gap = ish0 == 0 ? e->wav0_gap : Gap();
+  const bool plate = use_cppl && e->have_cppl;
+  e->wav_gap = ish0 == 0 && !(plate && e->cppl_inf) ? e->wav0_gap : Gap();
   err = jms::launch_offset_wave(e->wav.as<float2>(), e->wav0.as<float2>(), e->nx, e->ny, 1.f / e->a0x,
                                 1.f / e->a0y, dx, dy, dz * e->wl * 0.5f,
-                                (use_cppl && e->have_cppl) ? e->cppl.as<float>() : nullptr, ish0, ish1, e->st);
+                                plate ? e->cppl.as<float>() : nullptr, ish0, ish1, e->st);
   if (err != hipSuccess) return e->fail(106, "offset incoming wave", err);
   return 0;
 }

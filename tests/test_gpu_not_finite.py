@@ -34,3 +34,28 @@ def test_sums_are_not_finite(nx, ny, value):
     eng.multislice(np.zeros(2, np.int32), 1.0)
     assert not np.isfinite(eng.result(1)).any()
     eng.close()
+
+
+@pytest.mark.parametrize("nx,ny", [(64, 64), (256, 256), (96, 1024)])
+def test_phase_plate_is_not_finite(nx, ny):
+    """The constant phase plate multiplies every column of the incident wave,
+    also those where the probe and the propagators are zero."""
+    sp = random_setup(nx, ny, nslices=2, nvar=(1, 1), ndetper=1, seed=nx)
+    plate = np.zeros((ny, nx), np.float32)
+    plate[ny // 3, nx // 2] = np.nan
+    x = np.zeros(200, np.float32)
+    eng = Engine().setup(sp)
+    eng.stage_scan(x, x, None, np.ones(1, np.float32), np.zeros((200, 2), np.int32))
+    for p in (None, plate, None):
+        eng._c("jms_hip_set_phaseplate", None if p is None else p.ctypes.data)
+        for n in (2, 200):
+            eng.run_staged(0, n)
+            eng.sync()
+            out = eng.scan_results()[:n]
+            assert np.isfinite(out).all() if p is None else not np.isfinite(out).any(), f"{n} waves"
+    eng._c("jms_hip_set_phaseplate", plate.ctypes.data)
+    eng.wave_offset(0.0, 0.0)
+    eng._c("jms_hip_set_phaseplate", None)  # the wave has it already
+    eng.multislice(np.zeros(2, np.int32), 1.0)
+    assert not np.isfinite(eng.result(1)).any()
+    eng.close()
