@@ -320,7 +320,9 @@ __global__ __launch_bounds__(C_::T * C_::LPB) __attribute__((amdgpu_waves_per_eu
 // ---------------------------------------------------------------------------
 // block reduction of kMaxDet per-thread partial sums; thread 0 writes
 // partial[d * dstride] for d < ndet.  red: LDS scratch of >= 64*kMaxDet floats.
+// Sum: the type the wavefronts' sums are added in.
 // ---------------------------------------------------------------------------
+template <class Sum = float>
 __device__ __forceinline__ void block_reduce_det(float (&acc)[kMaxDet], int ndet, float* red,
                                                  float* out, long long dstride) {
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -340,9 +342,9 @@ __device__ __forceinline__ void block_reduce_det(float (&acc)[kMaxDet], int ndet
   __syncthreads();
   if (threadIdx.x < ndet && threadIdx.x < kMaxDet) {
     const int d = threadIdx.x;
-    float s = 0.f;
+    Sum s = 0;
     for (int i = 0; i < nw; ++i) s += red[i * kMaxDet + d];
-    out[d * dstride] = s;
+    out[d * dstride] = (float)s;
   }
 }
 

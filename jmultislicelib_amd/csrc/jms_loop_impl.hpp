@@ -105,18 +105,20 @@ __global__ __launch_bounds__((loop_block<NX, NY>())) void k_loop(LoopArgs a) {
       const int xs = wrap_sub(x, a.dsx, NX);  // de-scan: pixel i is weighted with det(i - d)
       for (int d = 0; d < a.ndet && d < kMaxDet; ++d) {
         const float* dw = a.detw_t + (long long)d * NX * NY + xs * NY;
-        float s = 0.f;
+        float s0 = 0.f, s1 = 0.f;  // two chains: eight terms each, as in a thread of the passes
         each_y1([&](auto K, int ky, auto Q) {
           if constexpr (!decltype(INC)::value && dead_y(decltype(Q)::value)) return;
           const float2 z = vy[decltype(K)::value];
-          s += (z.x * z.x + z.y * z.y) * dw[wrap_sub(ky, a.dsy, NY)];
+          (decltype(K)::value & 1 ? s1 : s0) += (z.x * z.x + z.y * z.y) * dw[wrap_sub(ky, a.dsy, NY)];
         });
 #pragma unroll
         for (int dd = 0; dd < kMaxDet; ++dd)
-          if (dd == d) acc[dd] += s;
+          if (dd == d) acc[dd] += s0 + s1;
       }
     }
-    block_reduce_det(acc, a.ndet, s_red, a.partial + w * a.part_wstride + off, 1);
+    // one tile holds the whole sum: the wavefronts' parts are added in double, as
+    // k_combine adds the tiles of the passes
+    block_reduce_det<double>(acc, a.ndet, s_red, a.partial + w * a.part_wstride + off, 1);
   };
   auto down = [&]() {  // inverse column transform, back into LDS
     LineFFT<NY, TY, +1, PY, true, LY, RY, CY::TWR>::run(vy, s_w, x, s_ty, ty, SyncWave{});
