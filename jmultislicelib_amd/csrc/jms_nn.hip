@@ -315,8 +315,8 @@ __global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float
 // block, eight threads each, which share the shares of a sum.  Sums j:
 // [0, PART) the convolutions' positions of the nb blocks' parts; then the
 // dense layers, over the n samples, from the features and gh, hid and dy of
-// the head; the last stands for the loss (loss_sum: the sum of squares,
-// loss_mean: over the n x 3 outputs; either may be null).
+// the head; the last stands for the loss, summed in double (loss_sum: the sum
+// of squares, loss_mean: over the n x 3 outputs; either may be null).
 static_assert(nnmfma::PART % 64 == 0 && FLAT % 64 == 0, "a block's sums are of one kind, one hidden unit");
 constexpr int UPD_SUMS = nnmfma::PART + NPARAM - OFF_D1W + 1;
 template <bool ADAM>
@@ -377,23 +377,27 @@ __global__ __launch_bounds__(512) void k_update(const float* __restrict__ part, 
     for (int y = q; y < ds; y += 8) {
       const int k1 = nnmfma::share_begin(n, y + 1, ds);
       float s = 0.f;
+      double l = 0.;
 #pragma unroll 4
       for (int k = nnmfma::share_begin(n, y, ds); k < k1; ++k) {
         const float av = a[(long long)k * lda];
         s = b ? fmaf(av, b[(long long)k * HID], s) : s + av;
+        l += av;
       }
-      red[y][c] = s;
+      red[y][c] = i == NPARAM ? (float)l : s;
     }
   }
   __syncthreads();
   if (q != 0 || i < 0 || i > NPARAM) return;
-  float s = 0.f;
-  for (int y = 0; y < (conv ? cs : ds); ++y) s += red[y][c];
   if (i == NPARAM) {
-    if (loss_sum) *loss_sum = s;
-    if (loss_mean) *loss_mean = s / (float)(n * NOUT);
+    double l = 0.;
+    for (int y = 0; y < ds; ++y) l += red[y][c];
+    if (loss_sum) *loss_sum = (float)l;
+    if (loss_mean) *loss_mean = (float)(l / (n * NOUT));
     return;
   }
+  float s = 0.f;
+  for (int y = 0; y < (conv ? cs : ds); ++y) s += red[y][c];
   g[i] = s;
   if constexpr (ADAM) adam_step(i, s, p, m, v, pbf, pack, lr, bc1, bc2);
 }
