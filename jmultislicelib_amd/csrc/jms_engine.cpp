@@ -582,17 +582,18 @@ int enqueue_batch(jms_hip_engine* e, void* waves, float* partial, int nwave, int
       return jms::launch_col_pass(e->ny, q.nw, false, j == S - 1, c, q.st);
     };
     for (int r = 0; r < sp.rounds; ++r) {
-      std::vector<Part> pt;
+      Part pt[2];  // no allocation: see jms_hip_run_batch_noalloc
+      int npt = 0;
       for (int h = 0; h < (two ? 2 : 1); ++h) {
         const int p = r * (two ? 2 : 1) + h;
         if (part >= 0 && p != part) continue;
         const int w0 = (int)((long long)nwave * p / parts), w1 = (int)((long long)nwave * (p + 1) / parts);
-        pt.push_back({w0, w1 - w0, h && part < 0 ? e->side : e->st});
+        pt[npt++] = {w0, w1 - w0, h && part < 0 ? e->side : e->st};
       }
-      if (pt.empty()) continue;
+      if (npt < 1) continue;
       plane_setup(islc0);
-      for (const Part& q : pt)
-        if ((err = init(q)) != hipSuccess) return e->fail(130, "column pass (init)", err);
+      for (int h = 0; h < npt; ++h)
+        if ((err = init(pt[h])) != hipSuccess) return e->fail(130, "column pass (init)", err);
       for (int j = islc0; j < S; ++j) {
         const int js = e->objslc[j] % e->nscslc;
         // real-space readout of plane j inside the row pass (ReadoutImgDet_d)
@@ -600,9 +601,9 @@ int enqueue_batch(jms_hip_engine* e, void* waves, float* partial, int nwave, int
         const int mode = (id >= 0 && ch.real_space()) ? 1 : 0;
         rc.chan_off = id >= 0 ? (long long)id * e->n : 0;
         plane_setup(j + 1);
-        for (const Part& q : pt) {
-          if ((err = row(q, j, js, mode)) != hipSuccess) return e->fail(131, "row pass", err);
-          if ((err = col(q, j, js)) != hipSuccess) return e->fail(132, "column pass", err);
+        for (int h = 0; h < npt; ++h) {
+          if ((err = row(pt[h], j, js, mode)) != hipSuccess) return e->fail(131, "row pass", err);
+          if ((err = col(pt[h], j, js)) != hipSuccess) return e->fail(132, "column pass", err);
         }
       }
     }
