@@ -127,9 +127,11 @@ struct jms_hip_engine {
   DevBuf pro, pro_t;  // row-major and column-major ([x][y]) copies
   std::vector<Gap> pro_gap;  // zero gap of each propagator
   // plane table of the one-launch slice loop (GrpPlane [nobjslc + 1]; sums of
-  // one tile), kept in step with the set-up calls
+  // one tile), kept in step with the set-up calls (refresh_loop); loop_host: what
+  // the device holds
   DevBuf loop_tab;
-  bool loop_ready = false;
+  std::vector<jms::GrpPlane> loop_host;
+  bool loop_ready = false, loop_stale = false;
   // object slices
   int nobjslc = 0;
   std::vector<int> objslc;
@@ -139,7 +141,7 @@ struct jms_hip_engine {
   DevBuf detw, detw_t, det_cols;
   // bit d of entry x: detector d has a weight in column x; in use (columns())
   // once every detector of the set-up has been uploaded (det_seen)
-  std::vector<unsigned> det_cols_h;
+  std::vector<unsigned> det_cols_h, det_cols_dev;  // det_cols_dev: what the device holds
   unsigned det_seen = 0;
   const unsigned* columns() const {
     return ndet > 0 && det_seen == (1u << ndet) - 1 ? (const unsigned*)det_cols.p : nullptr;
@@ -322,10 +324,16 @@ struct BatchChans {
   bool any() const { return real_space() || dif || dif_avg || wff || wff_avg; }
 };
 
-// The plane table of the one-launch slice loop, after a set-up call that it
-// depends on (the batch runs never allocate or copy it).
-void refresh_loop(jms_hip_engine* e) {
+// The plane table of the one-launch slice loop.  The set-up calls before the
+// detection's only mark it stale: it is made once, with the detection, or by the
+// next run where the detection stays (not by the allocation-free entry, which
+// takes the passes until then), and goes up only when it has changed.
+void stale_loop(jms_hip_engine* e) {
   e->loop_ready = false;
+  e->loop_stale = true;
+}
+void refresh_loop(jms_hip_engine* e) {
+  e->loop_ready = e->loop_stale = false;
   const int S = e->nobjslc;
   if (!jms::loop_ok(e->nx, e->ny, 256) || S < 1 || !e->pgr.p || !e->pro_t.p || e->npgx != e->nx || e->npgy != e->ny ||
       e->nscslc < 1 || (int)e->proidx.size() < e->nscslc || (int)e->slcoffset.size() < e->nscslc ||
@@ -341,11 +349,17 @@ void refresh_loop(jms_hip_engine* e) {
     const int id = e->det_objslc[p];
     pl[p].part_off = id >= 0 && (e->detflags & JMS_HIP_DETECT_INTEGRATED) ? (long long)id * e->ndet : -1;
   }
-  (void)hipSetDevice(e->device);
-  (void)hipStreamSynchronize(e->st);  // launches already enqueued may still read the old table
   const size_t nb = sizeof(jms::GrpPlane) * pl.size();
-  e->loop_ready = e->loop_tab.ensure(nb) == hipSuccess &&
-                  hipMemcpy(e->loop_tab.p, pl.data(), nb, hipMemcpyHostToDevice) == hipSuccess;
+  static_assert(sizeof(jms::GrpPlane) == 32, "compared bytewise: no padding");
+  if (pl.size() != e->loop_host.size() || std::memcmp(pl.data(), e->loop_host.data(), nb) != 0) {
+    (void)hipSetDevice(e->device);
+    (void)hipStreamSynchronize(e->st);  // launches already enqueued may still read the old table
+    e->loop_host.clear();
+    if (e->loop_tab.ensure(nb) != hipSuccess || hipMemcpy(e->loop_tab.p, pl.data(), nb, hipMemcpyHostToDevice) != hipSuccess)
+      return;
+    e->loop_host.swap(pl);
+  }
+  e->loop_ready = true;
 }
 
 // whether a batch of nwave waves without channels runs as one launch
@@ -740,7 +754,7 @@ int jms_hip_set_grid(jms_hip_engine* e, int nx, int ny, float a0x, float a0y, fl
   e->nx = nx; e->ny = ny; e->n = (long long)nx * ny;
   e->a0x = a0x; e->a0y = a0y; e->wl = wl;
   e->panel = jms::panel_ok(nx, ny);
-  e->loop_ready = false;
+  e->loop_ready = e->loop_stale = false;
   e->pro_gap.assign(e->pro_gap.size(), Gap());
   e->wav0_gap = e->wav_gap = Gap();
   std::vector<float> tw;
@@ -777,7 +791,7 @@ int jms_hip_setup_gratings(jms_hip_engine* e, int npgx, int npgy, int nslc, cons
   if (err != hipSuccess) return e->fail(104, "allocate phase gratings", err);
   err = hipMemset(e->pgr.p, 0, sizeof(float) * 2 * (size_t)off);
   if (err != hipSuccess) return e->fail(105, "clear phase gratings", err);
-  refresh_loop(e);
+  stale_loop(e);
   return 0;
 }
 
@@ -950,7 +964,7 @@ int jms_hip_setup_propagators(jms_hip_engine* e, int npro, int nslc, const int* 
   hipError_t err = e->pro.ensure(sizeof(float) * 2 * (size_t)npro * e->n);
   if (err == hipSuccess) err = e->pro_t.ensure(sizeof(float) * 2 * (size_t)npro * e->n);
   if (err != hipSuccess) return e->fail(102, "allocate propagators", err);
-  refresh_loop(e);
+  stale_loop(e);
   return 0;
 }
 
@@ -979,7 +993,7 @@ int jms_hip_setup_objects(jms_hip_engine* e, int nobjslc, const int* objslc) {
   e->drop_graphs();
   e->nobjslc = nobjslc;
   e->objslc.assign(objslc, objslc + nobjslc);
-  refresh_loop(e);
+  stale_loop(e);
   return 0;
 }
 
@@ -1051,24 +1065,35 @@ int jms_hip_upload_detector(jms_hip_engine* e, int idet, const float* det, int m
   } else {
     std::memcpy(wgt.data(), det, sizeof(float) * (size_t)e->n);
   }
-  e->det_inf[idet] = !finite(wgt.data(), wgt.size());
+  // the columns with a weight, and whether every weight is finite, row by row
+  std::vector<unsigned> any(e->nx, 0u);
+  unsigned inf = 0;
+  for (int y = 0; y < e->ny; ++y) {
+    const float* r = wgt.data() + (size_t)y * e->nx;
+    for (int x = 0; x < e->nx; ++x) {
+      uint32_t u;
+      std::memcpy(&u, r + x, 4);
+      any[x] |= u & 0x7fffffffu;
+      inf |= ((u & 0x7f800000u) == 0x7f800000u);
+    }
+  }
+  e->det_inf[idet] = inf != 0;
   std::vector<float> wt = to_colmajor(wgt.data(), e->nx, e->ny);
   const size_t nb = sizeof(float) * (size_t)e->n;
   hipError_t err = hipMemcpy(e->detw.as<float>() + (long long)idet * e->n, wgt.data(), nb, hipMemcpyHostToDevice);
   if (err == hipSuccess)
     err = hipMemcpy(e->detw_t.as<float>() + (long long)idet * e->n, wt.data(), nb, hipMemcpyHostToDevice);
   e->det_cols_h.resize(e->nx, ~0u);
-  for (int x = 0; x < e->nx; ++x) {
-    const float* col = wt.data() + (size_t)x * e->ny;
-    const bool any = std::any_of(col, col + e->ny, [](float v) { return !(v == 0.f); });
-    e->det_cols_h[x] = (e->det_cols_h[x] & ~(1u << idet)) | (any ? 1u << idet : 0u);
-  }
+  for (int x = 0; x < e->nx; ++x)
+    e->det_cols_h[x] = (e->det_cols_h[x] & ~(1u << idet)) | (any[x] ? 1u << idet : 0u);
   e->det_seen |= 1u << idet;
-  if (e->det_seen == (1u << e->ndet) - 1) {
+  if (e->det_seen == (1u << e->ndet) - 1 && e->det_cols_dev != e->det_cols_h) {
     const size_t nc = sizeof(unsigned) * (size_t)e->nx;
+    e->det_cols_dev.clear();
     if (err == hipSuccess) err = e->det_cols.ensure(nc);
     if (err == hipSuccess) err = hipMemcpy(e->det_cols.p, e->det_cols_h.data(), nc, hipMemcpyHostToDevice);
-    if (err != hipSuccess) e->det_seen = 0;
+    if (err == hipSuccess) e->det_cols_dev = e->det_cols_h;
+    else e->det_seen = 0;
   }
   if (err != hipSuccess) return e->fail(104, "upload detector", err);
   return 0;
@@ -1233,6 +1258,7 @@ int jms_hip_run_staged(jms_hip_engine* e, int pos0, int npos, int islc0) {
   if (!e->wav0.p) return e->fail(6, "probe not set");
   islc0 = std::max(0, std::min(islc0, e->nobjslc));
   (void)hipSetDevice(e->device);
+  if (e->loop_stale) refresh_loop(e);
   const int npass = e->s_npass;
   const int total = npos * npass;
   int bw = auto_batch(e, total);
@@ -1747,6 +1773,7 @@ int jms_hip_multislice(jms_hip_engine* e, int islc0, const int* var, float weigh
   }
   islc0 = std::max(0, std::min(islc0, S));
   (void)hipSetDevice(e->device);
+  if (e->loop_stale) refresh_loop(e);
   rc = ensure_batch(e, 1);
   if (rc) return rc;
   const int per = e->ndetslc * std::max(1, e->ndet);
