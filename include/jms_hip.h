@@ -131,15 +131,19 @@ int jms_hip_sync(jms_hip_engine* e);
  * loops).  Runs the slice loop from plane islc0 on nwave = npos * npass waves
  * of the set-up specimen, as one batch of jms_hip_run_staged does, with every
  * buffer in device memory that the caller owns: waves (nwave * nx * ny
- * complex64 of working storage, laid out as the staged batches keep their
- * waves), ppar (float4 per wave: dx, dy [nm],
+ * complex64 of working storage, not all of it used on every grid; its contents
+ * after the call are unspecified), ppar (float4 per wave: dx, dy [nm],
  * dz * lambda / 2, 0), var (nobjslc ints per wave), weights (npass), res
  * (npos * ndetslc * ndet floats, overwritten).  Enqueued on the engine's
  * stream; jms_hip_sync waits.  The readout partial sums use a fixed 16 MiB
  * scratch array per GPU (nwave * ndetslc * ndet * column tiles floats at
  * most 4 Mi; larger batches are refused with code 5); calls must not overlap
  * on one GPU, since all share that GPU's scratch.  No hipMalloc, hipFree or
- * allocating library call. */
+ * allocating library call, and no allocation on the host.  After set-up calls
+ * that replace gratings, propagators or object slices of an edge of 64, 96 or 128
+ * points without setting up the detection again, the one-launch slice loop comes
+ * back with the next jms_hip_setup_detection, jms_hip_run_staged or
+ * jms_hip_multislice; until then this entry runs pass by pass. */
 int jms_hip_run_batch_noalloc(jms_hip_engine* e, int islc0, int nwave, void* waves, const float* ppar,
                               const int* var, int npos, int npass, const float* weights, float* res);
 /* Uneven batch in grouped launches (no counterpart in the reference, which
@@ -174,8 +178,9 @@ int jms_hip_get_scan_results(jms_hip_engine* e, float* out);
 /* batch size in probe passes (waves resident at once, at most 65535); 0 =
  * automatic (about 2 GiB of waves, at most 8192) */
 int jms_hip_set_batch(jms_hip_engine* e, int nwave_max);
-/* 1: capture the per-batch launch sequence in HIP graphs (one for each part
- * of a batch larger than the Infinity Cache) and replay them */
+/* 1: capture the per-batch launch sequence in HIP graphs and replay them: one
+ * graph, two side by side on two streams from about 40 MiB of stored waves on, and
+ * such a pair for each part of a batch larger than the Infinity Cache */
 int jms_hip_set_graph(jms_hip_engine* e, int use_graph);
 
 /* single-wave path (CJMultiSlice::GPUMultislice) --------------------------- */

@@ -380,7 +380,10 @@ bool use_loop(const jms_hip_engine* e, int nwave, int islc0) {
 //   512^2 1.13 / 1.10 / 1.13   625^2 2.18 / 2.17 / 2.01   640^2 1.61 / 1.56 / 1.46
 //   720^2 1.74 / 1.71 / 1.60   1024^2 1.49 / 1.55 / 1.44
 // and a batch of that size as one streamed launch per pass: 256^2 1.21, 512^2
-// 1.20, 625^2 2.34, 720^2 1.78.  At 184 MiB stored 512^2 is back at 1.19.
+// 1.20, 625^2 2.34, 720^2 1.78.  At 184 MiB stored 512^2 is back at 1.19.  One
+// rule for all lengths: two streams, although 512^2 is 3% faster on one.  Engines
+// whose batches run at the same time each size their parts for the whole cache;
+// that was not measured.
 // Waves above kNearWave leave a part too few of them to fill the device (2048^2
 // 1.63, in parts 1.70); halves of less than kTwoBytes together are no faster
 // (256^2, 22 MiB stored: 1.66 on one stream, 1.73 on two; 44 MiB: 1.37, 1.32).

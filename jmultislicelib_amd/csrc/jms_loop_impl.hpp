@@ -2,14 +2,19 @@
 // (gfx950): one block per wave, the wave in LDS from the incident wave to the
 // exit plane.
 //
-// A 128^2 wave (128 KiB) fits the 160 KiB of a CU, so neither pass touches
-// memory: per slice a block reads its grating and the propagator (from L2) and
-// nothing else, and the launches of a pass, their fill and drain, are gone.
-// What bounds it is the arithmetic of the transforms, the same as in the two
-// passes (jms_kernels_impl.hpp): rows inverse, * grating, forward; columns
-// forward, * propagator, readout, inverse; the same plans and twiddles.
+// A 128^2 wave (128 KiB) fits the 160 KiB of a CU, so the wave does not leave it
+// between the passes, and the launches of a pass, their fill and drain, are gone.
+// Per slice a block reads its grating and the propagator (from L2).  The work is
+// that of the two passes (jms_kernels_impl.hpp): rows inverse, * grating, forward;
+// columns forward, * propagator, readout, inverse; the same plans and twiddles.
 // Lines are transformed in place, by 4 or 8 threads each, inside a
 // wavefront; two barriers per slice.
+// What bounds it: the vector instructions and LDS exchanges of one wave per CU,
+// and, where the columns have 128 points, spilled registers: a block of 1024
+// threads gets 128 VGPRs a thread, too few for 16 values of a column beside their
+// propagator or grating and the transform, so 86-107 of them (348-432 bytes a
+// lane) go through scratch memory.  128 x 96: 16 (with a band) and 35; the other
+// grids: none.
 #pragma once
 #include "jms_kernels_impl.hpp"
 
@@ -164,8 +169,8 @@ __global__ __launch_bounds__((loop_block<NX, NY>())) void k_loop(LoopArgs a) {
 #pragma unroll 1
   for (int j = a.islc0; j < a.nslc; ++j) {
     // hidden from the optimiser: the many offsets derived from the thread are
-    // formed where they are used instead of being kept (and spilled) over the
-    // slices
+    // formed where they are used instead of being kept over the slices (they
+    // would add to the spills)
     __asm__ volatile("" : "+v"(row), "+v"(tx), "+v"(x), "+v"(ty));
     __syncthreads();
     // ---- rows

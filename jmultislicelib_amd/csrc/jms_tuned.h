@@ -1,8 +1,8 @@
 // jms_tuned.h -- launch shapes per line length chosen by the autotuner
-// (csrc/tune/tune.py) from measured kernel times on MI355X (some revised by the
-// time of pairs of passes, see REVISED there).  Generated:
-// edit by re-running the tuner.  Fields not given keep the defaults of
-// jms_cfg.hpp: LPB (rows per row-pass block; 0 = default), GTW (row-pass
+// (csrc/tune/tune.py) from measured kernel times on MI355X.  Generated by emit()
+// there; at the six lengths of REVISED its fields come from that table (pairs of
+// passes timed outside the tuner) and a re-run does not change them.  Fields not
+// given keep the defaults of jms_cfg.hpp: LPB (rows per row-pass block; 0 = default), GTW (row-pass
 // twiddles from the global table with the product tree), CW (columns per
 // wave-local column block), WPE (waves per SIMD asked of the register
 // allocator for that kernel), TW (threads per column of that kernel; 0 =

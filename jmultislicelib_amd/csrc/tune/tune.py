@@ -190,10 +190,14 @@ def choose(results):
 
 
 # Choices by the time of a pair of passes over waves that keep their energy,
-# streamed and from the Infinity Cache, which replace those from single passes:
-# column tiles without LDS padding (320, 384), with ordinary loads and stores in
-# 8-column tiles (640 1.67 -> 1.63, 720 1.79 -> 1.69, 768 1.63 -> 1.60 ms per 2
-# GiB of waves, streamed), 625 in panels (2.20 -> 1.68; one wavefront per row).
+# streamed and from the Infinity Cache, which replace those from single passes
+# (timed here on waves cleared to zero, which run faster: less power).  They are
+# fixed: a re-run of the tuner does not produce them, and 625-point panels, whose
+# last one is partly filled, have no timer.  ms per 2 GiB of waves and pair:
+# column tiles without LDS padding (staged scans in parts: 320 1.47 -> 1.45, 384
+# 1.414 -> 1.406; a batch of one part 1.54 -> 1.52, 1.46 -> 1.43), with ordinary loads and stores in 8-column tiles (streamed: 640 1.67 ->
+# 1.63, 720 1.79 -> 1.69, 768 1.63 -> 1.60), 625 in panels (2.20 -> 1.68; one
+# wavefront per row).
 REVISED = {320: {"pad": 24}, 384: {"pad": 24}, 640: {"pad": 24, "ntc": False}, 720: {"pad": 24, "ntc": False},
            768: {"pad": 24, "ntc": False}, 625: {"cw": 8, "pad": 24, "padr": 24, "panel": True, "tr": 64}}
 
@@ -203,10 +207,10 @@ def emit(results, path):
     for n, k in REVISED.items():
         ch.setdefault(n, {}).update(k)
     lines = ["// jms_tuned.h -- launch shapes per line length chosen by the autotuner",
-             "// (csrc/tune/tune.py) from measured kernel times on MI355X (some revised by the",
-             "// time of pairs of passes, see REVISED there).  Generated:",
-             "// edit by re-running the tuner.  Fields not given keep the defaults of",
-             "// jms_cfg.hpp: LPB (rows per row-pass block; 0 = default), GTW (row-pass",
+             "// (csrc/tune/tune.py) from measured kernel times on MI355X.  Generated by emit()",
+             "// there; at the six lengths of REVISED its fields come from that table (pairs of",
+             "// passes timed outside the tuner) and a re-run does not change them.  Fields not",
+             "// given keep the defaults of jms_cfg.hpp: LPB (rows per row-pass block; 0 = default), GTW (row-pass",
              "// twiddles from the global table with the product tree), CW (columns per",
              "// wave-local column block), WPE (waves per SIMD asked of the register",
              "// allocator for that kernel), TW (threads per column of that kernel; 0 =",
