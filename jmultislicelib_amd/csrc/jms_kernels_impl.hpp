@@ -408,6 +408,23 @@ __device__ __forceinline__ void clear_gap_partials(const ColArgs& a, long long w
   for (int i = threadIdx.x; i < a.ndet * a.tgn; i += nthreads) p[(i / a.tgn) * a.part_dstride + i % a.tgn] = 0.f;
 }
 
+// What a band-limited pass leaves out is zero as long as the wave is finite; of
+// a wave that is not, the product with the zero propagator is no number.  Once a
+// value is not finite the transforms spread it over the whole plane, so a thread
+// tells from its own values, and column 0 stands for the columns left out.
+__device__ __forceinline__ float2 not_a_number() {
+  return make_float2(__builtin_nanf(""), __builtin_nanf(""));
+}
+__device__ __forceinline__ bool is_finite(const float2& z) { return z.x * 0.f + z.y * 0.f == 0.f; }
+// what an exit pass clears its left-out columns with, from column 0 of the wave
+// (row stride rs), as it was or as this pass has left it; all threads of a block
+template <int N, int NT>
+__device__ __forceinline__ float2 cleared_value(const float2* col0, int rs, int tid) {
+  int bad = 0;
+  for (int e = tid; e < N; e += NT) bad |= !is_finite(col0[(long long)e * rs]);
+  return __syncthreads_or(bad) ? not_a_number() : make_float2(0.f, 0.f);
+}
+
 // Tile of C adjacent columns x N rows staged through LDS (column c at
 // L::idx(c, e)); thread tid moves elements i = tid + k*BS, i.e. row i / C,
 // column i % C, so a wavefront covers 64/C whole 8*C-byte row segments.
@@ -555,6 +572,18 @@ __device__ __forceinline__ void col_body(const ColArgs& a, long long w, float2* 
       }
     });
   }
+  [[maybe_unused]] auto lost = [&]() {  // none of the thread's values is finite
+    bool some = t >= M1::NBF;  // a thread without values
+    static_for<0, M1::NB>([&](auto I) {
+      constexpr int i = decltype(I)::value;
+      if (M1::FULL || t + i * T < M1::NBF)
+        static_for<0, M1::R0>([&](auto Q) {
+          constexpr int q = decltype(Q)::value;
+          if constexpr (!dead(q)) some |= is_finite(v[i * M1::R0 + q]);
+        });
+    });
+    return !some;
+  };
   // a.detect is uniform over the block (one wave per block row): in a grouped
   // launch, jobs that do not read this plane out skip the readout
   if (DET && a.detect) {
@@ -616,26 +645,40 @@ __device__ __forceinline__ void col_body(const ColArgs& a, long long w, float2* 
     if (valid && (a.dif || a.wff || a.dif_avg || a.wff_avg)) {  // ReadoutDifDet_d channels (JMultiSlice.cpp:4310-4356)
       const float wg = a.cwgt[w];
       const long long cb = w * a.chan_wstride + a.chan_off;
+      auto put = [&](int xc, int ky, const float2& z) {
+        const long long idx = cb + (long long)wrap_sub(ky, a.dsy, N) * nx + wrap_sub(xc, a.dsx, nx);
+        const float pz = z.x * z.x + z.y * z.y;
+        if (a.dif) a.dif[idx] += wg * pz;
+        if (a.dif_avg) a.dif_avg[idx] += wg * pz;
+        if (a.wff) { float2 o = a.wff[idx]; o.x += z.x * wg; o.y += z.y * wg; a.wff[idx] = o; }
+        if (a.wff_avg) { float2 o = a.wff_avg[idx]; o.x += z.x * wg; o.y += z.y * wg; a.wff_avg[idx] = o; }
+      };
       static_for<0, M1::NB>([&](auto I) {
         constexpr int i = decltype(I)::value;
         const int b = t + i * T;
         if (M1::FULL || b < M1::NBF) {
           static_for<0, M1::R0>([&](auto Q) {
             constexpr int q = decltype(Q)::value;
-            if constexpr (dead(q)) return;
-            const long long idx = cb + (long long)wrap_sub(b + q * M1::NBF, a.dsy, N) * nx + wrap_sub(x, a.dsx, nx);
-            const float2 z = v[i * M1::R0 + q];
-            const float pz = z.x * z.x + z.y * z.y;
-            if (a.dif) a.dif[idx] += wg * pz;
-            if (a.dif_avg) a.dif_avg[idx] += wg * pz;
-            if (a.wff) { float2 o = a.wff[idx]; o.x += z.x * wg; o.y += z.y * wg; a.wff[idx] = o; }
-            if (a.wff_avg) { float2 o = a.wff_avg[idx]; o.x += z.x * wg; o.y += z.y * wg; a.wff_avg[idx] = o; }
+            if constexpr (!dead(q)) put(x, b + q * M1::NBF, v[i * M1::R0 + q]);
           });
         }
       });
+      if (lost()) {
+        const int xg = (x == 0 ? a.tgn : 0) * C_::CC;  // column 0: the columns left out too
+        constexpr int step = T < M1::NBF ? T : M1::NBF;
+        for (int ky = t; ky < N; ky += step) {
+          if (dead(ky / M1::NBF)) put(x, ky, not_a_number());
+          for (int xc = a.tg0 * C_::CC; xc < a.tg0 * C_::CC + xg; ++xc)
+            put(xc, ky, INIT ? a.src[w * a.src_stride + (long long)ky * nx + xc] : not_a_number());
+        }
+      }
     }
   }
   if constexpr (EXIT) {
+    [[maybe_unused]] float2 zero = make_float2(0.f, 0.f);  // the dead rows
+    if constexpr (BAND) {
+      if (a.keep && lost()) zero = not_a_number();
+    }
     CS{}();
     static_for<0, M1::NB>([&](auto I) {
       constexpr int i = decltype(I)::value;
@@ -643,6 +686,7 @@ __device__ __forceinline__ void col_body(const ColArgs& a, long long w, float2* 
       if (M1::FULL || b < M1::NBF) {
         static_for<0, M1::R0>([&](auto Q) {
           constexpr int q = decltype(Q)::value;
+          if constexpr (dead(q)) v[i * M1::R0 + q] = zero;
           s_buf[lds_slot<L, M1::NBF, q>(c, b, L::idx(c, b))] = v[i * M1::R0 + q];
         });
       }
@@ -743,8 +787,9 @@ __global__ __launch_bounds__(C_::TW * C_::CW) __attribute__((amdgpu_waves_per_eu
   const int cs = tid % C, bs = tid / C;  // sweep mapping: column, first-stage butterfly
   if constexpr (EXIT) {
     if (a.tclr && tile >= a.tg0 && tile < a.tg0 + a.tgn) {  // uniform over the block
+      const float2 z = cleared_value<N, BS>(a.wave + w * a.wave_stride, nx, tid);
       float2 st[TL::KST];
-      static_for<0, TL::KST>([&](auto K) { st[decltype(K)::value] = make_float2(0.f, 0.f); });
+      static_for<0, TL::KST>([&](auto K) { st[decltype(K)::value] = z; });
       TL::store(st, wv_base, wrs, ncol, tid);
       return;
     }
@@ -941,8 +986,9 @@ __global__ __launch_bounds__(64 * C_::XCT) __attribute__((amdgpu_waves_per_eu(4)
   const long long astep = 64LL * wrs;
   if constexpr (EXIT) {
     if (a.tclr && tile >= a.tg0 && tile < a.tg0 + a.tgn) {  // uniform over the block
+      const float2 z = cleared_value<N, NT>(a.wave + w * a.wave_stride, nx, tid);
       if (ca < ncol)
-        for (int n2 = 0; n2 < M; ++n2) *at32(wbase + n2 * astep, n1 * wrs + ca) = make_float2(0.f, 0.f);
+        for (int n2 = 0; n2 < M; ++n2) *at32(wbase + n2 * astep, n1 * wrs + ca) = z;
       return;
     }
   }
@@ -1041,16 +1087,27 @@ __global__ __launch_bounds__(64 * C_::XCT) __attribute__((amdgpu_waves_per_eu(4)
           const float wg = a.cwgt[w];
           const long long cbase = w * a.chan_wstride + a.chan_off;
           const int q = opaque(qs);
-          static_for<0, 16>([&](auto K) {
-            constexpr int c = decltype(K)::value;
-            const long long idx = cbase + ((16 * r + M * c + q) & (N - 1)) * nx + xs;
-            const float2 z = u[c];
+          auto put = [&](int c, int xd, const float2& z) {
+            const long long idx = cbase + ((16 * r + M * c + q) & (N - 1)) * nx + xd;
             const float pz = z.x * z.x + z.y * z.y;
             if (a.dif) a.dif[idx] += wg * pz;
             if (a.dif_avg) a.dif_avg[idx] += wg * pz;
             if (a.wff) { float2 o = a.wff[idx]; o.x += z.x * wg; o.y += z.y * wg; a.wff[idx] = o; }
             if (a.wff_avg) { float2 o = a.wff_avg[idx]; o.x += z.x * wg; o.y += z.y * wg; a.wff_avg[idx] = o; }
+          };
+          bool some = false;
+          static_for<0, 16>([&](auto K) {
+            constexpr int c = decltype(K)::value;
+            put(c, xs, u[c]);
+            some |= is_finite(u[c]);
           });
+          if (!some && xb == 0) {  // a wave that is not finite: the columns left out too
+            for (int k = 0; k < 16 * a.tgn * CT; ++k) {
+              const int c = k % 16, xc = a.tg0 * CT + k / 16;
+              put(c, wrap_sub(xc, a.dsx, nx),
+                  INIT ? a.src[w * a.src_stride + (long long)kyof(r, c) * nx + xc] : not_a_number());
+            }
+          }
         }
       }
     }

@@ -261,9 +261,23 @@ __global__ __launch_bounds__((loop_block<NX, NY>())) void k_loop(LoopArgs a) {
   }
   if (a.wave) {  // psi(k) of the exit plane
     float2* o = a.wave + w * a.wave_stride;
-    if (col_on) each_y1([&](auto K, int ky, auto) { o[ky * NX + x] = vy[decltype(K)::value]; });
+    float2 zero = make_float2(0.f, 0.f);  // the dead rows
     if constexpr (BAND) {
-      for (int i = tid; i < NY * gap; i += BS) o[(i / gap) * NX + a.gx0 + i % gap] = make_float2(0.f, 0.f);
+      bool some = !col_on;
+      each_y1([&](auto K, int, auto Q) {
+        if constexpr (!dead_y(decltype(Q)::value)) some |= is_finite(vy[decltype(K)::value]);
+      });
+      if (!some) zero = not_a_number();
+    }
+    if (col_on)
+      each_y1([&](auto K, int ky, auto Q) {
+        if constexpr (dead_y(decltype(Q)::value)) o[ky * NX + x] = zero;
+        else o[ky * NX + x] = vy[decltype(K)::value];
+      });
+    if constexpr (BAND) {
+      if (__syncthreads_or(cl == 0 && zero.x != 0.f)) zero = not_a_number();
+      else zero = make_float2(0.f, 0.f);
+      for (int i = tid; i < NY * gap; i += BS) o[(i / gap) * NX + a.gx0 + i % gap] = zero;
     }
   }
 }
